@@ -702,11 +702,10 @@ int rus_attn_varlen_fwd(const void* q, const void* k, const void* v, const int32
  * Backward of rus_attn_varlen_fwd: dq like q, dk / dv like k / v (fp16; dk and dv sum the h_q /
  * h_kv query heads of each group in fp32 and are rounded once). out and lse are the forward's.
  * workspace: fp32, at least 2 * h_q * n_tokens * 128 elements (per-query-head dK and dV
- * partials [h_q, n_tokens, 128] each, dK scaled). Both passes (dQ, and dK / dV with the sum over
- * each group's heads) run as one launch, each block forming D = rowsum(dO o O) of the query rows
- * it visits; max_blocks at most 32767.
- * counters: int32, at least max_blocks * h_kv, zero before the first call and left zero (calls
- * sharing them must not run concurrently).
+ * partials [h_q, n_tokens, 128] each, dK scaled). Both passes (dQ, and the partials of dK / dV)
+ * run as one launch, each block forming D = rowsum(dO o O) of the query rows it visits; a second
+ * one sums each group's heads. max_blocks at most 32767.
+ * counters: int32, at least max_blocks * h_kv (checked, but not read: no launch counts arrivals).
  * Replaces: the autograd backward of solution/ops.py:669-696 (torch SDPA backward plus the
  * sum over the expanded K/V heads), run by solution/ops.py:903-928.
  */

@@ -25,11 +25,15 @@
 //   * backward: one launch runs the dK / dV blocks (row, key block, query head; fp32 dK / dV
 //     partials per query head) and the dQ blocks (row, query block, head); each block forms
 //     D = rowsum(dO o O) of the query rows it visits from the dO tile in LDS and O rows loaded
-//     with that tile (no separate launch, no D array). The h_q / h_kv partials of a KV group are summed in head order
-//     and rounded once, either by the last of the group's blocks to finish a key block (arrival
-//     counter; no atomics on data) or, in the engine's path, by the RoPE backward that packs
-//     them (rus_qkv_rope_bwd_mid_parts).
+//     with that tile (no separate launch, no D array). The h_q / h_kv partials of a KV group are
+//     summed in head order and rounded once, by a second launch or, in the engine's path, by the
+//     RoPE backward that packs them (rus_qkv_rope_bwd_mid_parts);
+//   * two layouts of both passes, chosen by size (wide() below): the 32-token blocks above, whose
+//     waves split the other side's blocks, for batches that would leave the chip idle otherwise;
+//     and 128-token blocks (attn_*_wide_kernel), whose four waves share each streamed tile.
 #include <math.h>
+
+#include <algorithm>
 
 #include "common.h"
 
@@ -61,11 +65,10 @@ struct AttnArgs {
   float* dv_part;
   f16* dk;         // [n_tok, h_kv, 128]
   f16* dv;
-  int* counters;   // [max_blocks, h_kv] arrival counters (zero on entry, left zero)
   int64_t n_tok;
   int n_seq, h_q, h_kv;
   int max_blocks;  // backward: blocks per pass (grid y of each pass)
-  int group_sum;   // backward: 1 = sum each KV group's dK / dV partials into dk / dv
+  int n_blocks;    // wide kernels: bound of the 128-token blocks over all rows
   float scale, scale_log2;
 };
 
@@ -78,17 +81,18 @@ __device__ __forceinline__ f32x16 mfma(f16x8 a, f16x8 b, f32x16 c) {
 }
 
 // Row bounds of row s (clamped to [0, n_tok] and non-decreasing, so a malformed cu_seqlens
-// cannot send an access outside the token arrays) and its number of 32-token blocks.
+// cannot send an access outside the token arrays) and its number of kB-token blocks.
 struct RowInfo {
   int a, e, nb;
 };
 
+template <int kB>
 __device__ __forceinline__ RowInfo row_info(const int32_t* cu, int s, int n_seq, int n_tok) {
   RowInfo r{0, 0, 0};
   if (s < n_seq) {
     r.a = min(max(cu[s], 0), n_tok);
     r.e = min(max(cu[s + 1], r.a), n_tok);
-    r.nb = (r.e - r.a + kBlk - 1) / kBlk;
+    r.nb = (r.e - r.a + kB - 1) / kB;
   }
   return r;
 }
@@ -100,25 +104,25 @@ __device__ __forceinline__ int nth_bit(uint64_t m, int n) {
 }
 
 // Block id -> (row start, row end, block start), heaviest blocks first. A row of nb blocks has
-// one block of each work level w = 1 .. nb (the number of 32-token blocks on the other side of
+// one block of each work level w = 1 .. nb (the number of kB-token blocks on the other side of
 // the causal loop): block w - 1 when the work grows towards the row's end (kDiagLast: forward
 // and dQ, which loop over the keys up to the diagonal), block nb - w otherwise (dK/dV, which loop
 // over the queries from the diagonal on). Ids run over levels from the highest down, rows in
 // order within a level, so the longest blocks are dispatched first. Each lane holds one row of
 // a 64-row chunk; false if blk is past the last block. Uniform over the block.
-template <bool kDiagLast>
+template <bool kDiagLast, int kB = kBlk>
 __device__ __forceinline__ bool find_block(const int32_t* cu, int n_seq, int n_tok, int blk,
                                            int& start, int& end, int& b0) {
   const int lane = threadIdx.x & 63;
   const int n_chunks = (n_seq + 63) / 64;
-  const RowInfo r0 = row_info(cu, lane, n_seq, n_tok);
+  const RowInfo r0 = row_info<kB>(cu, lane, n_seq, n_tok);
   int max_nb = r0.nb;
-  for (int c = 1; c < n_chunks; ++c) max_nb = max(max_nb, row_info(cu, 64 * c + lane, n_seq, n_tok).nb);
+  for (int c = 1; c < n_chunks; ++c) max_nb = max(max_nb, row_info<kB>(cu, 64 * c + lane, n_seq, n_tok).nb);
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) max_nb = max(max_nb, __shfl_xor(max_nb, off, 64));
   for (int w = max_nb; w >= 1; --w) {
     for (int c = 0; c < n_chunks; ++c) {
-      const RowInfo r = c == 0 ? r0 : row_info(cu, 64 * c + lane, n_seq, n_tok);
+      const RowInfo r = c == 0 ? r0 : row_info<kB>(cu, 64 * c + lane, n_seq, n_tok);
       const uint64_t mask = __ballot(r.nb >= w);
       const int cnt = __popcll(mask);
       if (blk < cnt) {
@@ -126,7 +130,7 @@ __device__ __forceinline__ bool find_block(const int32_t* cu, int n_seq, int n_t
         start = __shfl(r.a, src, 64);
         end = __shfl(r.e, src, 64);
         const int nb = __shfl(r.nb, src, 64);
-        b0 = start + (kDiagLast ? w - 1 : nb - w) * kBlk;
+        b0 = start + (kDiagLast ? w - 1 : nb - w) * kB;
         return true;
       }
       blk -= cnt;
@@ -578,9 +582,8 @@ __device__ __forceinline__ void attn_bwd_dq_block(const AttnArgs& a, int blk, ch
 
 // This query head's dK = scale * dS^T Q and dV = P^T dO for one 32-key block, fp32. Block = (row,
 // key block, head): the K and V tiles are shared; the kWB waves take query blocks (Q and dO tiles
-// of their own). The h_q / h_kv heads of a KV group store fp32 partials; the last of them to
-// finish sums the group in head order and writes dK and dV once (no atomics on data, no separate
-// reduce launch).
+// of their own). Each query head stores its fp32 partials; attn_group_sum_kernel or the RoPE
+// backward adds a KV group's.
 __device__ __forceinline__ void attn_bwd_dkdv_block(const AttnArgs& a, int blk, char* smem) {
   int start, end, k0;
   if (!find_block<false>(a.cu, a.n_seq, static_cast<int>(a.n_tok), blk, start, end, k0)) return;
@@ -680,45 +683,6 @@ __device__ __forceinline__ void attn_bwd_dkdv_block(const AttnArgs& a, int blk, 
                       x[r] * sc);
     }
   }
-  if (!a.group_sum) return;  // the partials are the output (summed by the RoPE backward)
-  const int grp = a.h_q / a.h_kv;
-  // The verdict goes through the first word of the merge buffer, which every thread is done
-  // reading once arrive_last_at's first barrier has passed.
-  if (!arrive_last_at(a.counters + static_cast<int64_t>(blk) * a.h_kv + g, grp,
-                      reinterpret_cast<int*>(smem)))
-    return;
-  // Last head of the group: dk[key, g, :] = fp16(sum over the group's heads in head order).
-  // Thread (wave, lane) owns head dims (wave % 4) * 32 + col of its keys, as in the stores.
-#pragma unroll
-  for (int pass = 0; pass < 2; ++pass) {
-    const float* src = pass == 0 ? a.dk_part : a.dv_part;
-    f16* out = pass == 0 ? a.dk : a.dv;
-    // Every head's loads are issued together (the partials are read device-coherently, from
-    // beyond this XCD's L2: one latency instead of one per head), then added in head order;
-    // slots past the group re-read its last head and are not added.
-    float v[kMaxGroup][kRegsPerWave];
-#pragma unroll
-    for (int j = 0; j < kMaxGroup; ++j) {
-      const int jj = min(j, grp - 1);
-      const float* hsrc =
-          src + static_cast<int64_t>(g * grp + jj) * a.n_tok * kHD + dt4 * 32 + col;
-#pragma unroll
-      for (int r = 0; r < kRegsPerWave; ++r) {
-        const int key = min(k0 + acc_row(rb + r, h), end - 1);  // past the end: read, not stored
-        v[j][r] = load_partial(hsrc + static_cast<int64_t>(key) * kHD);
-      }
-    }
-#pragma unroll
-    for (int r = 0; r < kRegsPerWave; ++r) {
-      float acc = v[0][r];
-#pragma unroll
-      for (int j = 1; j < kMaxGroup; ++j)
-        if (j < grp) acc += v[j][r];
-      const int key = k0 + acc_row(rb + r, h);
-      if (key < end)
-        out[(static_cast<int64_t>(key) * a.h_kv + g) * kHD + dt4 * 32 + col] = from_f32<f16>(acc);
-    }
-  }
 }
 
 // Both backward passes in one launch: blocks y < max_blocks are dK/dV blocks (the heavier ones,
@@ -730,6 +694,564 @@ attn_bwd_kernel(AttnArgs a) {
     attn_bwd_dkdv_block(a, blockIdx.y, smem);
   else
     attn_bwd_dq_block(a, blockIdx.y - a.max_blocks, smem);
+}
+
+// ---------------------------------------------------------------------------------------------
+// Wide kernels, for batches with enough 128-token blocks to fill the chip: a block takes 128 tokens
+// of one side (4 waves of 32, their fragments in registers) and streams the other side's 32-token
+// tiles through double-buffered LDS, each tile copied once for all four waves while the previous
+// one is used. The 32-token blocks copy 16 KiB per wave and 32 x 32 score tile and wait for it
+// (9 TB/s of L2 reads at 8,161 tokens, and a memory latency per tile); here the copies are a
+// quarter of that and off the critical path, and the LDS reads (16 KiB per wave and tile forward,
+// 24-32 KiB backward, 128 B/clock per CU) and the exponentials bound it beside the MFMAs. Measured
+// at 8,161 tokens in rows of 377 to 2,048, 12 / 2 heads: forward 129 -> 64 us (665 TFLOP/s of the
+// causal half), backward with partials 398 -> 196, with the group sum 440 -> 210.
+// ---------------------------------------------------------------------------------------------
+constexpr int kWide = 128;  // tokens per block
+
+// Block id -> (block index, head): the query heads of a KV group that work on one block index take
+// ids 8 apart, i.e. one XCD (ids go round robin over the 8), so they read their shared K / V tiles
+// from one L2. False past the last block.
+__device__ __forceinline__ bool wide_item(const AttnArgs& a, int n_blocks, int& blk, int& head) {
+  const int grp = a.h_q / a.h_kv, chunk = 8 * grp;
+  const int t = blockIdx.x / chunk, r = blockIdx.x % chunk;
+  const int item = t * chunk + (r & 7) * grp + (r >> 3);
+  blk = item / a.h_q;
+  head = item % a.h_q;
+  return blk < n_blocks;
+}
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+// This wave's two of the 8 copies that fill a shared tile (rows 8 wave .. + 8; see tile_copy for the
+// layout). The tile's first row is a uniform pointer, so a lane's offsets are the same for every
+// whole tile; rows past the row's end repeat its last token.
+struct TileLane {
+  int row[2];      // tile row of copy i
+  uint32_t ch[2];  // byte offset of its chunk within the row
+  uint32_t off[2];
+  uint32_t stride;  // bytes per token
+
+  __device__ __forceinline__ TileLane(int wave, int lane, int64_t stride_el)
+      : stride(static_cast<uint32_t>(stride_el) * 2) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      row[i] = 8 * wave + 4 * i + (lane >> 4);
+      ch[i] = ((lane & 15) ^ swz(row[i])) << 4;
+      off[i] = row[i] * stride + ch[i];
+    }
+  }
+
+  __device__ __forceinline__ uint32_t at(int i, int rows) const {  // rows: tokens left in the row
+    return rows >= kBlk ? off[i] : min(row[i], rows - 1) * stride + ch[i];
+  }
+
+  // Copies the tile whose first row is x (uniform), with `rows` (>= 1) tokens left, into LDS. The
+  // builtin's LDS target must be one of two __shared__ arrays of its own, so that the compiler
+  // knows which LDS reads have to wait for it.
+  __device__ __forceinline__ void copy(char* tile, int wave, const f16* x, int rows) const {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      __builtin_amdgcn_global_load_lds(reinterpret_cast<const char*>(x) + at(i, rows),
+                                       (lds_void_ptr)(tile + (2 * wave + i) * 1024), 16, 0, 0);
+  }
+};
+
+// A lane's LDS offsets for the fragments of a 32-row tile in tile_frag's and tile_frag_t's layout:
+// both are one base per lane, changed by step and head-dim tile in a few bits only. The empty asm
+// keeps the compiler from holding all sixteen combinations in registers across the loop (the
+// dK / dV blocks need every register; an exclusive or per read is cheap).
+struct FragLane {
+  uint32_t row, tr;
+
+  __device__ __forceinline__ explicit FragLane(int lane) {
+    const int c = lane & 31, h = lane >> 5, j = lane & 15, r0 = 4 * h + (j >> 2);
+    row = c * 256 + ((h ^ swz(c)) << 4);
+    tr = r0 * 256 + (((((lane >> 4) & 1) * 2 + ((j & 3) >> 1)) ^ swz(r0)) << 4) + (j & 1) * 8;
+  }
+  __device__ __forceinline__ FragLane fresh() const {
+    FragLane f = *this;
+    asm("" : "+v"(f.row), "+v"(f.tr));
+    return f;
+  }
+  // tile_frag(tile, lane % 32, 2 s + lane / 32)
+  __device__ __forceinline__ f16x8 frag(const char* tile, int s) const {
+    return *reinterpret_cast<const f16x8*>(tile + (row ^ (s << 5)));
+  }
+  // tile_frag_t(tile, s, d): row r0 + 8 differs from r0 in one bit of the swizzle
+  __device__ __forceinline__ f16x8 frag_t(const char* tile, int s, int d) const {
+    const v4i16 x0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_v4i16*)(tile + (tr ^ (d << 6)) + s * 4096));
+    const v4i16 x1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+        (lds_v4i16*)(tile + (tr ^ (d << 6) ^ 32) + s * 4096 + 2048));
+    const f16x4 a = __builtin_bit_cast(f16x4, x0), b = __builtin_bit_cast(f16x4, x1);
+    return f16x8{a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+  }
+};
+
+// Every copy of this wave has landed and every LDS read of it has returned, then the block's barrier:
+// the buffer just filled may be read, the buffer just read may be filled.
+__device__ __forceinline__ void stage_barrier() {
+  __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+  __syncthreads();
+}
+
+// The values of lanes l and l ^ 32 (in some order).
+__device__ __forceinline__ float2 half_pair(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  const auto p = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return float2{__builtin_bit_cast(float, static_cast<uint32_t>(p[0])),
+                __builtin_bit_cast(float, static_cast<uint32_t>(p[1]))};
+}
+
+// fp16 row of one token, head dims 32 d + 8 r4 + 4 h + i from x[d][4 r4 + i] * f: the lane pair
+// (l, l ^ 32) exchanges halves so that each stores 16 contiguous bytes.
+__device__ __forceinline__ void store_row(f16* row, const f32x16 (&x)[4], float f, int h,
+                                          bool valid) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      f16x4 w0, w1;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        w0[i] = from_f32<f16>(x[d][8 * b + i] * f);
+        w1[i] = from_f32<f16>(x[d][8 * b + 4 + i] * f);
+      }
+      const u32x2 a = __builtin_bit_cast(u32x2, w0), c = __builtin_bit_cast(u32x2, w1);
+      const auto p0 = __builtin_amdgcn_permlane32_swap(a.x, c.x, false, false);
+      const auto p1 = __builtin_amdgcn_permlane32_swap(a.y, c.y, false, false);
+      const u32x4 o = {static_cast<uint32_t>(p0[0]), static_cast<uint32_t>(p1[0]),
+                       static_cast<uint32_t>(p0[1]), static_cast<uint32_t>(p1[1])};
+      if (valid) *reinterpret_cast<u32x4*>(row + 32 * d + 16 * b + 8 * h) = o;
+    }
+}
+
+// Forward on 32 NT keys (tiles kt, kt + kTile; the last one holds the diagonal when `diag`).
+template <int NT>
+__device__ __forceinline__ void fwd_keys(const FragLane& fl, const char* kt, const char* vt, const f16x8 (&qf)[8],
+                                         f32x16 (&o)[4], float& m, float& l, float sl2, bool diag,
+                                         int k0, int qi, int end, int h) {
+  f32x16 st[NT];
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    st[n] = f32x16{};
+#pragma unroll
+    for (int s = 0; s < 8; ++s)
+      st[n] = mfma(fl.frag(kt + n * kTile, s), qf[s], st[n]);  // S^T = K Q^T
+  }
+  if (diag) {
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int key = k0 + 32 * (NT - 1) + acc_row(r, h);
+      st[NT - 1][r] = (key <= qi && key < end) ? st[NT - 1][r] : -INFINITY;
+    }
+  }
+  float mx = -INFINITY;
+#pragma unroll
+  for (int n = 0; n < NT; ++n)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, st[n][r]);
+  const float2 mp = half_pair(mx);
+  mx = fmaxf(mp.x, mp.y) * sl2;  // scale > 0
+  const bool bump = mx > m + kLazy;  // lazy rescaling, as in attn_fwd_kernel
+  if (__ballot(bump)) {
+    const float mn = bump ? mx : m;
+    const float alpha = exp2_raw(m - mn);
+    l *= alpha;
+    m = mn;
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[d][r] *= alpha;
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    float rs = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const float p = exp2_raw(__builtin_fmaf(st[n][r], sl2, -m));
+      st[n][r] = p;
+      rs += p;
+    }
+    l += rs;  // this lane's 16 keys; the other half's join at the end
+  }
+#pragma unroll
+  for (int n = 0; n < NT; ++n) {
+    const f16x8 p0 = frag_acc(st[n], 0), p1 = frag_acc(st[n], 1);
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      o[d] = mfma(fl.frag_t(vt + n * kTile, 0, d), p0, o[d]);  // O^T += V^T P^T
+      o[d] = mfma(fl.frag_t(vt + n * kTile, 1, d), p1, o[d]);
+    }
+  }
+}
+
+constexpr int kFwdTiles = 2;  // key tiles per stage
+
+__global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+attn_fwd_wide_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) char buf0[2 * kFwdTiles * kTile];
+  __shared__ __attribute__((aligned(16))) char buf1[2 * kFwdTiles * kTile];
+  int blk, head, start, end, q0;
+  if (!wide_item(a, a.n_blocks, blk, head)) return;
+  const int n_tok = static_cast<int>(a.n_tok);
+  if (!find_block<true, kWide>(a.cu, a.n_seq, n_tok, blk, start, end, q0)) return;
+  start = __builtin_amdgcn_readfirstlane(start);
+  end = __builtin_amdgcn_readfirstlane(end);
+  q0 = __builtin_amdgcn_readfirstlane(q0);
+  const int g = head / (a.h_q / a.h_kv);
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
+  const int64_t sq = static_cast<int64_t>(a.h_q) * kHD, skv = static_cast<int64_t>(a.h_kv) * kHD;
+  const f16* kh = a.k + start * skv + g * kHD;  // the row's first token
+  const f16* vh = a.v + start * skv + g * kHD;
+  const int qw = q0 + 32 * wave, qi = qw + col;  // this wave's first query, this lane's
+  const int last = min(q0 + kWide, end) - 1;
+  const int tiles = (last - start) / 32 + 1;            // key tiles of the block
+  const int mine = qw < end ? (qw - start) / 32 + 1 : 0;  // and of this wave
+  const int stages = (tiles + kFwdTiles - 1) / kFwdTiles;
+
+  const TileLane tl(wave, lane, skv);
+  const FragLane fl0(lane);
+  auto copy = [&](char* dst, int j) {
+#pragma unroll
+    for (int n = 0; n < kFwdTiles; ++n) {
+      const int t = kFwdTiles * j + n;
+      if (t >= tiles) break;
+      const int rows = end - start - 32 * t;
+      tl.copy(dst + n * kTile, wave, kh + 32 * t * skv, rows);
+      tl.copy(dst + (kFwdTiles + n) * kTile, wave, vh + 32 * t * skv, rows);
+    }
+  };
+  copy(buf0, 0);
+  f16x8 qf[8];
+  const f16* qrow = a.q + static_cast<int64_t>(min(qi, end - 1)) * sq + head * kHD;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) qf[s] = *reinterpret_cast<const f16x8*>(qrow + 8 * (2 * s + h));
+  f32x16 o[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) o[d] = f32x16{};
+  float m = -INFINITY, l = 0.0f;
+  stage_barrier();
+  auto stage = [&](const char* cur, char* next, int j) {
+    if (j + 1 < stages) copy(next, j + 1);
+    const char* vt = cur + kFwdTiles * kTile;
+    const FragLane fl = fl0.fresh();
+    const int left = mine - kFwdTiles * j;  // this wave's tiles from here on (wave-uniform)
+    const int k0 = start + 32 * kFwdTiles * j;
+    if (left >= 2)
+      fwd_keys<2>(fl, cur, vt, qf, o, m, l, a.scale_log2, left == 2, k0, qi, end, h);
+    else if (left == 1)
+      fwd_keys<1>(fl, cur, vt, qf, o, m, l, a.scale_log2, true, k0, qi, end, h);
+    stage_barrier();
+  };
+  for (int j = 0; j < stages; j += 2) {
+    stage(buf0, buf1, j);
+    if (j + 1 < stages) stage(buf1, buf0, j + 1);
+  }
+  if (mine == 0) return;
+  const float2 lp = half_pair(l);
+  const float L = lp.x + lp.y;
+  store_row(a.out + static_cast<int64_t>(qi) * sq + head * kHD, o, 1.0f / L, h, qi < end);
+  if (h == 0 && qi < end) a.lse[head * a.n_tok + qi] = (m + log2f(L)) * kLn2;
+}
+
+// LDS of the backward: the streamed tiles' two buffers (separate arrays, see TileLane::copy), and for
+// the dK / dV blocks the block's V rows and the streamed queries' lse and D.
+struct BwdLds {
+  char* buf0;
+  char* buf1;
+  char* v;
+  float* ld0;  // lse (log2 units) of 32 queries, then D
+  float* ld1;
+};
+
+// dQ of 128 queries: key tiles stream through LDS, each wave owns 32 queries (Q and dO fragments in
+// registers; D = rowsum(dO o O) from the same fragments).
+__device__ __forceinline__ void bwd_wide_dq(const AttnArgs& a, int blk, int head, const BwdLds& lds) {
+  int start, end, q0;
+  if (!find_block<true, kWide>(a.cu, a.n_seq, static_cast<int>(a.n_tok), blk, start, end, q0)) return;
+  start = __builtin_amdgcn_readfirstlane(start);
+  end = __builtin_amdgcn_readfirstlane(end);
+  q0 = __builtin_amdgcn_readfirstlane(q0);
+  const int g = head / (a.h_q / a.h_kv);
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
+  const int64_t sq = static_cast<int64_t>(a.h_q) * kHD, skv = static_cast<int64_t>(a.h_kv) * kHD;
+  const f16* kh = a.k + start * skv + g * kHD;
+  const f16* vh = a.v + start * skv + g * kHD;
+  const int qw = q0 + 32 * wave, qi = qw + col;
+  const int last = min(q0 + kWide, end) - 1;
+  const int tiles = (last - start) / 32 + 1;
+  const int mine = qw < end ? (qw - start) / 32 + 1 : 0;
+
+  const TileLane tl(wave, lane, skv);
+  const FragLane fl0(lane);
+  auto copy = [&](char* dst, int j) {
+    const int rows = end - start - 32 * j;
+    tl.copy(dst, wave, kh + 32 * j * skv, rows);
+    tl.copy(dst + kTile, wave, vh + 32 * j * skv, rows);
+  };
+  copy(lds.buf0, 0);
+  const int qr = min(qi, end - 1);
+  const int64_t off = static_cast<int64_t>(qr) * sq + head * kHD;
+  f16x8 qf[8], df[8];
+  float ds = 0.0f;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) {
+    qf[s] = *reinterpret_cast<const f16x8*>(a.q + off + 8 * (2 * s + h));
+    df[s] = *reinterpret_cast<const f16x8*>(a.dout + off + 8 * (2 * s + h));
+    const f16x8 ov = *reinterpret_cast<const f16x8*>(a.o + off + 8 * (2 * s + h));
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      ds = __builtin_fmaf(static_cast<float>(ov[e]), static_cast<float>(df[s][e]), ds);
+  }
+  const float2 dp2 = half_pair(ds);
+  const float dsum = dp2.x + dp2.y;
+  const float lse2 = a.lse[head * a.n_tok + qr] * kLog2e;
+  f32x16 dq[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) dq[d] = f32x16{};
+  stage_barrier();
+  auto stage = [&](const char* kt, char* next, int j) {
+    if (j + 1 < tiles) copy(next, j + 1);
+    const char* vt = kt + kTile;
+    const FragLane fl = fl0.fresh();
+    if (j < mine) {
+      f32x16 st = f32x16{}, dp = f32x16{};
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        st = mfma(fl.frag(kt, s), qf[s], st);  // S^T = K Q^T
+        dp = mfma(fl.frag(vt, s), df[s], dp);  // dP^T = V dO^T
+      }
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        st[r] = exp2_raw(__builtin_fmaf(st[r], a.scale_log2, -lse2)) * (dp[r] - dsum);
+      if (j == mine - 1) {  // the diagonal tile
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int key = start + 32 * j + acc_row(r, h);
+          st[r] = (key <= qi && key < end) ? st[r] : 0.0f;
+        }
+      }
+      const f16x8 s0 = frag_acc(st, 0), s1 = frag_acc(st, 1);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        dq[d] = mfma(fl.frag_t(kt, 0, d), s0, dq[d]);  // dQ^T += K^T dS^T
+        dq[d] = mfma(fl.frag_t(kt, 1, d), s1, dq[d]);
+      }
+    }
+    stage_barrier();
+  };
+  for (int j = 0; j < tiles; j += 2) {
+    stage(lds.buf0, lds.buf1, j);
+    if (j + 1 < tiles) stage(lds.buf1, lds.buf0, j + 1);
+  }
+  if (mine == 0) return;
+  store_row(a.out + static_cast<int64_t>(qi) * sq + head * kHD, dq, a.scale, h, qi < end);
+}
+
+// dK and dV of 128 keys for one query head: Q and dO tiles stream through LDS with their lse and D,
+// each wave owns 32 keys (K fragments in registers, V fragments from LDS).
+__device__ __forceinline__ void bwd_wide_dkdv(const AttnArgs& a, int blk, int head,
+                                              const BwdLds& lds) {
+  int start, end, k0;
+  if (!find_block<false, kWide>(a.cu, a.n_seq, static_cast<int>(a.n_tok), blk, start, end, k0)) return;
+  start = __builtin_amdgcn_readfirstlane(start);
+  end = __builtin_amdgcn_readfirstlane(end);
+  k0 = __builtin_amdgcn_readfirstlane(k0);
+  const int grp = a.h_q / a.h_kv, g = head / grp;
+  const int tid = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lane = tid & 63, h = lane >> 5, col = lane & 31;
+  const int64_t sq = static_cast<int64_t>(a.h_q) * kHD, skv = static_cast<int64_t>(a.h_kv) * kHD;
+  const f16* qh = a.q + k0 * sq + head * kHD;  // from the block's first key on
+  const f16* doh = a.dout + k0 * sq + head * kHD;
+  const f16* oh = a.o + k0 * sq + head * kHD;
+  const float* lse = a.lse + head * a.n_tok + k0;
+  const int kw = k0 + 32 * wave, kj = kw + col;
+  const int tiles = (end - k0 + 31) / 32;
+
+  const TileLane tl(wave, lane, sq);
+  const FragLane fl0(lane);
+  f16x8 orow[2];  // the O chunks of the dO chunks this lane copies
+  float lr = 0.0f;
+  auto copy = [&](char* dst, int j) {
+    const int rows = end - k0 - 32 * j;
+    tl.copy(dst, wave, qh + 32 * j * sq, rows);
+    tl.copy(dst + kTile, wave, doh + 32 * j * sq, rows);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      orow[i] = *reinterpret_cast<const f16x8*>(reinterpret_cast<const char*>(oh + 32 * j * sq) +
+                                                tl.at(i, rows));
+    if (tid < kBlk) lr = lse[32 * j + min(tid, rows - 1)];
+  };
+  // D of the rows this wave copied (its copies have landed): each lane's 8 products, then the sum
+  // over the 16 lanes of a row.
+  auto finish = [&](const char* dst, float* ld) {
+    __builtin_amdgcn_s_waitcnt(0x0070 | 0x0F00);  // vmcnt(0)
+    if (tid < kBlk) ld[tid] = lr * kLog2e;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const f16x8 y = *reinterpret_cast<const f16x8*>(dst + kTile + (2 * wave + i) * 1024 + lane * 16);
+      float s = 0.0f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        s = __builtin_fmaf(static_cast<float>(orow[i][e]), static_cast<float>(y[e]), s);
+      s += row_ror<8>(s);
+      s += row_ror<4>(s);
+      s += row_ror<2>(s);
+      s += row_ror<1>(s);
+      if ((lane & 15) == 0) ld[kBlk + tl.row[i]] = s;
+    }
+  };
+  copy(lds.buf0, 0);
+  {
+    const TileLane tv(wave, lane, skv);
+#pragma unroll
+    for (int n = 0; n < 4; ++n)
+      if (k0 + 32 * n < end)
+        tv.copy(lds.v + n * kTile, wave, a.v + (k0 + 32 * n) * skv + g * kHD, end - k0 - 32 * n);
+  }
+  f16x8 kf[8];
+  const f16* krow = a.k + static_cast<int64_t>(min(kj, end - 1)) * skv + g * kHD;
+#pragma unroll
+  for (int s = 0; s < 8; ++s) kf[s] = *reinterpret_cast<const f16x8*>(krow + 8 * (2 * s + h));
+  f32x16 dk[4], dv[4];
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    dk[d] = f32x16{};
+    dv[d] = f32x16{};
+  }
+  finish(lds.buf0, lds.ld0);
+  stage_barrier();
+  const char* vt = lds.v + wave * kTile;
+  auto stage = [&](const char* qt, const float* ld, char* next, float* ldn, int j) {
+    if (j + 1 < tiles) copy(next, j + 1);
+    const char* dt = qt + kTile;
+    const FragLane fl = fl0.fresh();
+    if (j >= wave) {  // query tiles before the wave's keys see none of them
+      f32x16 st = f32x16{}, dp = f32x16{};
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        st = mfma(fl.frag(qt, s), kf[s], st);                          // S = Q K^T
+        dp = mfma(fl.frag(dt, s), fl.frag(vt, s), dp);  // dP = dO V^T
+      }
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        const f32x4 lv = *reinterpret_cast<const f32x4*>(ld + 8 * b + 4 * h);
+        const f32x4 dd = *reinterpret_cast<const f32x4*>(ld + kBlk + 8 * b + 4 * h);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int r = 4 * b + i;
+          const float p = exp2_raw(__builtin_fmaf(st[r], a.scale_log2, -lv[i]));
+          st[r] = p;                    // P
+          dp[r] = p * (dp[r] - dd[i]);  // dS
+        }
+      }
+      if (j == wave || j == tiles - 1) {  // the diagonal tile, and rows past the row's end
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int qi = k0 + 32 * j + acc_row(r, h);
+          const bool in = kj <= qi && qi < end;
+          st[r] = in ? st[r] : 0.0f;
+          dp[r] = in ? dp[r] : 0.0f;
+        }
+      }
+      const f16x8 p0 = frag_acc(st, 0), p1 = frag_acc(st, 1);
+      const f16x8 s0 = frag_acc(dp, 0), s1 = frag_acc(dp, 1);
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        dv[d] = mfma(p0, fl.frag_t(dt, 0, d), dv[d]);  // dV += P^T dO
+        dv[d] = mfma(p1, fl.frag_t(dt, 1, d), dv[d]);
+        dk[d] = mfma(s0, fl.frag_t(qt, 0, d), dk[d]);  // dK += dS^T Q
+        dk[d] = mfma(s1, fl.frag_t(qt, 1, d), dk[d]);
+      }
+    }
+    if (j + 1 < tiles) finish(next, ldn);
+    stage_barrier();
+  };
+  for (int j = 0; j < tiles; j += 2) {
+    stage(lds.buf0, lds.ld0, lds.buf1, lds.ld1, j);
+    if (j + 1 < tiles) stage(lds.buf1, lds.ld1, lds.buf0, lds.ld0, j + 1);
+  }
+  // This head's fp32 partial: keys are accumulator rows, head dims lanes.
+#pragma unroll
+  for (int d = 0; d < 4; ++d)
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int key = kw + acc_row(r, h);
+      if (key < end) {
+        const int64_t o = (static_cast<int64_t>(head) * a.n_tok + key) * kHD + 32 * d + col;
+        store_partial(a.dk_part + o, dk[d][r] * a.scale);
+        store_partial(a.dv_part + o, dv[d][r]);
+      }
+    }
+}
+
+// dk / dv [key, g, :] = fp16(sum over the KV group's heads in head order) of the partials: a launch
+// of its own, 4 us at 707 tokens. Summed by the last of a group's blocks to arrive it took 7 us
+// with 32-token blocks and 24 us with 128-token ones (one block reading 128 keys x 6 heads from
+// beyond its L2 at the end of the launch). Thread = 4 head dims of one key; y = dk, dv.
+__global__ __launch_bounds__(256) void attn_group_sum_kernel(AttnArgs a) {
+  const int grp = a.h_q / a.h_kv;
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  const int c = 4 * static_cast<int>(t & 31), g = static_cast<int>((t >> 5) % a.h_kv);
+  const int64_t key = (t >> 5) / a.h_kv;
+  if (key >= a.n_tok) return;
+  const float* src = (blockIdx.y == 0 ? a.dk_part : a.dv_part) +
+                     (static_cast<int64_t>(g) * grp * a.n_tok + key) * kHD + c;
+  f32x4 s = *reinterpret_cast<const f32x4*>(src);
+#pragma unroll 4
+  for (int j = 1; j < grp; ++j) s += *reinterpret_cast<const f32x4*>(src + j * a.n_tok * kHD);
+  f16x4 w;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = from_f32<f16>(s[i]);
+  *reinterpret_cast<f16x4*>((blockIdx.y == 0 ? a.dk : a.dv) + (key * a.h_kv + g) * kHD + c) = w;
+}
+
+// Blocks below n_blocks are dK / dV blocks (dispatched first), the rest dQ blocks.
+__global__ __launch_bounds__(64 * kW) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+attn_bwd_wide_kernel(AttnArgs a) {
+  __shared__ __attribute__((aligned(16))) char buf0[2 * kTile];
+  __shared__ __attribute__((aligned(16))) char buf1[2 * kTile];
+  __shared__ __attribute__((aligned(16))) char v[4 * kTile];
+  __shared__ __attribute__((aligned(16))) float ld0[2 * kBlk];
+  __shared__ __attribute__((aligned(16))) float ld1[2 * kBlk];
+  int blk, head;
+  if (!wide_item(a, 2 * a.n_blocks, blk, head)) return;
+  const BwdLds lds{buf0, buf1, v, ld0, ld1};
+  if (blk < a.n_blocks)
+    bwd_wide_dkdv(a, blk, head, lds);
+  else
+    bwd_wide_dq(a, blk - a.n_blocks, head, lds);
+}
+
+// Whether a batch takes the wide kernels: when its 128-token blocks are at least min_blocks, or
+// kShortWideBlocks if its rows average at most one such block. The lines are where both kernels
+// take the same time (256 CUs; 12 / 2 heads, old -> wide): forward 2,048 tokens = 192 blocks in
+// rows of 512 18.0 -> 17.0 us, as one row 43 -> 48, 3,072 tokens 37 -> 28; backward with partials
+// 1,536 tokens (144 blocks) in rows of 512 39 -> 34 us, of 1,024 and 512 50 -> 55, 2,048 tokens as
+// one row 113 -> 102, in rows of 512 45 -> 34; 14 rows of 100 forward 11.4 -> 8.6, backward
+// 27 -> 17. Scores are scaled after their maximum is taken, hence scale > 0.
+constexpr int kFwdWideBlocks = 256, kBwdWideBlocks = 192, kShortWideBlocks = 128;
+
+bool wide(int64_t n_tok, int n_seq, int h_q, float scale, int min_blocks) {
+  const int64_t blocks = (n_tok + kWide - 1) / kWide * h_q;
+  return scale > 0.0f &&
+         blocks >= (n_tok <= kWide * static_cast<int64_t>(n_seq) ? kShortWideBlocks : min_blocks);
+}
+
+// Bound of the 128-token blocks over all rows (at most the caller's bound of 32-token blocks).
+int wide_blocks(int64_t n_tok, int n_seq, int max_blocks) {
+  return static_cast<int>(std::min<int64_t>((n_tok + kWide - 1) / kWide + n_seq, max_blocks));
+}
+
+unsigned wide_grid(int n_blocks, const AttnArgs& a) {
+  const int64_t chunk = 8 * (a.h_q / a.h_kv), items = static_cast<int64_t>(n_blocks) * a.h_q;
+  return static_cast<unsigned>((items + chunk - 1) / chunk * chunk);
 }
 
 int check(const char* fn, const void* q, const void* k, const void* v, const int32_t* cu,
@@ -776,6 +1298,12 @@ extern "C" int rus_attn_varlen_fwd(const void* q, const void* k, const void* v,
   a.h_kv = h_kv;
   a.scale = scale;
   a.scale_log2 = scale * kLog2e;
+  if (wide(n_tokens, n_seq, h_q, scale, kFwdWideBlocks)) {
+    a.n_blocks = wide_blocks(n_tokens, n_seq, max_blocks);
+    hipLaunchKernelGGL(attn_fwd_wide_kernel, dim3(wide_grid(a.n_blocks, a)), dim3(64 * kW), 0,
+                       static_cast<hipStream_t>(stream), a);
+    return check_launch(fn);
+  }
   hipLaunchKernelGGL(attn_fwd_kernel, dim3(h_q, max_blocks), dim3(64 * kW), 0,
                      static_cast<hipStream_t>(stream), a);
   return check_launch(fn);
@@ -827,10 +1355,19 @@ static int attn_bwd(const char* fn, const void* q, const void* k, const void* v,
   a.out = static_cast<f16*>(dq);
   a.dk = static_cast<f16*>(dk);
   a.dv = static_cast<f16*>(dv);
-  a.counters = counters;
   a.max_blocks = max_blocks;
-  a.group_sum = group_sum ? 1 : 0;
-  hipLaunchKernelGGL(attn_bwd_kernel, dim3(h_q, 2 * max_blocks), dim3(64 * kWB), 0, st, a);
+  if (wide(n_tokens, n_seq, h_q, scale, kBwdWideBlocks)) {
+    a.n_blocks = wide_blocks(n_tokens, n_seq, max_blocks);
+    hipLaunchKernelGGL(attn_bwd_wide_kernel, dim3(wide_grid(2 * a.n_blocks, a)), dim3(64 * kW), 0,
+                       st, a);
+  } else {
+    hipLaunchKernelGGL(attn_bwd_kernel, dim3(h_q, 2 * max_blocks), dim3(64 * kWB), 0, st, a);
+  }
+  if (int e = check_launch(fn)) return e;
+  if (!group_sum) return RUS_OK;
+  hipLaunchKernelGGL(attn_group_sum_kernel,
+                     dim3(static_cast<unsigned>((n_tokens * h_kv * 32 + 255) / 256), 2), dim3(256),
+                     0, st, a);
   return check_launch(fn);
 }
 

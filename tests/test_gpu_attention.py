@@ -227,3 +227,14 @@ def test_rope_mid_over_attention_partials_equals_group_sum_path():
     torch.cuda.synchronize()
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("lens,hq,hkv", [
+    ([1100, 385, 129, 128, 127, 33, 1, 950], 12, 2),  # edges of the 128-token blocks
+    ([1537, 2048, 600], 8, 8),                         # no GQA
+    ([2047, 2050], 8, 1),                              # MQA
+])
+def test_attention_wide_blocks_match_oracle(lens, hq, hkv):
+    """Batches large enough for the 128-token blocks (edges of blocks and tiles, rows shorter than a
+    block, ragged offsets), with large scores in one of them so that the running maximum moves."""
+    _run(lens, hq, hkv, seed=sum(lens) + hq, qk_scale=3.0 if hkv == 1 else 1.0)
