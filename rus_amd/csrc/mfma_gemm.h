@@ -353,54 +353,94 @@ __device__ __forceinline__ void mainloop_t(const GemmArgs& g, const Tile& tl, ch
 // K-contiguous operand) instead of 16 half lines, which doubles what the copy path delivers per
 // CU. Rows of 128 bytes, the 16-byte chunk c of row r stored at c ^ ((r >> 1) & 7): the 16 rows a
 // quarter wave reads at one chunk then cover all 64 banks once. N-contiguous B: 64 K rows of 512
-// bytes per stage (the chunk c of row r at c ^ ((r & 3) << 2), as in the 32-deep stages). The
-// copies of stage k + 2 are issued after the barrier that ends the reads of stage k; one barrier
-// per 64 K.
+// bytes per stage (the chunk c of row r at c ^ ((r & 3) << 2), as in the 32-deep stages).
+//
+// A stage runs in four phases of eight MFMAs, one quadrant of the wave's tile (64 x 32) over all
+// 64 K each: A0 B0, A0 B1, A1 B0, A1 B1. Every LDS read of a stage is then issued by the second
+// phase and done before the third, so the stage's one barrier falls between them, with half of its
+// MFMAs ready in registers: the copies of stage k + 2 (into the buffer just read) and the first
+// reads of stage k + 1 go out between those MFMAs. Against one K step's fragments at a time, with
+// the copies and the next reads issued in a burst after the barrier, before the stage's last MFMAs:
+// 4096^3 127 -> 121 us (1,140 TFLOP/s), logits of 2,048 tokens x 32,768 rows 199 -> 186, of 744 x
+// 76,544 204 -> 195, the split-K product at 707 tokens 47.8 -> 46.5 (same bits). What is left is
+// power and the copies: with zero operands the same 4096^3 takes 83 us (the clock stays up), and
+// without copies 8192^3 runs at 1,430 TFLOP/s on random and 2,145 on zero operands.
 constexpr int kDK64 = 64;
 constexpr int kStage64 = 2 * kBM * kDK64 * 2;  // 64 KiB
 constexpr int kSmem64 = 2 * kStage64;          // 128 KiB
 
-template <int NW, bool KN>
+// Fragments of one 64-row half of A (2 MFMA tiles) or one 32-column tile of B, all four K steps.
+struct FragA {
+  u32x4v v[4][2];
+};
+template <bool KN>
+struct FragB;
+template <>
+struct FragB<false> {
+  u32x4v v[4];
+  __device__ __forceinline__ f16x8 get(int kk) const { return __builtin_bit_cast(f16x8, v[kk]); }
+};
+template <>
+struct FragB<true> {
+  u32x2v lo[4], hi[4];
+  __device__ __forceinline__ f16x8 get(int kk) const {
+    const u32x4v b = {lo[kk].x, lo[kk].y, hi[kk].x, hi[kk].y};
+    return __builtin_bit_cast(f16x8, b);
+  }
+};
+
+// Every LDS read issued so far has returned; ties the fragments read since the last wait.
+__device__ __forceinline__ void wait_set(FragA& f) {
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(f.v[0][0]), "+v"(f.v[0][1]), "+v"(f.v[1][0]), "+v"(f.v[1][1]),
+                 "+v"(f.v[2][0]), "+v"(f.v[2][1]), "+v"(f.v[3][0]), "+v"(f.v[3][1]));
+}
+__device__ __forceinline__ void wait_set(FragB<false>& f) {
+  asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f.v[0]), "+v"(f.v[1]), "+v"(f.v[2]), "+v"(f.v[3]));
+}
+__device__ __forceinline__ void wait_set(FragB<true>& f) {
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(f.lo[0]), "+v"(f.lo[1]), "+v"(f.lo[2]), "+v"(f.lo[3]), "+v"(f.hi[0]),
+                 "+v"(f.hi[1]), "+v"(f.hi[2]), "+v"(f.hi[3]));
+}
+
+template <bool KN>
 __device__ __forceinline__ void mainloop_k64(const GemmArgs& g, const Tile& tl, char* smem,
-                                             f32x16 (&acc)[kMT][16 / NW]) {
-  static_assert(NW == 4 || NW == 8, "four waves of 128 x 128 or eight of 128 x 64");
-  static_assert(!KN || NW == 8, "the N-contiguous B layout runs on eight waves");
-  constexpr int NT = 16 / NW;         // 32-column MFMA tiles per wave
-  constexpr int RW = kBN / (NW / 2);  // B rows (N) per wave: 128 or 64
-  constexpr int CP = 32 / NW;         // copies per wave per operand and stage: 8 or 4
+                                             f32x16 (&acc)[kMT][2]) {
+  constexpr int CP = 4;  // copies per wave per operand and stage
   constexpr int PER = 2 * CP;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6));
-  const int wm = wave / (NW / 2), wn = wave % (NW / 2);
+  const int wm = wave >> 2, wn = wave & 3;
   const int kb = tl.split * g.k_per_split;
   const int ke = min(kb + g.k_per_split, g.K);
   const int KT = ke > kb ? (ke - kb) / kDK64 : 0;
 #pragma unroll
   for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x16{};
+    for (int nt = 0; nt < 2; ++nt) acc[mt][nt] = f32x16{};
   if (KT == 0) {
     __syncthreads();
     return;
   }
-  // Copies: instruction i of wave w fills bytes 1024 (NW i + w) .. +1024 of the stage's A tile
-  // (rows 8 (NW i + w) .. +8; lane l covers row + l/8 at position l%8, i.e. the chunk
+  // Copies: instruction i of wave w fills bytes 1024 (8 i + w) .. +1024 of the stage's A tile
+  // (rows 8 (8 i + w) .. +8; lane l covers row + l/8 at position l%8, i.e. the chunk
   // (l%8) ^ ((row >> 1) & 7)) and the same bytes of the B tile (K-contiguous as A; N-contiguous:
-  // K rows 2 (NW i + w) + l/32 of 512 bytes, lane l at position l%32 of its row r, the chunk
+  // K rows 2 (8 i + w) + l/32 of 512 bytes, lane l at position l%32 of its row r, the chunk
   // (l%32) ^ ((r & 3) << 2), columns n0 + 8 chunk .. +8).
   const char* gA = reinterpret_cast<const char*>(g.A);
   const char* gB = reinterpret_cast<const char*>(g.B);
   uint32_t oa[CP], ob[CP];
 #pragma unroll
   for (int i = 0; i < CP; ++i) {
-    const int row = 8 * (NW * i + wave) + (lane >> 3);
+    const int row = 8 * (8 * i + wave) + (lane >> 3);
     const int ch = (lane & 7) ^ ((row >> 1) & 7);
     // Rows (columns) past the matrix edge re-read the last one: finite values the epilogues
     // discard.
     const int ra_ = min(tl.m0 + row, g.M - 1);
     oa[i] = static_cast<uint32_t>((ra_ * g.lda + kb + ch * 8) * 2);
     if constexpr (KN) {
-      const int krow = 2 * (NW * i + wave) + (lane >> 5);
+      const int krow = 2 * (8 * i + wave) + (lane >> 5);
       const int col = min(tl.n0 + 8 * ((lane & 31) ^ ((krow & 3) << 2)), g.N - 8);
       ob[i] = static_cast<uint32_t>(((kb + krow) * g.ldb + col) * 2);
     } else {
@@ -409,81 +449,78 @@ __device__ __forceinline__ void mainloop_k64(const GemmArgs& g, const Tile& tl, 
     }
   }
   const uint32_t bstep = KN ? static_cast<uint32_t>(kDK64 * g.ldb * 2) : kDK64 * 2;
-  auto issue = [&](int k) {  // stage k's copies into buffer k % 2
+  auto copy = [&](int k, auto I) {  // copy I of stage k into buffer k % 2
+    constexpr int i = decltype(I)::value;
     char* st = smem + (k & 1) * kStage64 + wave * 1024;
-    const uint32_t abytes = k * (kDK64 * 2), bbytes = k * bstep;
-#pragma unroll
-    for (int i = 0; i < CP; ++i) {
-      __builtin_amdgcn_global_load_lds(gA + oa[i] + abytes, (lds_void_ptr)(st + i * NW * 1024),
-                                       16, 0, 0);
-      __builtin_amdgcn_global_load_lds(gB + ob[i] + bbytes,
-                                       (lds_void_ptr)(st + kBM * 128 + i * NW * 1024), 16, 0, 0);
-    }
+    __builtin_amdgcn_global_load_lds(gA + oa[i] + static_cast<uint32_t>(k) * (kDK64 * 2),
+                                     (lds_void_ptr)(st + i * 8192), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds(gB + ob[i] + static_cast<uint32_t>(k) * bstep,
+                                     (lds_void_ptr)(st + kBM * 128 + i * 8192), 16, 0, 0);
+  };
+  using C0 = std::integral_constant<int, 0>;
+  using C1 = std::integral_constant<int, 1>;
+  using C2 = std::integral_constant<int, 2>;
+  using C3 = std::integral_constant<int, 3>;
+  auto issue = [&](int k) {
+    copy(k, C0{});
+    copy(k, C1{});
+    copy(k, C2{});
+    copy(k, C3{});
   };
   // Fragment addresses. A: row wm*128 + (l & 31) (+ 32 per MFMA tile: immediate 4096), chunk
   // 2 kk + l/32 at position chunk ^ ((l >> 1) & 7) (the low row bits are those of l). B
-  // K-contiguous likewise (rows wn*RW + ...); N-contiguous: lane l of group g = l/16 (j = l%16)
+  // K-contiguous likewise (rows wn*64 + ...); N-contiguous: lane l of group g = l/16 (j = l%16)
   // reads K row 16 kk + 8 (g/2) + j/4 (+ 4 for the high half), columns wn*64 + 32 nt + 16 (g%2)
   // + 4 (j%4).
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_ptr)smem));
-  const int sw = (lane >> 1) & 7, half = lane >> 5;
-  uint32_t cpos[4];
-#pragma unroll
-  for (int kk = 0; kk < 4; ++kk) cpos[kk] = static_cast<uint32_t>(((2 * kk + half) ^ sw) << 4);
-  const uint32_t arow = lds0 + (wm * kWM + (lane & 31)) * 128;
-  const uint32_t brow = lds0 + kBM * 128 + (wn * RW + (lane & 31)) * 128;
-  uint32_t bk[NT];
+  const int half = lane >> 5;
+  const uint32_t c0 = static_cast<uint32_t>((half ^ ((lane >> 1) & 7)) << 4);
+  const uint32_t arow = lds0 + (wm * kWM + (lane & 31)) * 128 + c0;  // kk: ^ (kk << 5)
+  const uint32_t brow = lds0 + kBM * 128 + (wn * 64 + (lane & 31)) * 128 + c0;
+  uint32_t bk[2];
   if constexpr (KN) {
     const int j = lane & 15, nh = (lane >> 4) & 1;
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const int col = wn * RW + nt * 32 + 16 * nh + 4 * (j & 3);
+    for (int nt = 0; nt < 2; ++nt) {
+      const int col = wn * 64 + nt * 32 + 16 * nh + 4 * (j & 3);
       bk[nt] = lds0 + kBM * 128 + (8 * half + (j >> 2)) * kKNRowBytes +
                (((col >> 3) ^ ((j >> 2) << 2)) << 4) + (col & 7) * 2;
     }
   }
-  u32x4v fa[2][kMT], fb[2][NT];
-  u32x2v lo[2][NT], hi[2][NT];
-  // Fragments of K step kk (0..3) of the stage at byte offset sb into register set S.
-  auto read = [&](auto S, uint32_t sb, int kk) {
-    constexpr int s = decltype(S)::value;
-    const uint32_t a = arow + sb + cpos[kk];
-    fa[s][0] = lds_read16<0>(a);
-    fa[s][1] = lds_read16<4096>(a);
-    fa[s][2] = lds_read16<8192>(a);
-    fa[s][3] = lds_read16<12288>(a);
+  FragA a0, a1;
+  FragB<KN> b0, b1;
+  auto read_a = [&](FragA& f, uint32_t sb, auto KK, auto H) {
+    constexpr int kk = decltype(KK)::value, h = decltype(H)::value;
+    const uint32_t a = (arow ^ (kk << 5)) + sb;
+    f.v[kk][0] = lds_read16<h * 8192>(a);
+    f.v[kk][1] = lds_read16<h * 8192 + 4096>(a);
+  };
+  auto read_b = [&](FragB<KN>& f, uint32_t sb, auto KK, auto N) {
+    constexpr int kk = decltype(KK)::value, nt = decltype(N)::value;
     if constexpr (KN) {
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt) {
-        lo[s][nt] = lds_read8_tr<0>(bk[nt] + sb + kk * 16 * kKNRowBytes);
-        hi[s][nt] = lds_read8_tr<4 * kKNRowBytes>(bk[nt] + sb + kk * 16 * kKNRowBytes);
-      }
+      f.lo[kk] = lds_read8_tr<kk * 16 * kKNRowBytes>(bk[nt] + sb);
+      f.hi[kk] = lds_read8_tr<kk * 16 * kKNRowBytes + 4 * kKNRowBytes>(bk[nt] + sb);
     } else {
-      const uint32_t b = brow + sb + cpos[kk];
-      fb[s][0] = lds_read16<0>(b);
-      fb[s][1] = lds_read16<4096>(b);
-      if constexpr (NT == 4) {
-        fb[s][2] = lds_read16<8192>(b);
-        fb[s][3] = lds_read16<12288>(b);
-      }
+      f.v[kk] = lds_read16<nt * 4096>((brow ^ (kk << 5)) + sb);
     }
   };
-  auto wait = [&](auto S) {
-    constexpr int s = decltype(S)::value;
-    if constexpr (KN)
-      wait_frags_kn<NT>(fa[s], lo[s], hi[s]);
-    else
-      wait_frags<NT>(fa[s], fb[s]);
+  auto mma = [&](const FragA& fa, const FragB<KN>& fb, auto KK, auto H, auto N) {
+    constexpr int kk = decltype(KK)::value, h = decltype(H)::value, nt = decltype(N)::value;
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+      acc[2 * h + m][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
+          __builtin_bit_cast(f16x8, fa.v[kk][m]), fb.get(kk), acc[2 * h + m][nt], 0, 0, 0);
   };
-  auto mma = [&](auto S) {
-    constexpr int s = decltype(S)::value;
-    if constexpr (KN)
-      mma16_kn<NT>(fa[s], lo[s], hi[s], acc);
-    else
-      mma16<NT>(fa[s], fb[s], acc);
+  auto each = [&](auto f) {  // the four K steps, kept apart so that what f interleaves stays so
+    f(C0{});
+    __builtin_amdgcn_sched_barrier(0);
+    f(C1{});
+    __builtin_amdgcn_sched_barrier(0);
+    f(C2{});
+    __builtin_amdgcn_sched_barrier(0);
+    f(C3{});
+    __builtin_amdgcn_sched_barrier(0);
   };
-  using S0 = std::integral_constant<int, 0>;
-  using S1 = std::integral_constant<int, 1>;
   issue(0);
   if (KT > 1) issue(1);
   if (KT > 1)
@@ -491,38 +528,45 @@ __device__ __forceinline__ void mainloop_k64(const GemmArgs& g, const Tile& tl, 
   else
     wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();  // ... and every wave's
-  read(S0{}, 0, 0);
-  wait(S0{});
-  for (int k = 0; k < KT; ++k) {
-    const uint32_t sb = (k & 1) * kStage64;
-    read(S1{}, sb, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(S0{});
-    __builtin_amdgcn_sched_barrier(0);
-    wait(S1{});
-    read(S0{}, sb, 2);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(S1{});
-    __builtin_amdgcn_sched_barrier(0);
-    wait(S0{});
-    read(S1{}, sb, 3);
-    __builtin_amdgcn_sched_barrier(0);
-    mma(S0{});
-    __builtin_amdgcn_sched_barrier(0);
-    wait(S1{});
-    if (k + 1 < KT) {
+  each([&](auto kk) { read_a(a0, 0, kk, C0{}); });
+  each([&](auto kk) { read_b(b0, 0, kk, C0{}); });
+  wait_set(a0);
+  wait_set(b0);
+  // MORE: stages beyond this one (0, 1, 2 = two or more: the copies of stage k + 2 go out).
+  auto stage = [&](int k, auto MORE) {
+    constexpr int more = decltype(MORE)::value;
+    const uint32_t sb = (k & 1) * kStage64, sn = sb ^ kStage64;
+    each([&](auto kk) {
+      read_b(b1, sb, kk, C1{});
+      mma(a0, b0, kk, C0{}, C0{});
+    });
+    wait_set(b1);
+    each([&](auto kk) {
+      read_a(a1, sb, kk, C1{});
+      mma(a0, b1, kk, C0{}, C1{});
+    });
+    wait_set(a1);
+    if constexpr (more > 0) {
       // Stage k + 1 has landed for every wave, and every wave has read stage k: its buffer
       // takes stage k + 2.
       wait_vmcnt<0>();
       __builtin_amdgcn_s_barrier();
-      if (k + 2 < KT) issue(k + 2);
-      read(S0{}, sb ^ kStage64, 0);
     }
-    __builtin_amdgcn_sched_barrier(0);
-    mma(S1{});
-    __builtin_amdgcn_sched_barrier(0);
-    if (k + 1 < KT) wait(S0{});
-  }
+    each([&](auto kk) {
+      mma(a1, b0, kk, C1{}, C0{});
+      if constexpr (more > 0) read_a(a0, sn, kk, C0{});
+      if constexpr (more > 1) copy(k + 2, kk);
+    });
+    if constexpr (more > 0) wait_set(a0);
+    each([&](auto kk) {
+      if constexpr (more > 0) read_b(b0, sn, kk, C0{});
+      mma(a1, b1, kk, C1{}, C1{});
+    });
+    if constexpr (more > 0) wait_set(b0);
+  };
+  for (int k = 0; k + 2 < KT; ++k) stage(k, C2{});
+  if (KT > 1) stage(KT - 2, C1{});
+  stage(KT - 1, C0{});
   __syncthreads();  // the epilogues reuse the LDS
 }
 
@@ -533,13 +577,13 @@ __device__ __forceinline__ void mainloop(const GemmArgs& g, const Tile& tl, char
 
 __device__ __forceinline__ void mainloop(const GemmArgs& g, const Tile& tl, char* smem,
                                          f32x16 (&acc)[kMT][2]) {
-  mainloop_k64<8, false>(g, tl, smem, acc);
+  mainloop_k64<false>(g, tl, smem, acc);
 }
 
 // The eight-wave mainloop with B stored [K, ldb] N-contiguous.
 __device__ __forceinline__ void mainloop_kn(const GemmArgs& g, const Tile& tl, char* smem,
                                             f32x16 (&acc)[kMT][2]) {
-  mainloop_k64<8, true>(g, tl, smem, acc);
+  mainloop_k64<true>(g, tl, smem, acc);
 }
 
 // Eight waves (two per SIMD): the accumulators of a 128 x 64 wave tile leave room for a second
