@@ -23,15 +23,30 @@ __device__ __forceinline__ f16x8 ld8(const f16* p) { return *reinterpret_cast<co
 
 __device__ __forceinline__ f16x8 zero8() { return f16x8{0, 0, 0, 0, 0, 0, 0, 0}; }
 
-// The reference's fp16 dropout of 8 values (keep bit sh + i of word w for value i).
-__device__ __forceinline__ f16x8 drop8(f16x8 x, uint32_t w, int sh, float scale) {
+// The reference's fp16 dropout of 8 values (keep bit sh + i of word w for value i): the scaled
+// values, then the dropped ones cleared, two per 32-bit word.
+__device__ __forceinline__ f16x8 scale8(f16x8 x, float scale) {
   f16x8 r;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const f16 v = from_f32<f16>(static_cast<float>(x[i]) * scale);
-    r[i] = (w >> (sh + i)) & 1u ? v : static_cast<f16>(0.0f);
-  }
+  for (int i = 0; i < 8; ++i) r[i] = from_f32<f16>(static_cast<float>(x[i]) * scale);
   return r;
+}
+
+__device__ __forceinline__ f16x8 keep8(f16x8 x, uint32_t w, int sh) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  u32x4 v = __builtin_bit_cast(u32x4, x);
+  const uint32_t b = w >> sh;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {  // each keep bit sign-extended over its half word
+    const uint32_t lo = static_cast<uint32_t>(static_cast<int32_t>(b << (31 - 2 * i)) >> 31) & 0xffffu;
+    const uint32_t hi = static_cast<uint32_t>(static_cast<int32_t>(b << (30 - 2 * i)) >> 31) & 0xffff0000u;
+    v[i] &= lo | hi;
+  }
+  return __builtin_bit_cast(f16x8, v);
+}
+
+__device__ __forceinline__ f16x8 drop8(f16x8 x, uint32_t w, int sh, float scale) {
+  return keep8(scale8(x, scale), w, sh);
 }
 
 struct DownRows {
@@ -77,20 +92,46 @@ inline int lora_rows_args(const char* fn, const rus_lora_rows& q, DownRows& a) {
 constexpr int kDownRows = 4;             // tokens per block
 constexpr int kDownParkFloats = 4 * 128;  // LDS the block's four wave sums take
 
-// mid_q / mid_v of tokens t0 .. t0 + 3 (those below n_tok), by all four waves of the block: wave
-// w reduces columns [w d/4, (w+1) d/4) on v_mfma_f32_32x32x16_f16 with ranks as rows (rows
-// 0 .. r-1 the q ranks against drop_q(x), r .. 2r-1 the v ranks against drop_v(x), the rest
-// zero) and tokens as columns (4 .. 31 zero); the waves' sums meet in `park` (kDownParkFloats of
-// LDS) and are added in wave order, then rounded to fp16 once. Every thread of the block must
-// call it (it holds barriers); x's rows must be visible to the whole block.
-template <int U = 4>
-__device__ __forceinline__ void lora_down_rows4(const DownRows& a, int64_t t0, float* park) {
+// The block's four wave sums (register j of lane l: rank row 8 (j / 4) + 4 (l / 32) + j % 4, token
+// column l % 32) added in wave order through `park` (T * 128 floats), rounded and stored.
+template <int T>
+__device__ __forceinline__ void down_rows_finish(const DownRows& a, int64_t t0, const f32x16& acc,
+                                                 float* park) {
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
+  if (col < T) {
+#pragma unroll
+    for (int j = 0; j < 16; ++j)
+      park[wave * T * 32 + col * 32 + 8 * (j >> 2) + 4 * h + (j & 3)] = acc[j];
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < T * 32; e += 256) {
+    const int tok = e >> 5, row = e & 31;
+    const float s = ((park[e] + park[T * 32 + e]) + park[2 * T * 32 + e]) + park[3 * T * 32 + e];
+    const int64_t tt = t0 + tok;
+    if (tt < a.n_tok && row < 2 * a.r) {
+      if (row < a.r)
+        a.mid_q[tt * a.r + row] = from_f32<f16>(s);
+      else
+        a.mid_v[tt * a.r + row - a.r] = from_f32<f16>(s);
+    }
+  }
+}
+
+// mid_q / mid_v of tokens t0 .. t0 + T - 1 (those below n_tok; T 4 to 32), by all four waves of
+// the block: wave w reduces columns [w d/4, (w+1) d/4) on v_mfma_f32_32x32x16_f16 with ranks as
+// rows (rows 0 .. r-1 the q ranks against drop_q(x), r .. 2r-1 the v ranks against drop_v(x), the
+// rest zero) and tokens as columns (T .. 31 zero); the waves' sums meet in `park` (T * 128 floats
+// of LDS) and are added in wave order, then rounded to fp16 once: a token's result does not depend
+// on T. Every thread of the block must call it (it holds barriers); x's rows must be visible to
+// the whole block.
+template <int U, int T>
+__device__ __forceinline__ void lora_down_rows(const DownRows& a, int64_t t0, float* park) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
   const bool is_q = col < a.r, is_v = col >= a.r && col < 2 * a.r;
   const f16* arow = is_q ? a.aq + static_cast<int64_t>(col) * a.d
                          : a.av + static_cast<int64_t>(is_v ? col - a.r : 0) * a.d;
   const int64_t t = t0 + col;
-  const bool live = col < kDownRows && t < a.n_tok;
+  const bool live = col < T && t < a.n_tok;
   const f16* xrow = a.x + (live ? t : 0) * a.sx;
   const bool drop = a.bits_q != nullptr;  // uniform
   const uint32_t* mq = drop ? a.bits_q + (live ? t : 0) * a.words : nullptr;
@@ -127,25 +168,97 @@ __device__ __forceinline__ void lora_down_rows4(const DownRows& a, int64_t t0, f
       }
     }
   }
-  // Register j of lane l: rank row 8 (j / 4) + 4 h + j % 4, token column l % 32.
-  if (col < kDownRows) {
+  down_rows_finish<T>(a, t0, acc, park);
+}
+
+// lora_down_rows with both operands through LDS: the same MFMA sequence on the same operands, so
+// the same bits. A fragment read straight from memory touches 32 rows x 32 bytes; here each wave
+// copies its quarter of the columns in tiles of 128 (32 rank rows of A and T token rows of x, whole
+// 256-byte rows per 16 lanes, chunk c of row r at c ^ swz(r)), all at once: one memory latency.
+// d a multiple of 512, at most 512 * kDownTiles; keep-bit rows 16-byte aligned.
+constexpr int kDownTiles = 3;  // 128-column tiles per wave
+constexpr int kDownTileA = 32 * 256;
+typedef __attribute__((address_space(3))) void* lds_void_ptr;
+
+__device__ __forceinline__ int down_swz(int r) { return ((r & 3) << 2) | ((r >> 2) & 3); }
+
+template <int T>
+constexpr int down_tiled_bytes() {
+  return 4 * kDownTiles * (kDownTileA + T * 256);
+}
+
+template <int T>
+__device__ __forceinline__ void lora_down_tiled(const DownRows& a, int64_t t0, char* smem) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) >> 6);
+  const int lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
+  const int nt = a.d / 512, per = a.d / 4, c_begin = wave * per;
+  char* at = smem + wave * kDownTiles * kDownTileA;
+  char* xt = smem + 4 * kDownTiles * kDownTileA + wave * kDownTiles * (T * 256);
+  for (int p = 0; p < nt; ++p) {
 #pragma unroll
-    for (int j = 0; j < 16; ++j)
-      park[wave * 128 + col * 32 + 8 * (j >> 2) + 4 * h + (j & 3)] = acc[j];
-  }
-  __syncthreads();
-  if (threadIdx.x < 128) {
-    const int tok = threadIdx.x >> 5, row = threadIdx.x & 31;
-    const float s = ((park[threadIdx.x] + park[128 + threadIdx.x]) + park[256 + threadIdx.x]) +
-                    park[384 + threadIdx.x];
-    const int64_t tt = t0 + tok;
-    if (tt < a.n_tok && row < 2 * a.r) {
-      if (row < a.r)
-        a.mid_q[tt * a.r + row] = from_f32<f16>(s);
-      else
-        a.mid_v[tt * a.r + row - a.r] = from_f32<f16>(s);
+    for (int i = 0; i < 8; ++i) {  // copy i: rows 4 i .. 4 i + 3
+      const int r = 4 * i + (lane >> 4);
+      const f16* row = r < a.r ? a.aq + static_cast<int64_t>(r) * a.d
+                               : a.av + static_cast<int64_t>(r < 2 * a.r ? r - a.r : 0) * a.d;
+      __builtin_amdgcn_global_load_lds(
+          row + c_begin + 128 * p + 8 * ((lane & 15) ^ down_swz(r)),
+          (lds_void_ptr)(at + p * kDownTileA + i * 1024), 16, 0, 0);
+    }
+#pragma unroll
+    for (int i = 0; i < T / 4; ++i) {
+      const int r = 4 * i + (lane >> 4);
+      const int64_t t = t0 + r < a.n_tok ? t0 + r : a.n_tok - 1;
+      __builtin_amdgcn_global_load_lds(
+          a.x + t * a.sx + c_begin + 128 * p + 8 * ((lane & 15) ^ down_swz(r)),
+          (lds_void_ptr)(xt + p * (T * 256) + i * 1024), 16, 0, 0);
     }
   }
+  const bool is_q = col < a.r, is_v = col >= a.r && col < 2 * a.r;
+  const int64_t t = t0 + col;
+  const bool live = col < T && t < a.n_tok;
+  const bool drop = a.bits_q != nullptr;               // uniform
+  const bool one_scale = a.scale_q == a.scale_v;       // uniform
+  const int xr = col < T ? col : 0;
+  const u32x4 none = {0, 0, 0, 0};
+  u32x4 wq[kDownTiles], wv[kDownTiles];  // a tile's 128 columns: 4 keep-bit words
+  if (drop) {
+    const int64_t o = (live ? t : 0) * a.words + c_begin / 32;
+#pragma unroll
+    for (int p = 0; p < kDownTiles; ++p) {
+      const int q = p < nt ? p : 0;
+      wq[p] = live ? *reinterpret_cast<const u32x4*>(a.bits_q + o + 4 * q) : none;
+      wv[p] = live ? *reinterpret_cast<const u32x4*>(a.bits_v + o + 4 * q) : none;
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0): this wave's tiles have landed
+  asm volatile("" ::: "memory");
+  f32x16 acc = f32x16{};
+#pragma unroll
+  for (int p = 0; p < kDownTiles; ++p) {
+    if (p >= nt) break;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const int c = 2 * s + h;
+      const f16x8 af =
+          *reinterpret_cast<const f16x8*>(at + p * kDownTileA + col * 256 + ((c ^ down_swz(col)) << 4));
+      const f16x8 xf =
+          *reinterpret_cast<const f16x8*>(xt + p * (T * 256) + xr * 256 + ((c ^ down_swz(xr)) << 4));
+      const f16x8 x = live ? xf : zero8();
+      if (drop) {
+        const int sh = 8 * (c & 3);
+        const f16x8 xq = scale8(x, a.scale_q);
+        const f16x8 xv = one_scale ? xq : scale8(x, a.scale_v);
+        acc = mfma(is_q ? af : zero8(), keep8(xq, wq[p][s >> 1], sh), acc);
+        acc = mfma(is_v ? af : zero8(), keep8(xv, wv[p][s >> 1], sh), acc);
+      } else {
+        acc = mfma(is_q || is_v ? af : zero8(), x, acc);
+      }
+    }
+  }
+  __syncthreads();  // every wave is done with its tiles: the sums take their place
+  float* park = reinterpret_cast<float*>(smem);
+  down_rows_finish<T>(a, t0, acc, park);
 }
 
 // LDS that lora_down_rows4_staged needs beside `park` (kDownParkFloats floats): the block's
@@ -183,7 +296,7 @@ __device__ __forceinline__ void stage_down_rows(const DownRows& a, int64_t t0, f
   __syncthreads();
 }
 
-// lora_down_rows4 with the block's x rows and keep bits already in LDS (stage_down_rows): the
+// lora_down_rows<., 4> with the block's x rows and keep bits already in LDS (stage_down_rows): the
 // same MFMA sequence on the same operands, so the same bits. Only the A fragments come from
 // global memory, U K steps of them issued together; x and the bits are read from LDS at each
 // step, so a batch holds 4 U registers per lane.
@@ -215,7 +328,7 @@ __device__ __forceinline__ void lora_down_rows4_staged(const DownRows& a, int64_
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = c_begin + min(s0 + 16 * u, per - 16) + 8 * h;
-      // Steps past the wave's range add zero products, as in lora_down_rows4.
+      // Steps past the wave's range add zero products, as in lora_down_rows.
       const f16x8 x = (live && s0 + 16 * u < per) ? ld8(xrow + c) : zero8();
       if (drop) {
         const uint32_t wq = live ? mq[c >> 5] : 0u, wv = live ? mv[c >> 5] : 0u;

@@ -414,3 +414,52 @@ def test_engine_lora_fp16_t_is_the_cast_launch_copy():
     again = eng.lora_views(torch.cat([x.reshape(-1) for x in lora16]))
     for a, b in zip(again, eng.lora_fp16_t(again)):
         assert torch.equal(b, a.t())
+
+
+@pytest.mark.parametrize("drop", [False, True])
+@pytest.mark.parametrize("n,d,dq_dim,dv_dim", [
+    (255, 1536, 1536, 256), (256, 1536, 1536, 256), (1100, 1536, 1536, 256),
+    (321, 200, 136, 72), (700, 64, 128, 8)])
+def test_lora_weight_gradients_of_long_batches(drop, n, d, dq_dim, dv_dim):
+    """The MFMA weight-gradient blocks (rank 16, from 256 tokens on: stages of 64 tokens, 64 or 128
+    columns per block, several token chunks) at partial stages, chunks and column blocks."""
+    r = 16
+    g, x, aq, av, bq, bv = _inputs(n, d, dq_dim, dv_dim, r, seed=5 + n + d)
+    dq, dv = torch.randn(n, dq_dim, generator=g).half(), torch.randn(n, dv_dim, generator=g).half()
+    mq, mv, dmq, dmv = ((torch.randn(n, r, generator=g) * 0.5).half() for _ in range(4))
+    args = (31, 2, 3, 0.05, 0.1) if drop else (None,)
+    _, _, xq, xv = ref.lora_down_fwd(x, aq, av, *args)
+    want = ref.lora_bwd_w(xq, xv, dq, dv, mq, mv, dmq, dmv)
+    bits = _bits(31, 2, n, d, 0.05, 0.1) if drop else (None, None)
+    outs = [torch.full(w.shape, 7.0, dtype=torch.float16, device=DEV) for w in want]
+    dev = [t.to(DEV) for t in (x, dq, dv, mq, mv, dmq, dmv)]
+    K.lora_bwd_w(*dev, *outs, *bits, 0.05, 0.1)
+    again = [torch.empty_like(o) for o in outs]
+    K.lora_bwd_w(*dev, *again, *bits, 0.05, 0.1)
+    torch.cuda.synchronize()
+    for got, w, (aa, bb) in zip(outs, want, ((dmq.t(), xq), (dq.t(), mq), (dmv.t(), xv), (dv.t(), mv))):
+        ok, err = _close(got, w, a=aa, b=bb)
+        assert ok, err
+    assert all(torch.equal(a, b) for a, b in zip(outs, again))
+
+
+@pytest.mark.parametrize("drop", [False, True])
+@pytest.mark.parametrize("n,d,r", [(1025, 512, 16), (1031, 1536, 8), (2051, 1536, 16), (2060, 1024, 4)])
+def test_lora_down_rows_of_long_batches_equals_short_ones(drop, n, d, r):
+    """A token's LoRA-down does not depend on how many tokens share its block: the batch at once
+    (8 or 16 tokens per block) and in pieces of at most 301 (4 per block) give the same bits."""
+    _, x, aq, av, _, _ = _inputs(n, d, 8, 8, r, seed=r + n + d)
+    bits = _bits(9, 2, n, d, 0.05, 0.1) if drop else (None, None)
+    xd, aqd, avd = x.to(DEV), aq.to(DEV), av.to(DEV)
+    whole = K.lora_down_rows(xd, aqd, avd, *bits, 0.05, 0.1)
+    for t0 in range(0, n, 301):
+        cut = slice(t0, min(t0 + 301, n))
+        sub = [None if b is None else b[cut].contiguous() for b in bits]
+        piece = K.lora_down_rows(xd[cut], aqd, avd, *sub, 0.05, 0.1)
+        for a, b in zip(whole, piece):
+            assert torch.equal(a[cut], b)
+    args = (9, 2, 3, 0.05, 0.1) if drop else (None,)
+    mq, mv, xq, xv = ref.lora_down_fwd(x, aq, av, *args)
+    for got, want, xx, aa in zip(whole, (mq, mv), (xq, xv), (aq, av)):
+        ok, err = _close(got, want, a=xx, b=aa.t())
+        assert ok, err
