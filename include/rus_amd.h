@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define RUS_ABI_VERSION 17
+#define RUS_ABI_VERSION 18
 
 #define RUS_DTYPE_F16 0
 #define RUS_DTYPE_F32 1
@@ -631,6 +631,36 @@ int rus_lmhead_ce_grad_hidden_scaled(const void* probs, int64_t ld_p, const void
                                      int64_t ld_wt, int64_t n_tok, int64_t d, int64_t n_vocab,
                                      float* parts, int32_t n_split, int32_t accumulate,
                                      const float* alpha, void* stream);
+
+/*
+ * rus_lmhead_ce_fwd that also stores the chunk's probabilities P[t][v - vocab_start] =
+ * fp16(2^(z log2 e - K)) (columns up to round_up(n_vocab, 64), zeros past n_vocab), K a
+ * reference per token and 128 vocabulary rows: ref[t] (log2 units, as rus_lmhead_ce_probs_rescale
+ * left it; NULL for the first chunk) unless the largest logit there lies more than 15 above it, else
+ * a reference of its own, written like the others to half_ref[2 * (r / 256) + (r / 128) % 2][t]
+ * (row stride part_stride). chunk_max[t] (0 before the call) receives the chunk's maximum as
+ * ordered bits. Replaces: as rus_lmhead_ce_fwd_keep, with the exponentials of the gradient pass.
+ */
+int rus_lmhead_ce_fwd_probs(const void* hidden, const void* weight, const int64_t* labels,
+                            int64_t n_tok, int64_t d, int64_t ld_h, int64_t ld_w, int64_t n_vocab,
+                            int64_t vocab_start, float* part_m, float* part_s, float* part_w,
+                            int32_t* part_idx, int64_t part_base, int64_t part_stride,
+                            float* target, void* probs, int64_t ld_p, const float* ref,
+                            float* half_ref, uint32_t* chunk_max, void* stream);
+
+/*
+ * Between rus_lmhead_ce_fwd_probs and rus_lmhead_ce_grad_hidden_scaled of one chunk: brings a
+ * token's P to one reference where its half tiles took different ones, and steps the token's state
+ * (all n_tok floats; ref_in / run_in NULL for the first chunk, else the outputs of the chunk before,
+ * in buffers of their own): run_out = this chunk's reference, alpha = 2^(run_in - run_out) (0 at
+ * first), ref_out = the reference for the next chunk, m_run = run_out in natural log (for
+ * rus_lmhead_ce_dh_finish). Replaces: as rus_lmhead_ce_chunk_scale.
+ */
+int rus_lmhead_ce_probs_rescale(void* probs, int64_t ld_p, int64_t n_tok, int64_t n_vocab,
+                                const float* half_ref, int64_t half_stride,
+                                const uint32_t* chunk_max, const float* ref_in,
+                                const float* run_in, float* ref_out, float* run_out, float* alpha,
+                                float* m_run, void* stream);
 
 /*
  * One vocabulary chunk of the single-pass head, between its statistics GEMM (which kept the

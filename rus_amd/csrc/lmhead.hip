@@ -109,16 +109,50 @@ struct StatsParams {
   int64_t part_stride;  // entries per partial row (>= n_tok)
   int part_base;        // partial row of A's first 256-row tile
   int vocab_start;      // global vocabulary index of A's row 0
-  f16* z;               // KEEP: the fp16 logits [n_tok][ld_z], columns up to kpad (0 past M)
+  f16* z;               // kLogits / kProbs: [n_tok][ld_z], columns up to kpad (0 past M)
   int64_t ld_z;
   int kpad;
+  // kProbs: P = 2^(z log2 e - K), with a reference K per token and 128 vocabulary rows
+  const float* ref;     // [n_tok] reference from the chunks before (nullptr: the first chunk)
+  float* half_ref;      // [2 * parts of the chunk][part_stride]: the K each half tile used
+  uint32_t* chunk_max;  // [n_tok] ordered bits of the chunk's maximum (0 before the launch)
 };
+
+// What the statistics kernel leaves besides its partials. kProbs exists for the single pass: with
+// kLogits a kernel between the two GEMMs of a chunk read and rewrote all its logits (43 us per
+// [2048, 32768] chunk, memory-bound, 9 us at 100 tokens); probabilities written once need a launch
+// that only looks at the references (5 us). 2048 tokens x 151936: 2571 -> 2372 us, 345: 770 -> 725.
+enum StatsOut { kNone = 0, kLogits = 1, kProbs = 2 };
+
+// A token's reference stays the one it came with unless a half tile's largest logit lies more than
+// kRefWindow (log2 units) above it; P is at most 2^15 in fp16. A half tile past the window (every
+// one of the first chunk) takes its own, a multiple of kRefStep not above its maximum, so that the
+// half tiles of a token mostly agree (P < 2^kRefStep) and none needs rescaling. Either way the
+// largest P is at least 2^-1/2: fp16 resolves every probability as well as it would against the
+// maximum (dH against float64 at 707 tokens: 1.29e-6 relative either way). The offset is free: it only
+// moves where P's roundings fall (with 0 one gradient of the 28-layer comparison with the oracle,
+// within 1% of it by a hair, lands at 1.003%).
+constexpr float kRefWindow = 15.0f, kRefStep = 8.0f, kRefOffset = 0.5f;
+
+__device__ __forceinline__ float own_ref(float y) {
+  return kRefStep * floorf(y / kRefStep) + kRefOffset;
+}
+
+// fp32 -> uint32 in the same order (NaN aside); 0 is below every value.
+__device__ __forceinline__ uint32_t ordered_bits(float x) {
+  const uint32_t u = __builtin_bit_cast(uint32_t, x);
+  return u ^ ((u >> 31) ? 0xffffffffu : 0x80000000u);
+}
+__device__ __forceinline__ float from_ordered(uint32_t u) {
+  return __builtin_bit_cast(float, u ^ ((u >> 31) ? 0x80000000u : 0xffffffffu));
+}
 
 // The statistics epilogue of a block's 256 (vocab) x 256 (token) tile of logits, on NW waves in
 // the mainloop's layout (4: 128 x 128 each, 8: 128 x 64): per token, the maximum, the sums of e^{z-m}
 // and e^{z-m} z, the first argmax and the target logit over the tile's vocab rows (the two 128-row
-// halves merged through the LDS); with KEEP the fp16 logits are stored first.
-template <int NW, bool KEEP>
+// halves merged through the LDS); kLogits stores the fp16 logits first, kProbs P once the sums are
+// formed from the same exponentials.
+template <int NW, int OUT>
 __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, const Tile& tl,
                                                const StatsParams& p,
                                                f32x16 (&acc)[kMT][16 / NW]) {
@@ -136,7 +170,7 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) acc[mt][nt][r] = round16(acc[mt][nt][r]);
-  if constexpr (KEEP)
+  if constexpr (OUT == kLogits)
     store_tile_tv<NW>(smem, g, tl, p.z, p.ld_z, p.kpad,
                       [&](int mt, int nt, int r, int) { return acc[mt][nt][r]; });
   // Accumulator row of (mt, r) for this lane: mt*32 + 8*(r/4) + 4*h + r%4 (local to vrow0).
@@ -185,8 +219,17 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
       idx = i2;
     }
     float s = 0.0f, w = 0.0f;
-    if (m > -INFINITY) {
-      const float mb = m * kLog2e;
+    float mb = m * kLog2e;  // the exponentials' reference (log2 units)
+    float ref = mb;
+    if constexpr (OUT == kProbs) {
+      const float given = p.ref && tok < g.N ? p.ref[tok] : -INFINITY;
+      ref = mb > given + kRefWindow ? own_ref(mb) : given;
+      if (!(m > -INFINITY)) ref = given > -INFINITY ? given : 0.0f;  // no finite logit here
+      if (h == 0 && tok < g.N)
+        p.half_ref[static_cast<int64_t>(2 * (tl.m0 / kBM) + wm) * p.part_stride + tok] = ref;
+    }
+    if (OUT == kProbs || m > -INFINITY) {
+      mb = ref;
       if (full) {
 #pragma unroll
         for (int mt = 0; mt < kMT; ++mt)
@@ -196,6 +239,7 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
             const float e = exp2_fast(__builtin_fmaf(z, kLog2e, -mb));
             s += e;
             w = __builtin_fmaf(e, z, w);
+            if constexpr (OUT == kProbs) acc[mt][nt][r] = e;
           }
       } else {
 #pragma unroll
@@ -208,12 +252,22 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
               const float e = exp2_fast(__builtin_fmaf(z, kLog2e, -mb));
               s += e;
               w = __builtin_fmaf(e, z, w);
+              if constexpr (OUT == kProbs) acc[mt][nt][r] = e;
             }
           }
       }
     }
     s += __shfl_xor(s, 32, kWave);
     w += __shfl_xor(w, 32, kWave);
+    if constexpr (OUT == kProbs) {
+      // The partial's sums are relative to its maximum. Far below the reference (2^-100 of the
+      // token's total at most) the exponentials may be all zero: any bounded sum will do.
+      const float up = ref - m * kLog2e;
+      const float f = exp2_fast(up);
+      s = up > 100.0f ? 1.0f : s * f;
+      w = up > 100.0f ? m : w * f;
+      if (!(m > -INFINITY)) s = w = 0.0f;
+    }
     rm[nt] = m;
     rs[nt] = s;
     rw[nt] = w;
@@ -222,8 +276,12 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
     if (lab_adj + 4 * h >= 0 && ((lab_adj + 4 * h) >> 2 & 1) == h) p.target[tok] = tgt;
   }
 
+  if constexpr (OUT == kProbs)
+    store_tile_tv<NW>(smem, g, tl, p.z, p.ld_z, p.kpad,
+                      [&](int mt, int nt, int r, int) { return acc[mt][nt][r]; });
+
   // Merge the two vocab halves (wm = 0, 1) of the block through LDS; wm = 0 writes the partial.
-  if constexpr (KEEP) __syncthreads();  // the logits' staging reads of the LDS are done
+  if constexpr (OUT != kNone) __syncthreads();  // the stored tile's staging reads of the LDS are done
   float* xm = reinterpret_cast<float*>(smem);  // [token column of the tile] x (m, s, w, idx)
   if (wm == 1 && h == 0) {
 #pragma unroll
@@ -260,12 +318,13 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
         p.part_s[o2] = s;
         p.part_w[o2] = w;
         p.part_idx[o2] = idx + p.vocab_start;
+        if constexpr (OUT == kProbs) atomicMax(p.chunk_max + tok, ordered_bits(m));
       }
     }
   }
 }
 
-template <bool KEEP>
+template <int OUT>
 __global__ __launch_bounds__(kThreads8) __attribute__((amdgpu_waves_per_eu(2, 2))) void
 lmhead_stats_kernel(GemmArgs g, StatsParams p) {
   __shared__ __attribute__((aligned(16))) char smem[kSmemBytes];
@@ -273,7 +332,7 @@ lmhead_stats_kernel(GemmArgs g, StatsParams p) {
   if (!tile_of(g, tl)) return;
   f32x16 acc[kMT][2];
   mainloop(g, tl, smem, acc);
-  stats_epilogue<8, KEEP>(smem, g, tl, p, acc);
+  stats_epilogue<8, OUT>(smem, g, tl, p, acc);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -488,6 +547,47 @@ __global__ __launch_bounds__(kZgThreads) void lmhead_chunk_scale_kernel(
   }
 }
 
+// The same between the statistics kernel that stored P (kProbs) and the hidden-gradient GEMM: the
+// token's reference for the chunk is the one it came with, or, past the window, the largest its half
+// tiles took; half tiles with another are brought to it (by a power of two, exact but for values
+// below fp16's range). Block = (token, kZgCols columns); without a half tile past the window nothing
+// is read. Block (token, 0) writes the token's next state: run (the reference of the accumulated
+// partials), alpha = 2^(run before - run), the reference of the next chunk, and run in natural log.
+__global__ __launch_bounds__(kZgThreads) void lmhead_probs_rescale_kernel(
+    f16* zg, int64_t ld, int n_vocab, int kpad, const float* __restrict__ half_ref,
+    int64_t half_stride, const uint32_t* __restrict__ chunk_max, const float* __restrict__ ref_in,
+    const float* __restrict__ run_in, float* __restrict__ ref_out, float* __restrict__ run_out,
+    float* __restrict__ alpha, float* __restrict__ m_run) {
+  const int tok = blockIdx.x;
+  const uint32_t mo = chunk_max[tok];
+  const float m = mo ? from_ordered(mo) : -INFINITY, y = m * kLog2e;  // 0: no finite logit
+  const float given = ref_in ? ref_in[tok] : -INFINITY;
+  const bool past = y > given + kRefWindow;
+  float run = past ? own_ref(y) : given;
+  if (!(run > -INFINITY)) run = 0.0f;
+  if (blockIdx.y == 0 && threadIdx.x == 0) {
+    run_out[tok] = run;
+    ref_out[tok] = y > -INFINITY ? fmaxf(run, own_ref(y)) : run;
+    alpha[tok] = run_in ? exp2_fast(run_in[tok] - run) : 0.0f;
+    m_run[tok] = run * 0.6931471805599453f;
+  }
+  if (!past) return;
+  f16* row = zg + static_cast<int64_t>(tok) * ld;
+  const int c0 = blockIdx.y * kZgCols + threadIdx.x * 8;
+#pragma unroll
+  for (int u = 0; u < kZgUnroll; ++u) {
+    const int c = c0 + u * kZgThreads * 8;
+    if (c >= n_vocab) continue;
+    const float k = half_ref[static_cast<int64_t>(c >> 7) * half_stride + tok];
+    if (k == run) continue;
+    const float f = exp2_fast(fminf(k - run, 0.0f));  // k <= run but where P is all zero
+    f16x8 v = *reinterpret_cast<const f16x8*>(row + c);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = from_f32<f16>(static_cast<float>(v[e]) * f);
+    *reinterpret_cast<f16x8*>(row + c) = v;
+  }
+}
+
 // dH (times 2^16 / denom, times scale) from the online accumulation:
 //   out[t][c] = (sum_s parts[s][t][c] * e^{M[t] - lse[t]} - W[y_t][c]) * 2^16 / denom * scale
 // for labelled tokens (y_t != -100; the W row term only when y_t indexes the vocabulary), 0 for
@@ -670,12 +770,13 @@ __global__ __launch_bounds__(kRowThreads) void lmhead_rows_kernel(
 }
 
 // ---------------------------------------------------------------------------------------------
-// Combine partial statistics: one lane per token, 16 waves per 64 tokens, each wave merging a
-// contiguous range of partials eight loads at a time, then wave 0 merging the 16 results in
-// wave order (deterministic; ties keep the smallest vocabulary index).
+// Combine partial statistics: 16 tokens per block, 64 threads per token, each merging a contiguous
+// range of partials eight loads at a time; then 8 threads per token merge 8 of those results each in
+// order, and one the last 8 (deterministic; ties keep the smallest vocabulary index). With 64 tokens
+// per block (one lane each, 16 waves) a batch of 345 tokens had six blocks, 16 us of load latency.
 // ---------------------------------------------------------------------------------------------
 
-constexpr int kCombWaves = 16, kCombDepth = 8;
+constexpr int kCombTok = 16, kCombSub = 64, kCombDepth = 8;
 
 struct Stat {
   float m, s, w;
@@ -697,18 +798,17 @@ __device__ __forceinline__ void merge_stat(Stat& a, float m, float s, float w, i
   }
 }
 
-__global__ __launch_bounds__(kCombWaves * 64) void lmhead_combine_kernel(
+__global__ __launch_bounds__(kCombTok * kCombSub) void lmhead_combine_kernel(
     const float* __restrict__ pm, const float* __restrict__ ps, const float* __restrict__ pw,
     const int32_t* __restrict__ pi, int n_parts, int64_t stride, const float* __restrict__ target,
     const int64_t* __restrict__ labels, int n_tok, float* __restrict__ lse,
     float* __restrict__ nll, float* __restrict__ ent, int64_t* __restrict__ amax) {
-  __shared__ float sm[kCombWaves][64], ss[kCombWaves][64], sw[kCombWaves][64];
-  __shared__ int si[kCombWaves][64];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int tok = blockIdx.x * 64 + lane;
+  __shared__ Stat part[kCombSub][kCombTok + 1];
+  const int col = threadIdx.x % kCombTok, sub = threadIdx.x / kCombTok;
+  const int tok = blockIdx.x * kCombTok + col;
   Stat st{-INFINITY, 0.0f, 0.0f, 0x7fffffff};
-  const int per = (n_parts + kCombWaves - 1) / kCombWaves;
-  const int q0 = wave * per, q1 = min(q0 + per, n_parts);
+  const int per = (n_parts + kCombSub - 1) / kCombSub;
+  const int q0 = sub * per, q1 = min(q0 + per, n_parts);
   if (tok < n_tok) {
     for (int q = q0; q < q1; q += kCombDepth) {
       float m[kCombDepth], s[kCombDepth], w[kCombDepth];
@@ -726,15 +826,21 @@ __global__ __launch_bounds__(kCombWaves * 64) void lmhead_combine_kernel(
         if (q + j < q1) merge_stat(st, m[j], s[j], w[j], ix[j]);
     }
   }
-  sm[wave][lane] = st.m;
-  ss[wave][lane] = st.s;
-  sw[wave][lane] = st.w;
-  si[wave][lane] = st.i;
+  part[sub][col] = st;
   __syncthreads();
-  if (wave != 0 || tok >= n_tok) return;
-  Stat t{-INFINITY, 0.0f, 0.0f, 0x7fffffff};
-  for (int k = 0; k < kCombWaves; ++k)
-    merge_stat(t, sm[k][lane], ss[k][lane], sw[k][lane], si[k][lane]);
+  for (int width = kCombSub / 8; width >= 1; width /= 8) {  // 64 -> 8 -> 1
+    Stat t{-INFINITY, 0.0f, 0.0f, 0x7fffffff};
+    if (sub < width)
+      for (int k = 0; k < 8; ++k) {
+        const Stat a = part[8 * sub + k][col];
+        merge_stat(t, a.m, a.s, a.w, a.i);
+      }
+    __syncthreads();
+    if (sub < width) part[sub][col] = t;
+    __syncthreads();
+  }
+  if (sub != 0 || tok >= n_tok) return;
+  const Stat t = part[0][col];
   const float L = t.m + logf(t.s);
   lse[tok] = L;
   ent[tok] = L - t.w / t.s;
@@ -805,7 +911,9 @@ static int lmhead_fwd(const char* fn, const void* hidden, const void* weight,
                       const int64_t* labels, int64_t n_tok, int64_t d, int64_t ld_h, int64_t ld_w,
                       int64_t n_vocab, int64_t vocab_start, float* part_m, float* part_s,
                       float* part_w, int32_t* part_idx, int64_t part_base, int64_t part_stride,
-                      float* target, void* logits, int64_t ld_z, void* stream) {
+                      float* target, void* logits, int64_t ld_z, void* stream,
+                      bool probs = false, const float* ref = nullptr, float* half_ref = nullptr,
+                      uint32_t* chunk_max = nullptr) {
   if (n_tok < 0 || n_tok >= (1 << 30) || n_vocab < 0 || n_vocab >= (1 << 30) || d <= 0 ||
       d % kBK || vocab_start < 0 || vocab_start + n_vocab >= (int64_t(1) << 31))
     return fail(RUS_ERR_INVALID,
@@ -839,12 +947,15 @@ static int lmhead_fwd(const char* fn, const void* hidden, const void* weight,
   StatsParams p{labels,      part_m,      part_s, part_w,  part_idx,
                 target,      part_stride, static_cast<int>(part_base),
                 static_cast<int>(vocab_start), static_cast<f16*>(logits), ld_z,
-                static_cast<int>((n_vocab + kBK - 1) / kBK * kBK)};
-  if (logits)
-    hipLaunchKernelGGL(lmhead_stats_kernel<true>, dim3(launch_grid(g)), dim3(kThreads8), 0,
+                static_cast<int>((n_vocab + kBK - 1) / kBK * kBK), ref, half_ref, chunk_max};
+  if (probs)
+    hipLaunchKernelGGL(lmhead_stats_kernel<kProbs>, dim3(launch_grid(g)), dim3(kThreads8), 0,
+                       static_cast<hipStream_t>(stream), g, p);
+  else if (logits)
+    hipLaunchKernelGGL(lmhead_stats_kernel<kLogits>, dim3(launch_grid(g)), dim3(kThreads8), 0,
                        static_cast<hipStream_t>(stream), g, p);
   else
-    hipLaunchKernelGGL(lmhead_stats_kernel<false>, dim3(launch_grid(g)), dim3(kThreads8), 0,
+    hipLaunchKernelGGL(lmhead_stats_kernel<kNone>, dim3(launch_grid(g)), dim3(kThreads8), 0,
                        static_cast<hipStream_t>(stream), g, p);
   return check_launch(fn);
 }
@@ -872,6 +983,23 @@ extern "C" int rus_lmhead_ce_fwd_keep(const void* hidden, const void* weight,
   return lmhead_fwd(fn, hidden, weight, labels, n_tok, d, ld_h, ld_w, n_vocab, vocab_start,
                     part_m, part_s, part_w, part_idx, part_base, part_stride, target, logits,
                     ld_z, stream);
+}
+
+extern "C" int rus_lmhead_ce_fwd_probs(const void* hidden, const void* weight,
+                                       const int64_t* labels, int64_t n_tok, int64_t d,
+                                       int64_t ld_h, int64_t ld_w, int64_t n_vocab,
+                                       int64_t vocab_start, float* part_m, float* part_s,
+                                       float* part_w, int32_t* part_idx, int64_t part_base,
+                                       int64_t part_stride, float* target, void* probs,
+                                       int64_t ld_p, const float* ref, float* half_ref,
+                                       uint32_t* chunk_max, void* stream) {
+  const char* fn = "rus_lmhead_ce_fwd_probs";
+  if (n_tok > 0 && n_vocab > 0 && (!probs || !half_ref || !chunk_max || !aligned(half_ref, 4) ||
+                                   !aligned(chunk_max, 4)))
+    return fail(RUS_ERR_INVALID, "%s: null or misaligned buffer", fn);
+  return lmhead_fwd(fn, hidden, weight, labels, n_tok, d, ld_h, ld_w, n_vocab, vocab_start,
+                    part_m, part_s, part_w, part_idx, part_base, part_stride, target, probs,
+                    ld_p, stream, true, ref, half_ref, chunk_max);
 }
 
 extern "C" int rus_lmhead_ce_grad_from_logits(void* logits_grad, int64_t ld_g,
@@ -913,8 +1041,8 @@ extern "C" int rus_lmhead_ce_combine(const float* part_m, const float* part_s, c
   if (!part_m || !part_s || !part_w || !part_idx || !target || !labels || !lse || !nll ||
       !entropy || !argmax)
     return fail(RUS_ERR_INVALID, "%s: null pointer argument", fn);
-  const dim3 grid(static_cast<unsigned>((n_tok + 63) / 64));
-  hipLaunchKernelGGL(lmhead_combine_kernel, grid, dim3(kCombWaves * 64), 0,
+  const dim3 grid(static_cast<unsigned>((n_tok + kCombTok - 1) / kCombTok));
+  hipLaunchKernelGGL(lmhead_combine_kernel, grid, dim3(kCombTok * kCombSub), 0,
                      static_cast<hipStream_t>(stream), part_m, part_s, part_w, part_idx,
                      static_cast<int>(n_parts), part_stride, target, labels,
                      static_cast<int>(n_tok), lse, nll, entropy, argmax);
@@ -1097,6 +1225,34 @@ extern "C" int rus_lmhead_ce_chunk_scale(void* logits, int64_t ld_z, int64_t n_t
                      static_cast<f16*>(logits), ld_z, static_cast<int>(n_vocab),
                      static_cast<int>(kpad), part_m, part_stride, static_cast<int>(part_base),
                      n_parts, m_run, alpha, first ? 1 : 0);
+  return check_launch(fn);
+}
+
+extern "C" int rus_lmhead_ce_probs_rescale(void* probs, int64_t ld_p, int64_t n_tok,
+                                           int64_t n_vocab, const float* half_ref,
+                                           int64_t half_stride, const uint32_t* chunk_max,
+                                           const float* ref_in, const float* run_in,
+                                           float* ref_out, float* run_out, float* alpha,
+                                           float* m_run, void* stream) {
+  const char* fn = "rus_lmhead_ce_probs_rescale";
+  if (n_tok < 0 || n_tok >= (1 << 30) || n_vocab < 0 || n_vocab >= (1 << 30) ||
+      half_stride < n_tok)
+    return fail(RUS_ERR_INVALID, "%s: bad sizes", fn);
+  if (n_tok == 0 || n_vocab == 0) return RUS_OK;
+  const int64_t kpad = (n_vocab + kBK - 1) / kBK * kBK;
+  if (ld_p < kpad) return fail(RUS_ERR_INVALID, "%s: ld_p must be >= %lld", fn, (long long)kpad);
+  if (int e = check_operand(fn, probs, ld_p, "probs")) return e;
+  if (!half_ref || !chunk_max || !ref_out || !run_out || !alpha || !m_run ||
+      (ref_in == nullptr) != (run_in == nullptr) || ref_in == ref_out || run_in == run_out)
+    return fail(RUS_ERR_INVALID, "%s: null pointer, or a state updated in place", fn);
+  const int64_t col_blocks = (kpad + kZgCols - 1) / kZgCols;
+  if (col_blocks > 65535) return fail(RUS_ERR_INVALID, "%s: n_vocab too large", fn);
+  hipLaunchKernelGGL(lmhead_probs_rescale_kernel,
+                     dim3(static_cast<unsigned>(n_tok), static_cast<unsigned>(col_blocks)),
+                     dim3(kZgThreads), 0, static_cast<hipStream_t>(stream),
+                     static_cast<f16*>(probs), ld_p, static_cast<int>(n_vocab),
+                     static_cast<int>(kpad), half_ref, half_stride, chunk_max, ref_in, run_in,
+                     ref_out, run_out, alpha, m_run);
   return check_launch(fn);
 }
 

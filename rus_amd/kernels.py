@@ -1457,11 +1457,13 @@ def _lm_operand(fn: str, t: torch.Tensor, d: int, name: str) -> torch.Tensor:
 
 def lm_head_ce_fwd_chunk(hidden: torch.Tensor, weight_rows: torch.Tensor, labels: torch.Tensor,
                          vocab_start: int, parts: LMHeadPartials, target: torch.Tensor,
-                         logits_out: torch.Tensor | None = None) -> None:
+                         logits_out: torch.Tensor | None = None, probs=None) -> None:
     """Forward partial statistics of vocabulary rows [vocab_start, vocab_start + len(weight_rows))
     (replaces one iteration of the reference's forward chunk loop, ops.py:217-251). With
     ``logits_out`` ([n_tok, >= round_up(n, 64)] fp16) the rounded logits are kept there too, for
-    ``lm_head_ce_grad_from_logits``."""
+    ``lm_head_ce_grad_from_logits``. ``probs`` (out like logits_out, reference [n_tok] or None,
+    half-tile references [>= 2 parts, n_tok], zeroed maxima [n_tok]) stores the chunk's
+    probabilities relative to per-token references instead (``LMHeadPass``)."""
     fn = "lm_head_ce_fwd_chunk"
     _require_device(fn, hidden, weight_rows, labels, target, logits_out)
     if vocab_start % LM_TILE:
@@ -1481,19 +1483,28 @@ def lm_head_ce_fwd_chunk(hidden: torch.Tensor, weight_rows: torch.Tensor, labels
     args = (h.data_ptr(), w.data_ptr(), lab.data_ptr(), n_tok, d, h.stride(0), w.stride(0),
             n_vocab, vocab_start, parts.m.data_ptr(), parts.s.data_ptr(), parts.w.data_ptr(),
             parts.idx.data_ptr(), part_base, n_tok, target.data_ptr())
-    if logits_out is None:
+    if logits_out is None and probs is None:
         _launch("lmhead_ce_fwd", nbytes, 2.0 * n_tok * d * n_vocab, "rus_lmhead_ce_fwd", *args,
                 _stream(h))
         return
     kp = _round_up(n_vocab, LM_K)
-    z = logits_out
+    z = logits_out if probs is None else probs[0]
     if z.dtype != torch.float16 or z.dim() != 2 or z.shape[0] != n_tok or z.shape[1] < kp \
             or z.stride(1) != 1:
         raise ValueError(f"{fn}: logits_out must be fp16 [{n_tok}, >= {kp}] with contiguous rows")
     if z.shape[0] * z.stride(0) * 2 >= 1 << 32:
         raise ValueError(f"{fn}: logits_out exceeds the 4 GiB operand limit of the MFMA kernels")
-    _launch("lmhead_ce_fwd_keep", nbytes + n_tok * kp * 2, 2.0 * n_tok * d * n_vocab,
-            "rus_lmhead_ce_fwd_keep", *args, z.data_ptr(), z.stride(0), _stream(h))
+    if probs is None:
+        _launch("lmhead_ce_fwd_keep", nbytes + n_tok * kp * 2, 2.0 * n_tok * d * n_vocab,
+                "rus_lmhead_ce_fwd_keep", *args, z.data_ptr(), z.stride(0), _stream(h))
+        return
+    _, ref, half_ref, chunk_max = probs
+    if half_ref.dtype != torch.float32 or not half_ref.is_contiguous() or half_ref.shape[1] != n_tok \
+            or half_ref.shape[0] < 2 * lm_head_num_parts(n_vocab) or chunk_max.numel() != n_tok:
+        raise ValueError(f"{fn}: half-tile references or maxima too small for this chunk")
+    _launch("lmhead_ce_fwd_probs", nbytes + n_tok * kp * 2, 2.0 * n_tok * d * n_vocab,
+            "rus_lmhead_ce_fwd_probs", *args, z.data_ptr(), z.stride(0), _ptr(ref),
+            half_ref.data_ptr(), chunk_max.data_ptr(), _stream(h))
 
 
 def lm_head_ce_combine(parts: LMHeadPartials, target: torch.Tensor, labels: torch.Tensor):
@@ -1875,9 +1886,9 @@ class LMHeadPass:
     """One single pass of the lm_head cross-entropy over vocabulary chunks (in order).
 
     Per chunk: the statistics GEMM (partial m, s, w, argmax and the target logit per 256 rows)
-    and, when the hidden gradient is wanted, its fp16 logits kept in a [n_tok, chunk] buffer,
-    turned in place into P = e^{z - M} (M the running maximum) and accumulated as P . W_chunk into
-    fp32 split-K partials rescaled whenever M grows. ``finish`` combines the statistics (lse,
+    and, when the hidden gradient is wanted, P = fp16(2^(z log2 e - K)) in a [n_tok, chunk] buffer
+    (K a reference per token, from the chunks before), accumulated as P . W_chunk into
+    fp32 split-K partials rescaled whenever K grows. ``finish`` combines the statistics (lse,
     nll, entropy, argmax, loss) and forms dH = sum_v (softmax - onehot) W_v x 2^16 / denom. W is
     read once, and no [n_tok, V] array exists (the reference reads W twice and recomputes the
     logits, solution/ops.py:217-322)."""
@@ -1886,13 +1897,21 @@ class LMHeadPass:
         self.n_tok, self.d, self.n_vocab, self.chunk = n_tok, d, n_vocab, int(chunk)
         self.need_grad = need_grad
         self.parts = LMHeadPartials(lm_head_num_parts(n_vocab), n_tok, device)
-        self.target = torch.zeros(n_tok, dtype=torch.float32, device=device)
-        self.first = True
+        self.done = 0  # chunks added
+        n_chunks = -(-n_vocab // self.chunk) if need_grad else 0
+        # the label logits and every chunk's maxima start at zero: one fill
+        zeros = torch.zeros((1 + n_chunks, n_tok), dtype=torch.float32, device=device)
+        self.target, *self.chunk_max = zeros.unbind(0)
         if need_grad:
-            self.z = torch.empty((n_tok, _round_up(min(self.chunk, n_vocab), LM_K)),
-                                 dtype=torch.float16, device=device)
-            self.m_run = torch.empty(n_tok, dtype=torch.float32, device=device)
-            self.alpha = torch.empty(n_tok, dtype=torch.float32, device=device)
+            cols = min(self.chunk, n_vocab)
+            self.z = torch.empty((n_tok, _round_up(cols, LM_K)), dtype=torch.float16,
+                                 device=device)
+            self.half_ref = torch.empty((2 * lm_head_num_parts(cols), n_tok),
+                                        dtype=torch.float32, device=device)
+            # per token: the next chunk's reference and the partials' reference of each chunk
+            # parity, the running maximum, and the partials' factor
+            rows = torch.empty((6, n_tok), dtype=torch.float32, device=device).unbind(0)
+            self.state, self.m_run, self.alpha = (rows[0:2], rows[2:4]), rows[4], rows[5]
             # every chunk's GEMM reads and rewrites all the fp32 partials (the rescaled
             # accumulation), so splits beyond one round of CUs cost a partial pass per chunk for
             # a few percent of mainloop: at most one round
@@ -1910,12 +1929,18 @@ class LMHeadPass:
         if not self.need_grad:
             lm_head_ce_fwd_chunk(hidden, w_rows, labels, start, self.parts, self.target)
             return
+        c = self.done
+        before = self.state[(c + 1) % 2] if c else (None, None)
+        after = self.state[c % 2]
         lm_head_ce_fwd_chunk(hidden, w_rows, labels, start, self.parts, self.target,
-                             logits_out=self.z)
-        lm_head_ce_chunk_scale(self.z, n, self.parts, start // LM_TILE, self.m_run, self.alpha,
-                               self.first)
-        lm_head_ce_grad_hidden_scaled(self.z, w_t, n, self.dparts, not self.first, self.alpha)
-        self.first = False
+                             probs=(self.z, before[0], self.half_ref, self.chunk_max[c]))
+        _launch("lmhead_ce_probs_rescale", 20 * self.n_tok, 0, "rus_lmhead_ce_probs_rescale",
+                self.z.data_ptr(), self.z.stride(0), self.n_tok, n, self.half_ref.data_ptr(),
+                self.n_tok, self.chunk_max[c].data_ptr(), _ptr(before[0]), _ptr(before[1]),
+                after[0].data_ptr(), after[1].data_ptr(), self.alpha.data_ptr(),
+                self.m_run.data_ptr(), _stream(self.z))
+        lm_head_ce_grad_hidden_scaled(self.z, w_t, n, self.dparts, c > 0, self.alpha)
+        self.done = c + 1
 
     def finish(self, labels: torch.Tensor, num_items_in_batch, w_rows_all: torch.Tensor,
                dh_scale: float = 1.0, dh_dtype=torch.float32, scale_dev=None):
@@ -2100,6 +2125,8 @@ def lm_head_ce(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor,
         chunk = int(v_chunk)
         if chunk <= 0 or (chunk < V and chunk % LM_TILE):
             raise ValueError(f"{fn}: v_chunk must be a positive multiple of {LM_TILE}")
+        if not need_grad:  # no logits are kept: one launch over the whole vocabulary, whose tiles
+            chunk = V      # fill 5 rounds of the CUs at 345 tokens where two chunks take 3 + 3
         wt = None
         if need_grad:
             wt = weight_t if weight_t is not None else lm_head_weight_t(weight)

@@ -316,3 +316,42 @@ def test_row_kernel_statistics_and_gradient(n, d, v):
     top2 = zo.topk(2, dim=-1).values
     near_tie = (top2[:, 0] - top2[:, 1]) <= ref.fp16_ulp(top2[:, 0])
     assert torch.all((amax.cpu() == o["argmax"]) | near_tie)
+
+
+@pytest.mark.parametrize("n,v,chunk", [(37, 1216, 256), (300, 1100, 512), (5, 700, 256)])
+@pytest.mark.parametrize("shifts", [(0, 0, 0, 0, 0), (-300, 0, 12, 40, 300), (300, 40, 0, -8, -1000),
+                                    (0, 5, -1000, 9, -60)])
+def test_single_pass_probabilities_over_logit_ranges(n, v, chunk, shifts):
+    """The stored probabilities are relative to references that follow the chunks' maxima: logits
+    whose level jumps between 256-row tiles, by less and by more than the window, up and down. The
+    reference forms softmax from the device's own fp16 logits in float64; each element of dH may
+    differ by P's fp16 rounding (2^-11 of each product, doubled) and fp32 sums of terms that size."""
+    g = torch.Generator().manual_seed(n + v)
+    d = 128
+    h = torch.randn(n, d, generator=g)
+    h[:, 0] = 4.0
+    w = torch.randn(v, d, generator=g) * 0.1
+    for t, s in enumerate(shifts):
+        w[256 * t: 256 * (t + 1), 0] = s / 4.0
+    h, w = h.half().to(DEV), w.half().to(DEV)
+    labels = torch.randint(0, v, (n,), generator=g)
+    labels[::3] = -100
+    labels = labels.to(DEV)
+    z = torch.empty(n, K._round_up(v, 64), dtype=torch.float16, device=DEV)
+    K.lm_head_ce_logits(h, w, z)
+    nll, lse, ent, amax, denom, dh, loss = K.lm_head_ce(h, w, labels, v_chunk=chunk)
+    torch.cuda.synchronize()
+    z = z[:, :v].double().cpu()
+    p = torch.softmax(z, -1)
+    assert torch.allclose(lse.double().cpu(), torch.logsumexp(z, -1), rtol=1e-6, atol=1e-5)
+    want_ent = torch.logsumexp(z, -1) - (p * z).sum(-1)
+    # w / s is of the logits' size and is subtracted from lse: fp32 resolution of that size
+    assert torch.all((ent.double().cpu() - want_ent).abs() <= 1e-5 + 1e-6 * z.abs().amax(-1))
+    assert torch.equal(amax.cpu(), z.argmax(-1))
+    valid = (labels != -100).cpu()
+    scale = 65536.0 / max(1, int(valid.sum()))
+    wd, y = w.double().cpu(), labels.clamp(min=0).cpu()
+    want = (p @ wd - wd[y]) * scale * valid[:, None]
+    tol = scale * (2.0**-10 * (p @ wd.abs()) + 1e-5 * (wd[y].abs() + p @ wd.abs())) + 1e-6
+    err = (dh.double().cpu() - want).abs()
+    assert bool((err <= tol).all()), float((err / tol).max())
