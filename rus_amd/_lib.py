@@ -181,10 +181,15 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_entry: dict = {}  # name -> C function of the loaded library
+
+
 def call(name: str, *args) -> None:
     """Calls one C entry point and raises RuntimeError with the library's message on failure."""
-    lib = load()
-    rc = getattr(lib, name)(*args)
+    fn = _entry.get(name)
+    if fn is None:
+        fn = _entry[name] = getattr(load(), name)
+    rc = fn(*args)
     if rc != 0:
-        msg = lib.rus_last_error().decode(errors="replace")
+        msg = load().rus_last_error().decode(errors="replace")
         raise RuntimeError(f"{name} failed (code {rc}): {msg}")

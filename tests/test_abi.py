@@ -242,6 +242,34 @@ def test_kept_logit_entry_points_validate_on_the_host(name, args, msg):
         _lib.call(name, *args)
 
 
+def test_lm_head_plans_equal_their_exhaustive_search():
+    """The chunk length and split count against every candidate, over token counts, vocabularies,
+    CU counts and budgets (ties: the longest chunk, the fewest splits)."""
+    import random
+
+    from rus_amd import kernels as K
+
+    def chunk_cost(k, tiles_v, tt, n_cu):
+        full, rest = divmod(tiles_v, k)
+        rounds = lambda t: -(-(-(-t * tt // 8) * 8) // n_cu)
+        return 50.0 * (full * rounds(k) + (rounds(rest) if rest else 0)) + 15.0 * (full + (rest > 0))
+
+    rng = random.Random(7)
+    for _ in range(300):
+        n, v = rng.choice([rng.randint(1, 600), rng.randint(1, 20000)]), rng.randint(257, 160000)
+        n_cu, budget = rng.choice([256, 128, 304, 7]), rng.choice([1 << 20, 128 << 20])
+        tiles_v, tt = -(-v // 256), -(-n // 256)
+        cap = max(1, min(tiles_v, budget // (512 * n)))
+        want = min(range(1, cap + 1), key=lambda k: (chunk_cost(k, tiles_v, tt, n_cu), -k))
+        assert K.lm_head_chunk_cols(n, v, n_cu, budget) == 256 * want, (n, v, n_cu, budget)
+
+        d, limit, kpad = 64 * rng.randint(1, 64), rng.randint(1, 80), -(-v // 64) * 64
+        tiles = tt * -(-d // 256)
+        counts = {-(-kpad // (-(-kpad // w // 64) * 64)) for w in range(1, min(64, limit, kpad // 64) + 1)}
+        best = max(counts, key=lambda c: (K._round_fill(tiles * c, n_cu), -c))
+        assert K.lm_head_split_count(n, d, v, n_cu, limit) == best, (n, d, v, n_cu, limit)
+
+
 def test_lm_head_split_count_fills_whole_rounds_of_workgroups():
     from rus_amd import kernels as K
 
