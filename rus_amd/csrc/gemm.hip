@@ -18,7 +18,7 @@ namespace {
 __device__ __forceinline__ void store_parts(const GemmArgs& g, const Tile& tl, float* parts,
                                             const f32x16 (&acc)[kMT][2]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 2, wn = wave & 3, h = lane >> 5;
+  const int wm = wave8_m(wave), wn = wave8_n(g, tl, wave), h = lane >> 5;
   float* base = parts + static_cast<int64_t>(tl.split) * g.M * g.N;
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {

@@ -58,7 +58,9 @@ __device__ __forceinline__ void store_tile_tv(char* smem, const GemmArgs& g, con
                                               f16* out, int64_t ld, int kpad, F value) {
   constexpr int NT = 16 / NW, RW = kBN / (NW / 2);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / (NW / 2), wn = wave % (NW / 2), h = lane >> 5;
+  const int wm = NW == 8 ? wave8_m(wave) : wave >> 1;
+  const int wn = NW == 8 ? wave8_n(g, tl, wave) : wave & 1;
+  const int h = lane >> 5;
   const int vrow0 = tl.m0 + wm * kWM;
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
@@ -158,7 +160,9 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
                                                f32x16 (&acc)[kMT][16 / NW]) {
   constexpr int NT = 16 / NW, RW = kBN / (NW / 2);  // token columns per wave: 128 or 64
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave / (NW / 2), wn = wave % (NW / 2), h = lane >> 5;
+  const int wm = NW == 8 ? wave8_m(wave) : wave >> 1;
+  const int wn = NW == 8 ? wave8_n(g, tl, wave) : wave & 1;
+  const int h = lane >> 5;
   const int vrow0 = tl.m0 + wm * kWM;  // local vocab row of this wave's first accumulator row
   const bool full = tl.m0 + kBM <= g.M;
   float rm[NT], rs[NT], rw[NT];
@@ -185,6 +189,8 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
     }
     float m = -INFINITY, tgt = 0.0f;
     int idx = 0x7fffffff;  // local row minus 4h until the end
+    rm[nt] = m, rs[nt] = rw[nt] = 0.0f, ri[nt] = idx;
+    if (tl.n0 + wn * RW + nt * 32 >= g.N) continue;  // no token here
     if (full) {
 #pragma unroll
       for (int mt = 0; mt < kMT; ++mt)
@@ -472,7 +478,7 @@ lmhead_grad_hidden_kernel(GemmArgs g, StoreParams p) {
   mainloop(g, tl, smem, acc);
 
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wm = wave >> 2, wn = wave & 3, h = lane >> 5;
+  const int wm = wave8_m(wave), wn = wave8_n(g, tl, wave), h = lane >> 5;
   float* base = p.parts + static_cast<int64_t>(tl.split) * g.M * g.N;
 #pragma unroll
   for (int nt = 0; nt < 2; ++nt) {

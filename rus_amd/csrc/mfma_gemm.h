@@ -57,14 +57,14 @@ __device__ __forceinline__ bool tile_of(const GemmArgs& g, Tile& t) {
 // split's K range. Accumulator layout (v_mfma_f32_32x32x16_f16): register r of lane l holds
 // row 8*(r/4) + 4*(l/32) + r%4, column l%32 of the 32x32 tile.
 //
-// Two pipelines. mainloop_t (the four-wave kernels: statistics and logit gradient) stages K 32 at
-// a time through NS LDS buffers of 32 KiB (A then B, 256 rows x 64 bytes each; NS = 4);
+// Two pipelines. mainloop_t (the four-wave logit-gradient kernel) stages K 32 at a time through
+// four LDS buffers of 32 KiB (A then B, 256 rows x 64 bytes each);
 // mainloop_k64 (the eight-wave kernels) stages K 64 at a time, below. Global memory is copied
 // straight into LDS (global_load_lds_dwordx4: each lane's 16 bytes land at buffer + lane * 16),
-// NS - 1 stages ahead of the MFMAs, so no register holds a tile in flight. The 16-byte chunk c of row r is stored
-// at chunk c ^ ((r >> 2) & 3) of its 64-byte row, which a lane realises by loading the chunk
-// that belongs at its position; the MFMAs' 16-byte fragment reads (16 consecutive rows per quarter
-// wave, one chunk) then hit all 64 banks once. The fragment reads are explicit ds_read_b128 with
+// three stages ahead of the MFMAs, so no register holds a tile in flight. The 16-byte chunk c of
+// row r is stored at chunk c ^ ((r >> 2) & 3) of its 64-byte row, which a lane realises by loading
+// the chunk that belongs at its position; the MFMAs' 16-byte fragment reads (16 consecutive rows
+// per quarter wave, one chunk) then hit all 64 banks once. The fragment reads are explicit ds_read_b128 with
 // explicit lgkmcnt waits (the compiler would otherwise wait for every LDS-bound global load before
 // any LDS read); vmcnt waits and the one barrier per stage sit inside the stage's second K step,
 // so the MFMA pipe keeps busy across stages.
@@ -83,48 +83,39 @@ __device__ __forceinline__ u32x4v lds_read16(uint32_t addr) {
   return v;
 }
 
-// The fragments of one K step of 16 from LDS addresses a (4 A row groups) / b (NT B row groups).
-template <int NT>
+// The fragments of one K step of 16 from LDS addresses a / b (4 row groups of A and of B).
 __device__ __forceinline__ void read_frags(uint32_t a, uint32_t b, u32x4v (&fa)[kMT],
-                                           u32x4v (&fb)[NT]) {
+                                           u32x4v (&fb)[kNT]) {
   fa[0] = lds_read16<0>(a);
   fa[1] = lds_read16<2048>(a);
   fa[2] = lds_read16<4096>(a);
   fa[3] = lds_read16<6144>(a);
   fb[0] = lds_read16<0>(b);
   fb[1] = lds_read16<2048>(b);
-  if constexpr (NT == 4) {
-    fb[2] = lds_read16<4096>(b);
-    fb[3] = lds_read16<6144>(b);
-  }
+  fb[2] = lds_read16<4096>(b);
+  fb[3] = lds_read16<6144>(b);
 }
 
 // Every LDS read issued so far has returned; ties the fragments so that no MFMA using them is
 // scheduled before the wait.
-template <int NT>
-__device__ __forceinline__ void wait_frags(u32x4v (&fa)[kMT], u32x4v (&fb)[NT]) {
-  if constexpr (NT == 4)
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fb[0]), "+v"(fb[1]),
-                   "+v"(fb[2]), "+v"(fb[3]));
-  else
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fb[0]), "+v"(fb[1]));
+__device__ __forceinline__ void wait_frags(u32x4v (&fa)[kMT], u32x4v (&fb)[kNT]) {
+  asm volatile("s_waitcnt lgkmcnt(0)"
+               : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(fb[0]), "+v"(fb[1]),
+                 "+v"(fb[2]), "+v"(fb[3]));
 }
 
-template <int NT>
-__device__ __forceinline__ void mma16(const u32x4v (&fa)[kMT], const u32x4v (&fb)[NT],
-                                      f32x16 (&acc)[kMT][NT]) {
+__device__ __forceinline__ void mma16(const u32x4v (&fa)[kMT], const u32x4v (&fb)[kNT],
+                                      f32x16 (&acc)[kMT][kNT]) {
 #pragma unroll
   for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
+    for (int nt = 0; nt < kNT; ++nt)
       acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
           __builtin_bit_cast(f16x8, fa[mt]), __builtin_bit_cast(f16x8, fb[nt]), acc[mt][nt], 0,
           0, 0);
 }
 
-// B stored [K][N] (N-contiguous) in LDS: 32 rows of 256 columns (512 bytes) per stage, the
+// B stored [K][N] (N-contiguous) in LDS: 64 rows of 256 columns (512 bytes) per stage, the
 // 16-byte chunk c of row r at chunk c ^ ((r & 3) << 2). ds_read_b64_tr_b16 lets each group of 16
 // lanes read a 4 x 16 block and transposes it: lane i of the group receives the 16-bit element
 // i % 4 of the 8 bytes read by lanes i / 4 + 4 e (e = 0..3) of the group. With lane j of the group
@@ -142,49 +133,6 @@ __device__ __forceinline__ u32x2v lds_read8_tr(uint32_t addr) {
 }
 
 constexpr int kKNRowBytes = kBN * 2;  // one K row of the B stage: 512 bytes
-
-// The fragments of K step KK (0 or 1) of a stage: A as read_frags, B from the per-tile addresses
-// b[nt] (+ sb, the stage's offset).
-template <int NT, int KK>
-__device__ __forceinline__ void read_frags_kn(uint32_t a, const uint32_t (&b)[NT], uint32_t sb,
-                                              u32x4v (&fa)[kMT], u32x2v (&lo)[NT],
-                                              u32x2v (&hi)[NT]) {
-  fa[0] = lds_read16<0>(a);
-  fa[1] = lds_read16<2048>(a);
-  fa[2] = lds_read16<4096>(a);
-  fa[3] = lds_read16<6144>(a);
-#pragma unroll
-  for (int nt = 0; nt < NT; ++nt) {
-    lo[nt] = lds_read8_tr<KK * 16 * kKNRowBytes>(b[nt] + sb);
-    hi[nt] = lds_read8_tr<KK * 16 * kKNRowBytes + 4 * kKNRowBytes>(b[nt] + sb);
-  }
-}
-
-template <int NT>
-__device__ __forceinline__ void wait_frags_kn(u32x4v (&fa)[kMT], u32x2v (&lo)[NT],
-                                              u32x2v (&hi)[NT]) {
-  if constexpr (NT == 4)
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(lo[0]), "+v"(lo[1]),
-                   "+v"(lo[2]), "+v"(lo[3]), "+v"(hi[0]), "+v"(hi[1]), "+v"(hi[2]), "+v"(hi[3]));
-  else
-    asm volatile("s_waitcnt lgkmcnt(0)"
-                 : "+v"(fa[0]), "+v"(fa[1]), "+v"(fa[2]), "+v"(fa[3]), "+v"(lo[0]), "+v"(lo[1]),
-                   "+v"(hi[0]), "+v"(hi[1]));
-}
-
-template <int NT>
-__device__ __forceinline__ void mma16_kn(const u32x4v (&fa)[kMT], const u32x2v (&lo)[NT],
-                                         const u32x2v (&hi)[NT], f32x16 (&acc)[kMT][NT]) {
-#pragma unroll
-  for (int mt = 0; mt < kMT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const u32x4v b = {lo[nt].x, lo[nt].y, hi[nt].x, hi[nt].y};
-      acc[mt][nt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(
-          __builtin_bit_cast(f16x8, fa[mt]), __builtin_bit_cast(f16x8, b), acc[mt][nt], 0, 0, 0);
-    }
-}
 
 // s_waitcnt vmcnt(N) (expcnt and lgkmcnt not waited on).
 template <int N>
@@ -208,37 +156,27 @@ __device__ __forceinline__ void wait_stages(int stages) {
     wait_vmcnt<0>();
 }
 
-// NW = 4: waves 2 (M halves) x 2 (N halves) of 128 x 128 (acc[4][4], one wave per SIMD), the
-// layout of the kernels whose epilogues need 4 x 4 accumulator tiles per wave; NW = 8: 2 x 4 waves
-// of 128 x 64 (acc[4][2]). Same LDS stages and A swizzle either way. KN: B is [K, ldb]
-// N-contiguous (NW = 8 only), staged as 32 K rows of 512 bytes per stage. The eight-wave kernels
-// run mainloop_k64 instead: its whole-line copies made them ~10% faster (isolated, same bits).
-template <int NW, bool KN = false, int NS = kNStages>
+// Waves 2 (M halves) x 2 (N halves) of 128 x 128 (acc[4][4], one wave per SIMD).
 __device__ __forceinline__ void mainloop_t(const GemmArgs& g, const Tile& tl, char* smem,
-                                           f32x16 (&acc)[kMT][16 / NW]) {
-  static_assert(!KN || NW == 8, "the N-contiguous B layout runs on eight waves");
-  constexpr int NT = 16 / NW;        // 32-column MFMA tiles per wave
-  constexpr int RW = kBN / (NW / 2);  // B rows (N) per wave: 128 or 64
-  constexpr int CP = 16 / NW;        // copies per thread per operand and stage: 4 or 2
+                                           f32x16 (&acc)[kMT][kNT]) {
+  constexpr int CP = 4;  // copies per thread per operand and stage
   constexpr int PER = 2 * CP;
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
-  const int wm = wave / (NW / 2), wn = wave % (NW / 2);
+  const int wm = wave >> 1, wn = wave & 1;
   const int kb = tl.split * g.k_per_split;
   const int ke = min(kb + g.k_per_split, g.K);
   const int KT = ke > kb ? (ke - kb) / kDK : 0;
 #pragma unroll
   for (int mt = 0; mt < kMT; ++mt)
 #pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x16{};
+    for (int nt = 0; nt < kNT; ++nt) acc[mt][nt] = f32x16{};
   if (KT == 0) {
     __syncthreads();
     return;
   }
-  // Copies: instruction i of wave w fills bytes 1024 (NW i + w) .. +1024 of the stage's A and B
-  // tiles. A (and K-contiguous B): rows 16 NW i + 16 w .. +16 of 64 bytes; lane l covers row
-  // 16 NW i + 16 w + l/4 at position l%4, i.e. the chunk (l%4) ^ ((l/16) & 3). N-contiguous B:
-  // K rows 2 (NW i + w) + l/32 of 512 bytes; lane l covers position l%32 of its row r, i.e. the
-  // chunk (l%32) ^ ((r & 3) << 2), columns n0 + 8 chunk .. +8.
+  // Copies: instruction i of wave w fills bytes 1024 (4 i + w) .. +1024 of the stage's A and B
+  // tiles: rows 64 i + 16 w .. +16 of 64 bytes; lane l covers row 64 i + 16 w + l/4 at position
+  // l%4, i.e. the chunk (l%4) ^ ((l/16) & 3).
   const int lrow = 16 * wave + (lane >> 2);
   const int lchunk = (lane & 3) ^ ((lane >> 4) & 3);
   const char* gA = reinterpret_cast<const char*>(g.A);
@@ -246,106 +184,62 @@ __device__ __forceinline__ void mainloop_t(const GemmArgs& g, const Tile& tl, ch
   uint32_t oa[CP], ob[CP];
 #pragma unroll
   for (int i = 0; i < CP; ++i) {
-    // Rows (columns) past the matrix edge re-read the last one: finite values the epilogues
-    // discard.
-    const int ra_ = min(tl.m0 + lrow + 16 * NW * i, g.M - 1);
+    // Rows past the matrix edge re-read the last one: finite values the epilogue discards.
+    const int ra_ = min(tl.m0 + lrow + 64 * i, g.M - 1);
+    const int rb_ = min(tl.n0 + lrow + 64 * i, g.N - 1);
     oa[i] = static_cast<uint32_t>((ra_ * g.lda + kb + lchunk * 8) * 2);
-    if constexpr (KN) {
-      const int krow = 2 * (NW * i + wave) + (lane >> 5);
-      const int col = min(tl.n0 + 8 * ((lane & 31) ^ ((krow & 3) << 2)), g.N - 8);
-      ob[i] = static_cast<uint32_t>(((kb + krow) * g.ldb + col) * 2);
-    } else {
-      const int rb_ = min(tl.n0 + lrow + 16 * NW * i, g.N - 1);
-      ob[i] = static_cast<uint32_t>((rb_ * g.ldb + kb + lchunk * 8) * 2);
-    }
+    ob[i] = static_cast<uint32_t>((rb_ * g.ldb + kb + lchunk * 8) * 2);
   }
-  const uint32_t bstep = KN ? static_cast<uint32_t>(kDK * g.ldb * 2) : kDK * 2;
-  auto issue = [&](int k) {  // stage k's copies into buffer k % NS
-    char* st = smem + (k % NS) * kStageBytes;
-    const uint32_t abytes = k * (kDK * 2), bbytes = k * bstep;
+  auto issue = [&](int k) {  // stage k's copies into buffer k % kNStages
+    char* st = smem + (k % kNStages) * kStageBytes;
+    const uint32_t bytes = k * (kDK * 2);
 #pragma unroll
     for (int i = 0; i < CP; ++i) {
-      __builtin_amdgcn_global_load_lds(gA + oa[i] + abytes,
-                                       (lds_void_ptr)(st + (NW * i + wave) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds(gB + ob[i] + bbytes,
-                                       (lds_void_ptr)(st + kBM * 64 + (NW * i + wave) * 1024), 16,
+      __builtin_amdgcn_global_load_lds(gA + oa[i] + bytes,
+                                       (lds_void_ptr)(st + (4 * i + wave) * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds(gB + ob[i] + bytes,
+                                       (lds_void_ptr)(st + kBM * 64 + (4 * i + wave) * 1024), 16,
                                        0, 0);
     }
   };
-  const int pre = min(NS, KT);
+  const int pre = min(kNStages, KT);
   for (int k = 0; k < pre; ++k) issue(k);
   wait_stages<PER>(pre - 1);  // stage 0 landed (this wave's copies)
   __builtin_amdgcn_s_barrier();  // ... and every wave's
-  // Fragment addresses: A row wm*128 + (l & 31), B row wn*RW + (l & 31) (+ 32 per MFMA tile,
-  // immediate), chunk 2 kk + l/32 stored at chunk ^ ((l >> 2) & 3). N-contiguous B: lane l of
-  // group g = l/16 (j = l%16) reads K row 16 kk + 8 (g/2) + j/4 (+ 4 for the high half), columns
-  // wn*64 + 32 nt + 16 (g%2) + 4 (j%4).
+  // Fragment addresses: A row wm*128 + (l & 31), B row wn*128 + (l & 31) (+ 32 per MFMA tile,
+  // immediate), chunk 2 kk + l/32 stored at chunk ^ ((l >> 2) & 3).
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_void_ptr)smem));
   const int sw = (lane >> 2) & 3, half = lane >> 5;
   const uint32_t c0 = ((0 + half) ^ sw) << 4, c1 = ((2 + half) ^ sw) << 4;
   const uint32_t arow = lds0 + (wm * kWM + (lane & 31)) * 64;
   const uint32_t a0 = arow + c0, a1 = arow + c1;
-  if constexpr (KN) {
-    const int j = lane & 15, nh = (lane >> 4) & 1;
-    uint32_t bk[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) {
-      const int col = wn * RW + nt * 32 + 16 * nh + 4 * (j & 3);
-      bk[nt] = lds0 + kBM * 64 + (8 * half + (j >> 2)) * kKNRowBytes +
-               (((col >> 3) ^ ((j >> 2) << 2)) << 4) + (col & 7) * 2;
+  const uint32_t brow = lds0 + kBM * 64 + (wn * kWN + (lane & 31)) * 64;
+  const uint32_t b0 = brow + c0, b1 = brow + c1;
+  u32x4v fa0[kMT], fb0[kNT], fa1[kMT], fb1[kNT];
+  read_frags(a0, b0, fa0, fb0);
+  wait_frags(fa0, fb0);
+  for (int k = 0; k < KT; ++k) {
+    const uint32_t sb = (k % kNStages) * kStageBytes;
+    read_frags(a1 + sb, b1 + sb, fa1, fb1);  // step 1 of stage k
+    __builtin_amdgcn_sched_barrier(0);
+    mma16(fa0, fb0, acc);  // step 0 of stage k
+    __builtin_amdgcn_sched_barrier(0);
+    wait_frags(fa1, fb1);
+    if (k + 1 < KT) {
+      // Stage k + 1 has landed for every wave, and every wave has read stage k: its buffer
+      // takes stage k + 4.
+      wait_stages<PER>(min(kNStages - 2, KT - 2 - k));
+      __builtin_amdgcn_s_barrier();
+      if (k + kNStages < KT) issue(k + kNStages);
+      const uint32_t nb = ((k + 1) % kNStages) * kStageBytes;
+      read_frags(a0 + nb, b0 + nb, fa0, fb0);  // step 0 of stage k + 1
     }
-    u32x4v fa0[kMT], fa1[kMT];
-    u32x2v lo0[NT], hi0[NT], lo1[NT], hi1[NT];
-    read_frags_kn<NT, 0>(a0, bk, 0, fa0, lo0, hi0);
-    wait_frags_kn<NT>(fa0, lo0, hi0);
-    for (int k = 0; k < KT; ++k) {
-      const uint32_t sb = (k % NS) * kStageBytes;
-      read_frags_kn<NT, 1>(a1 + sb, bk, sb, fa1, lo1, hi1);  // step 1 of stage k
-      __builtin_amdgcn_sched_barrier(0);
-      mma16_kn<NT>(fa0, lo0, hi0, acc);  // step 0 of stage k
-      __builtin_amdgcn_sched_barrier(0);
-      wait_frags_kn<NT>(fa1, lo1, hi1);
-      if (k + 1 < KT) {
-        wait_stages<PER>(min(NS - 2, KT - 2 - k));
-        __builtin_amdgcn_s_barrier();
-        if (k + NS < KT) issue(k + NS);
-        const uint32_t nb = ((k + 1) % NS) * kStageBytes;
-        read_frags_kn<NT, 0>(a0 + nb, bk, nb, fa0, lo0, hi0);  // step 0 of stage k + 1
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      mma16_kn<NT>(fa1, lo1, hi1, acc);  // step 1 of stage k
-      __builtin_amdgcn_sched_barrier(0);
-      if (k + 1 < KT) wait_frags_kn<NT>(fa0, lo0, hi0);
-    }
-  } else {
-    const uint32_t brow = lds0 + kBM * 64 + (wn * RW + (lane & 31)) * 64;
-    const uint32_t b0 = brow + c0, b1 = brow + c1;
-    u32x4v fa0[kMT], fb0[NT], fa1[kMT], fb1[NT];
-    read_frags<NT>(a0, b0, fa0, fb0);
-    wait_frags<NT>(fa0, fb0);
-    for (int k = 0; k < KT; ++k) {
-      const uint32_t sb = (k % NS) * kStageBytes;
-      read_frags<NT>(a1 + sb, b1 + sb, fa1, fb1);  // step 1 of stage k
-      __builtin_amdgcn_sched_barrier(0);
-      mma16<NT>(fa0, fb0, acc);  // step 0 of stage k
-      __builtin_amdgcn_sched_barrier(0);
-      wait_frags<NT>(fa1, fb1);
-      if (k + 1 < KT) {
-        // Stage k + 1 has landed for every wave, and every wave has read stage k: its buffer
-        // takes stage k + 4.
-        wait_stages<PER>(min(NS - 2, KT - 2 - k));
-        __builtin_amdgcn_s_barrier();
-        if (k + NS < KT) issue(k + NS);
-        const uint32_t nb = ((k + 1) % NS) * kStageBytes;
-        read_frags<NT>(a0 + nb, b0 + nb, fa0, fb0);  // step 0 of stage k + 1
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      mma16<NT>(fa1, fb1, acc);  // step 1 of stage k
-      __builtin_amdgcn_sched_barrier(0);
-      if (k + 1 < KT) wait_frags<NT>(fa0, fb0);
-    }
+    __builtin_amdgcn_sched_barrier(0);
+    mma16(fa1, fb1, acc);  // step 1 of stage k
+    __builtin_amdgcn_sched_barrier(0);
+    if (k + 1 < KT) wait_frags(fa0, fb0);
   }
-  __syncthreads();  // the epilogues reuse the LDS
+  __syncthreads();  // the epilogue reuses the LDS
 }
 
 // Eight waves (2 x 4 of 128 x 64) with K staged 64 at a time through two 64 KiB LDS buffers:
@@ -404,6 +298,20 @@ __device__ __forceinline__ void wait_set(FragB<true>& f) {
                  "+v"(f.hi[1]), "+v"(f.hi[2]), "+v"(f.hi[3]));
 }
 
+// Wave w of eight's rows (128 wave8_m) and columns (64 wave8_n) of the tile. A wave with none of
+// them inside the matrix takes part in the copies and barriers only, and so that the others still
+// use four SIMDs (wave w is on SIMD w % 4), a tile that is not whole deals its waves so that those
+// of either half of the rows, or of two neighbouring quarters of the columns, are on different
+// ones. Such a tile then takes about half the time where its MFMAs count (345 tokens' statistics
+// 262 -> 248 us, a training pass at 16 tokens 383 -> 342, at 100 465 -> 435, at 345 675 -> 642; the
+// other deal costs a whole tile 0.5%). Leaving out the copies as well gave another 1-3% below 128
+// tokens, at seven conditions in the loop.
+__device__ __forceinline__ int wave8_m(int wave) { return wave >> 2; }
+__device__ __forceinline__ int wave8_n(const GemmArgs& g, const Tile& tl, int wave) {
+  const bool whole = tl.m0 + kWM < g.M && tl.n0 + 192 < g.N;
+  return (wave & 3) ^ (whole ? 0 : (wave >> 2) << 1);
+}
+
 template <bool KN>
 __device__ __forceinline__ void mainloop_k64(const GemmArgs& g, const Tile& tl, char* smem,
                                              f32x16 (&acc)[kMT][2]) {
@@ -411,7 +319,7 @@ __device__ __forceinline__ void mainloop_k64(const GemmArgs& g, const Tile& tl, 
   constexpr int PER = 2 * CP;
   const int t = threadIdx.x, lane = t & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(t >> 6));
-  const int wm = wave >> 2, wn = wave & 3;
+  const int wm = wave8_m(wave), wn = wave8_n(g, tl, wave);
   const int kb = tl.split * g.k_per_split;
   const int ke = min(kb + g.k_per_split, g.K);
   const int KT = ke > kb ? (ke - kb) / kDK64 : 0;
@@ -528,6 +436,15 @@ __device__ __forceinline__ void mainloop_k64(const GemmArgs& g, const Tile& tl, 
   else
     wait_vmcnt<0>();
   __builtin_amdgcn_s_barrier();  // ... and every wave's
+  if (tl.m0 + wm * kWM >= g.M || tl.n0 + wn * 64 >= g.N) {  // the stages' copies and barriers
+    for (int k = 0; k + 1 < KT; ++k) {
+      wait_vmcnt<0>();
+      __builtin_amdgcn_s_barrier();
+      if (k + 2 < KT) issue(k + 2);
+    }
+    __syncthreads();
+    return;
+  }
   each([&](auto kk) { read_a(a0, 0, kk, C0{}); });
   each([&](auto kk) { read_b(b0, 0, kk, C0{}); });
   wait_set(a0);
@@ -572,7 +489,7 @@ __device__ __forceinline__ void mainloop_k64(const GemmArgs& g, const Tile& tl, 
 
 __device__ __forceinline__ void mainloop(const GemmArgs& g, const Tile& tl, char* smem,
                                          f32x16 (&acc)[kMT][4]) {
-  mainloop_t<4>(g, tl, smem, acc);
+  mainloop_t(g, tl, smem, acc);
 }
 
 __device__ __forceinline__ void mainloop(const GemmArgs& g, const Tile& tl, char* smem,

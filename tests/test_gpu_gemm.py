@@ -64,6 +64,17 @@ def test_gemm_parts_matches_fp32_product(m, n, k, n_split, b_kn):
 
 
 @pytest.mark.parametrize("b_kn", [True, False])
+@pytest.mark.parametrize("m", [1, 128, 129, 256, 385])
+@pytest.mark.parametrize("n", [8, 64, 72, 128, 136, 192, 200, 256, 264, 384])
+def test_gemm_parts_of_tiles_partly_inside_the_matrix(m, n, b_kn):
+    """Row halves and column quarters of a tile outside the matrix are neither copied nor
+    multiplied: sizes on both sides of each, over one to three 64-deep stages per split."""
+    for k, n_split in ((64, 1), (128, 1), (320, 2)):
+        a, b = _operands(m, n, k, b_kn, seed=m + n + k)
+        _check(a, b, b_kn, n_split, k)
+
+
+@pytest.mark.parametrize("b_kn", [True, False])
 def test_gemm_parts_strided_operands(b_kn):
     m, n, k = 130, 264, 320
     a, b = _operands(m, n, k, b_kn, seed=5, pad_a=24, pad_b=40)

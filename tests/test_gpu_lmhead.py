@@ -355,3 +355,24 @@ def test_single_pass_probabilities_over_logit_ranges(n, v, chunk, shifts):
     tol = scale * (2.0**-10 * (p @ wd.abs()) + 1e-5 * (wd[y].abs() + p @ wd.abs())) + 1e-6
     err = (dh.double().cpu() - want).abs()
     assert bool((err <= tol).all()), float((err / tol).max())
+
+
+@pytest.mark.parametrize("n", [1, 32, 33, 64, 65, 128, 129, 192, 193, 256, 257, 352])
+def test_lmhead_of_token_tiles_partly_filled(n):
+    """Column quarters of a tile without a token are left out: token counts on both sides of each
+    (and of the 32 tokens of an MFMA tile), with a last vocabulary tile half inside. 64 items: the
+    oracle's gradient is 2^16 / items times at most 1 x |w|, |w| < 0.6, in fp16 (with the one item
+    of the smallest case it overflows)."""
+    g = torch.Generator().manual_seed(n)
+    d, v = 128, 1100
+    h = torch.randn(n, d, generator=g).half()
+    w = (torch.randn(v, d, generator=g) * 0.1).half()
+    lab = torch.randint(0, v, (n,), generator=g)
+    lab[1::7] = -100
+    for chunk in (512, None):
+        out = K.lm_head_ce(h.to(DEV), w.to(DEV), lab.to(DEV), num_items_in_batch=64.0,
+                           v_chunk=chunk)
+        _check_against_oracle(h, w, lab, out, denom=64.0)
+    out = K.lm_head_ce(h.to(DEV), w.to(DEV), lab.to(DEV), num_items_in_batch=64.0,
+                       need_grad=False)
+    _check_against_oracle(h, w, lab, out, denom=64.0, check_dh=False)
