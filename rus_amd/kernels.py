@@ -1424,31 +1424,51 @@ LM_CHUNK_BUDGET = 128 << 20  # bytes of fp16 logits one chunk of the single-pass
 
 
 def lm_head_chunk_cols(n_tok: int, n_vocab: int, n_cu: int = 256,
-                       budget: int = LM_CHUNK_BUDGET) -> int:
+                       budget: int = LM_CHUNK_BUDGET, at_least_two: bool = False) -> int:
     """Vocabulary rows per chunk of the single-pass head: a multiple of 256 whose fp16 logits
     [n_tok, cols] fit ``budget``, chosen to minimise an estimate of the statistics GEMM time
-    (whole rounds of one-per-CU 256x256 tiles, ~50 us each) plus a per-chunk cost for the three
-    launches of a chunk (~15 us). Among the chunks of one number of rounds the longest costs the
-    least (no more chunks, no more rounds of the rest), so only those are compared: a few per call,
-    which every new n_tok makes (150 us of host time when every length was)."""
+    (whole rounds of one-per-CU 256x256 tiles, ~45 us each) plus a per-chunk cost (~60 us: two
+    launches, the fp32 partials read and rewritten, a GEMM's ramp). Among the chunks of one number
+    of rounds the longest costs the least (no more chunks, no more rounds of the rest), so only
+    those are compared: a few per call, which every new n_tok makes (150 us of host time when
+    every length was).
+
+    ``at_least_two``: never the whole vocabulary in one chunk; where one would be best, two halves,
+    or two chunks of unequal length where that saves a round (up to 256 tokens, 594 tiles: 512 + 82
+    take 2 + 1 rounds of 256 where halves take 2 + 2; a pass at 100 tokens 413 -> 360 us, at 256
+    525 -> 456; at 345 tokens 4 + 1 rounds instead of 3 + 3, 621 -> 577)."""
     tiles_v = -(-n_vocab // LM_TILE)
     if tiles_v <= 1 or n_tok <= 0:
         return max(LM_TILE, tiles_v * LM_TILE)
     tt = -(-n_tok // 256)
-    cap = max(1, min(tiles_v, budget // (2 * LM_TILE * n_tok)))
-    best, best_cost, k, per_chunk = 1, None, 0, 0
-    while k < cap:
-        per_chunk += 1
-        k = min(cap, (per_chunk * n_cu // 8 * 8) // tt)
-        if k < 1:
-            continue
+
+    def rounds(tiles):
+        return -(-(-(-tiles * tt // 8) * 8) // n_cu)
+
+    def cost(k):
         full, rest = divmod(tiles_v, k)
-        rounds = full * -(-(-(-k * tt // 8) * 8) // n_cu)
-        if rest:
-            rounds += -(-(-(-rest * tt // 8) * 8) // n_cu)
-        cost = 50.0 * rounds + 15.0 * (full + (1 if rest else 0))
-        if best_cost is None or cost <= best_cost:
-            best, best_cost = k, cost
+        return 45.0 * (full * rounds(k) + (rounds(rest) if rest else 0)) + \
+            60.0 * (full + (1 if rest else 0))
+
+    def best_up_to(cap):
+        best, best_cost, k, per_chunk = 1, None, 0, 0
+        while k < cap:
+            per_chunk += 1
+            k = min(cap, (per_chunk * n_cu // 8 * 8) // tt)
+            if k < 1:
+                continue
+            c = cost(k)
+            if best_cost is None or c <= best_cost:
+                best, best_cost = k, c
+        return best
+
+    cap = max(1, min(tiles_v, budget // (2 * LM_TILE * n_tok)))
+    best = best_up_to(cap)
+    if at_least_two and best == tiles_v:
+        half = -(-tiles_v // 2)
+        best = best_up_to(min(cap, tiles_v - 1))
+        if cost(half) <= cost(best):
+            best = half
     return best * LM_TILE
 
 
@@ -2139,8 +2159,7 @@ def lm_head_ce(hidden: torch.Tensor, weight: torch.Tensor, labels: torch.Tensor,
         # A batch within one 256-token tile: split into token blocks, each block's GEMMs would
         # read all of W on a half-empty tile (twice the cost of one pass); the pass over at
         # least two vocabulary chunks reads W once and still never holds [N, V] logits.
-        v_chunk = min(lm_head_chunk_cols(n_tok, V, cu_count(dev)),
-                      _round_up(-(-V // 2), LM_TILE))
+        v_chunk = lm_head_chunk_cols(n_tok, V, cu_count(dev), at_least_two=True)
     if v_chunk is not None:
         chunk = int(v_chunk)
         if chunk <= 0 or (chunk < V and chunk % LM_TILE):

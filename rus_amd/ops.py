@@ -191,10 +191,7 @@ def lm_head_layout(v_chunk, n_tok: int, n_vocab: int, device):
     two chunks, so that no buffer holds a logit row of the whole vocabulary; a positive multiple
     of 256 -> that chunk; 0 -> None (the token-blocked head)."""
     if v_chunk is None or v_chunk < 0:
-        c = K.lm_head_chunk_cols(n_tok, n_vocab, K.cu_count(device))
-        if c >= n_vocab and n_vocab > K.LM_TILE:  # two chunks of whole 256-row tiles
-            return K._round_up(-(-n_vocab // 2), K.LM_TILE)
-        return c
+        return K.lm_head_chunk_cols(n_tok, n_vocab, K.cu_count(device), at_least_two=True)
     return int(v_chunk) if v_chunk > 0 else None
 
 

@@ -252,7 +252,7 @@ def test_lm_head_plans_equal_their_exhaustive_search():
     def chunk_cost(k, tiles_v, tt, n_cu):
         full, rest = divmod(tiles_v, k)
         rounds = lambda t: -(-(-(-t * tt // 8) * 8) // n_cu)
-        return 50.0 * (full * rounds(k) + (rounds(rest) if rest else 0)) + 15.0 * (full + (rest > 0))
+        return 45.0 * (full * rounds(k) + (rounds(rest) if rest else 0)) + 60.0 * (full + (rest > 0))
 
     rng = random.Random(7)
     for _ in range(300):
@@ -262,6 +262,11 @@ def test_lm_head_plans_equal_their_exhaustive_search():
         cap = max(1, min(tiles_v, budget // (512 * n)))
         want = min(range(1, cap + 1), key=lambda k: (chunk_cost(k, tiles_v, tt, n_cu), -k))
         assert K.lm_head_chunk_cols(n, v, n_cu, budget) == 256 * want, (n, v, n_cu, budget)
+        if want == tiles_v:  # at least two chunks: the best of those, halves on a tie
+            half = -(-tiles_v // 2)
+            want = min(range(1, tiles_v), key=lambda k: (chunk_cost(k, tiles_v, tt, n_cu), k != half, -k))
+        two = K.lm_head_chunk_cols(n, v, n_cu, budget, at_least_two=True)
+        assert two == 256 * want and two < v, (n, v, n_cu, budget)
 
         d, limit, kpad = 64 * rng.randint(1, 64), rng.randint(1, 80), -(-v // 64) * 64
         tiles = tt * -(-d // 256)
