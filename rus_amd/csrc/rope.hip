@@ -19,6 +19,9 @@
 namespace rus {
 namespace {
 
+typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
+
 constexpr int kThreads = 256;
 constexpr int kSpan = 8;  // elements per thread in each half of a head
 constexpr int kMaxMidHead = 256;  // largest head_dim of the in-kernel LoRA delta (B rows in LDS)
@@ -64,23 +67,31 @@ __device__ __forceinline__ int b_slot(int c) { return (c & ~7) | ((c & 7) ^ ((c 
 
 // The LoRA delta of columns col0 .. col0+7 and col0+half .. +7 from mid row m and B [cols, R]
 // (rows in b_slot order): fp16(sum_k m[k] * B[col, k]), the reference's fp16 mid B^T product
-// (ops.py:776-778).
-template <typename T, int R>
-__device__ __forceinline__ void lora_up(const float (&m)[R], const T* __restrict__ b, int col0,
+// (ops.py:776-778), products and sums in fp32, two per instruction (one at a time, with the
+// conversions: 22.8 us at 8,161 tokens, now 20.6; 70 MB, 14 us at the rate of a copy).
+template <int R, int ALIGN>
+struct alignas(ALIGN) RankRow {
+  f16x2_t v[R / 2];
+};
+template <int R>
+using MidRow = RankRow<R, 8>;
+
+template <int R>
+__device__ __forceinline__ float dot_row(const MidRow<R>& m, const f16* __restrict__ b) {
+  const auto row = *reinterpret_cast<const RankRow<R, (R >= 8 ? 16 : 8)>*>(b);  // in the LDS
+  float s = 0.0f;
+#pragma unroll
+  for (int k = 0; k < R / 2; ++k) s = __builtin_amdgcn_fdot2(m.v[k], row.v[k], s, false);
+  return s;
+}
+
+template <int R>
+__device__ __forceinline__ void lora_up(const MidRow<R>& m, const f16* __restrict__ b, int col0,
                                         int half, float (&dl)[kSpan], float (&dh)[kSpan]) {
 #pragma unroll
   for (int i = 0; i < kSpan; ++i) {
-    float bl[R], bh[R];
-    load_f32<T, R>(b + b_slot(col0 + i) * R, bl);
-    load_f32<T, R>(b + b_slot(col0 + half + i) * R, bh);
-    float sl = 0.0f, sh = 0.0f;
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-      sl = __builtin_fmaf(m[k], bl[k], sl);
-      sh = __builtin_fmaf(m[k], bh[k], sh);
-    }
-    dl[i] = round_to<T>(sl);
-    dh[i] = round_to<T>(sh);
+    dl[i] = round_to<f16>(dot_row<R>(m, b + b_slot(col0 + i) * R));
+    dh[i] = round_to<f16>(dot_row<R>(m, b + b_slot(col0 + half + i) * R));
   }
 }
 
@@ -130,9 +141,9 @@ __global__ __launch_bounds__(kThreads) void rope_fwd_kernel(RopeFwdArgs<T> a) {
   if (is_v) {  // V head: LoRA delta only
     const int kv = hd - a.h_q - a.h_kv;
     if constexpr (LORA == 2) {
-      float m[R], dl[kSpan], dh[kSpan];
-      load_f32<T, R>(a.mid_v + t * R, m);
-      lora_up<T, R>(m, s_b, j, half, dl, dh);
+      float dl[kSpan], dh[kSpan];
+      const MidRow<R> m = *reinterpret_cast<const MidRow<R>*>(a.mid_v + t * R);
+      lora_up<R>(m, s_b, j, half, dl, dh);
 #pragma unroll
       for (int i = 0; i < kSpan; ++i) {
         lo[i] = lo[i] + dl[i] * a.scale_v;
@@ -159,9 +170,9 @@ __global__ __launch_bounds__(kThreads) void rope_fwd_kernel(RopeFwdArgs<T> a) {
   } else {
     if constexpr (LORA == 2) {
       if (is_q) {
-        float m[R], dl[kSpan], dh[kSpan];
-        load_f32<T, R>(a.mid_q + t * R, m);
-        lora_up<T, R>(m, s_b, j, half, dl, dh);
+        float dl[kSpan], dh[kSpan];
+        const MidRow<R> m = *reinterpret_cast<const MidRow<R>*>(a.mid_q + t * R);
+        lora_up<R>(m, s_b, j, half, dl, dh);
 #pragma unroll
         for (int i = 0; i < kSpan; ++i) {
           lo[i] = lo[i] + dl[i] * a.scale_q;
@@ -344,24 +355,20 @@ __device__ __forceinline__ float group16_transpose_sum(const float (&p)[16], int
   return (b0 ? v2[1] : v2[0]) + __shfl_xor(send, 1);
 }
 
-typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
-
-// p[r] += sum_i lo[i] bt[r][c + i] + hi[i] bt[r][c + half + i], the B^T fragments loaded rank by
-// rank (holding all sixteen ranks' fragments at once took 213 VGPRs, two waves per SIMD).
-__device__ __forceinline__ void mid_partial(float (&p)[kMidR], const float (&lo)[kSpan],
-                                                     const float (&hi)[kSpan],
-                                                     const f16* __restrict__ bt, int64_t d,
-                                                     int64_t c, int half) {
-#pragma unroll
-  for (int r = 0; r < kMidR; ++r) {
-    const f16x8_t bl = *reinterpret_cast<const f16x8_t*>(bt + r * d + c);
-    const f16x8_t bh = *reinterpret_cast<const f16x8_t*>(bt + r * d + c + half);
-#pragma unroll
-    for (int i = 0; i < kSpan; ++i)
-      p[r] += lo[i] * static_cast<float>(bl[i]) + hi[i] * static_cast<float>(bh[i]);
-  }
+// acc + x . y over 8 fp16 pairs, products and sums in fp32 (two per instruction).
+__device__ __forceinline__ float dot8(f16x8_t x, f16x8_t y, float acc) {
+  acc = __builtin_amdgcn_fdot2(f16x2_t{x[0], x[1]}, f16x2_t{y[0], y[1]}, acc, false);
+  acc = __builtin_amdgcn_fdot2(f16x2_t{x[2], x[3]}, f16x2_t{y[2], y[3]}, acc, false);
+  acc = __builtin_amdgcn_fdot2(f16x2_t{x[4], x[5]}, f16x2_t{y[4], y[5]}, acc, false);
+  return __builtin_amdgcn_fdot2(f16x2_t{x[6], x[7]}, f16x2_t{y[6], y[7]}, acc, false);
 }
 
+// Bound by memory (190 MB at 8,161 tokens with the fp32 partials: 37 us at the rate of a copy) once
+// the products are out of the way: with the ranks' fragments converted and multiplied element by
+// element, and loaded again for every token (57 KB per token, more than the L1 holds), that shape
+// took 50.1 us and 707 tokens 8.5; two products per instruction 45.4 and 7.1; and T tokens per
+// thread (the same columns of tokens tpb apart) sharing each load 36.1.
+template <int T>
 __global__ __launch_bounds__(kThreads) void rope_bwd_mid_kernel(RopeBwdMidArgs m) {
   const RopeBwdArgs<f16>& a = m.b;
   const int half = a.head_dim / 2;
@@ -371,25 +378,24 @@ __global__ __launch_bounds__(kThreads) void rope_bwd_mid_kernel(RopeBwdMidArgs m
   const int tpb = kThreads / slots;
   const int tb = threadIdx.x / slots;
   const int slot = threadIdx.x - tb * slots;
-  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * tpb;
-  const int64_t t = t0 + tb;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * (tpb * T);
   const int hd = slot / per_head;
   const int j = (slot - hd * per_head) * kSpan;
   const int lane = threadIdx.x & 63;
   const int64_t d_q = static_cast<int64_t>(a.h_q) * a.head_dim;
   const int64_t d_v = static_cast<int64_t>(a.h_kv) * a.head_dim;
 
-  float p[kMidR];
-#pragma unroll
-  for (int r = 0; r < kMidR; ++r) p[r] = 0.0f;
   const bool is_q = hd < a.h_q, is_v = hd >= a.h_q + a.h_kv;
-  const f16* bt = is_q ? m.bt_q : m.bt_v;
-  const int64_t bd = is_q ? d_q : d_v;
-  const int64_t bc = static_cast<int64_t>(is_q ? hd : hd - a.h_q - a.h_kv) * a.head_dim + j;
-  if (t < a.n_tokens) {
+  const int kv = is_v ? hd - a.h_q - a.h_kv : hd - a.h_q;  // KV head of a k / v slot
+  f16x8_t gl[T], gh[T];  // the stored dq_lora / dv_lora values
+#pragma unroll
+  for (int u = 0; u < T; ++u) {
+    gl[u] = f16x8_t{};
+    gh[u] = f16x8_t{};
+    const int64_t t = t0 + u * tpb + tb;
+    if (t >= a.n_tokens) continue;
     // One store site per output for every head kind (see rope_fwd_kernel).
     f16* out = a.dqkv + t * a.stride_dqkv + static_cast<int64_t>(hd) * a.head_dim;
-    const int kv = is_v ? hd - a.h_q - a.h_kv : hd - a.h_q;  // KV head of a k / v slot
     float lo[kSpan], hi[kSpan], ol[kSpan], oh[kSpan];
     const float* part = is_v ? m.dv_part : is_q ? nullptr : m.dk_part;
     if (part) {  // dK / dV from the attention backward's per-query-head partials
@@ -426,33 +432,53 @@ __global__ __launch_bounds__(kThreads) void rope_bwd_mid_kernel(RopeBwdMidArgs m
     }
     store_from_f32<f16, kSpan>(out + j, ol);
     store_from_f32<f16, kSpan>(out + j + half, oh);
-    if (is_v || is_q) {  // the scaled LoRA gradient rows and their d_mid partials
+    if (is_v || is_q) {  // the scaled LoRA gradient rows
       const float sc = is_v ? a.scale_v : a.scale_q;
 #pragma unroll
       for (int i = 0; i < kSpan; ++i) {
-        ol[i] = round_to<f16>(ol[i] * sc);  // the stored dq_lora / dv_lora values
-        oh[i] = round_to<f16>(oh[i] * sc);
+        gl[u][i] = from_f32<f16>(ol[i] * sc);
+        gh[u][i] = from_f32<f16>(oh[i] * sc);
       }
       f16* l = is_v ? a.dv_lora + (t * a.h_kv + kv) * a.head_dim
                     : a.dq_lora + (t * a.h_q + hd) * a.head_dim;
-      store_from_f32<f16, kSpan>(l + j, ol);
-      store_from_f32<f16, kSpan>(l + j + half, oh);
-      mid_partial(p, ol, oh, bt, bd, bc, half);
+      *reinterpret_cast<f16x8_t*>(l + j) = gl[u];
+      *reinterpret_cast<f16x8_t*>(l + j + half) = gh[u];
     }
   }
-  __shared__ float red[kThreads / 16][kMidR];
-  red[threadIdx.x >> 4][threadIdx.x & 15] = group16_transpose_sum(p, lane);
+  // The d_mid partials, the B^T fragments loaded rank by rank for the T tokens (holding all sixteen
+  // ranks' fragments at once took 213 VGPRs, two waves per SIMD).
+  float p[T][kMidR];
+#pragma unroll
+  for (int u = 0; u < T; ++u)
+#pragma unroll
+    for (int r = 0; r < kMidR; ++r) p[u][r] = 0.0f;
+  if (is_q || is_v) {
+    const int64_t bd = is_q ? d_q : d_v;
+    const f16* bt = (is_q ? m.bt_q : m.bt_v) + static_cast<int64_t>(is_q ? hd : kv) * a.head_dim + j;
+#pragma unroll
+    for (int r = 0; r < kMidR; ++r) {
+      const f16x8_t bl = *reinterpret_cast<const f16x8_t*>(bt + r * bd);
+      const f16x8_t bh = *reinterpret_cast<const f16x8_t*>(bt + r * bd + half);
+#pragma unroll
+      for (int u = 0; u < T; ++u) p[u][r] = dot8(gh[u], bh, dot8(gl[u], bl, 0.0f));
+    }
+  }
+  __shared__ float red[T][kThreads / 16][kMidR];
+#pragma unroll
+  for (int u = 0; u < T; ++u)
+    red[u][threadIdx.x >> 4][threadIdx.x & 15] = group16_transpose_sum(p[u], lane);
   __syncthreads();
   const int groups = slots / 16;
   const int gq = a.h_q * per_head / 16, gv0 = (a.h_q + a.h_kv) * per_head / 16;
-  if (threadIdx.x < tpb * 2 * kMidR) {
-    const int tk = threadIdx.x / (2 * kMidR), rr = threadIdx.x % (2 * kMidR);
+  for (int i = threadIdx.x; i < T * tpb * 2 * kMidR; i += kThreads) {
+    const int tk = i / (2 * kMidR), rr = i % (2 * kMidR);  // token t0 + tk
     const int64_t tt = t0 + tk;
     if (tt < a.n_tokens) {
       const bool out_q = rr < kMidR;
       const int r = out_q ? rr : rr - kMidR;
+      const int u = tk / tpb, row = (tk - u * tpb) * groups;
       float acc = 0.0f;
-      for (int g = out_q ? 0 : gv0; g < (out_q ? gq : groups); ++g) acc += red[tk * groups + g][r];
+      for (int g = out_q ? 0 : gv0; g < (out_q ? gq : groups); ++g) acc += red[u][row + g][r];
       (out_q ? m.dmid_q : m.dmid_v)[tt * kMidR + r] = from_f32<f16>(acc);
     }
   }
@@ -536,6 +562,11 @@ int bwd_typed(const RopeBwdArgs<T>& a, hipStream_t st) {
   return check_launch("rus_qkv_rope_bwd");
 }
 
+// Tokens from which a thread takes two / four: fewer fragment loads per token against fewer blocks.
+// One / two / four tokens: 1,500 tokens 10.4 / 11.6 / 15.8 us, 2,048 13.2 / 13.1 / 17.3, 3,000 19.4 /
+// 17.0 / 20.2, 6,000 34.4 / 29.5 / 29.0, 8,161 45.4 / 39.7 / 36.1.
+constexpr int64_t kMidTokens2 = 2048, kMidTokens4 = 6144;
+
 int bwd_mid(const char* fn, const RopeBwdMidArgs& m, hipStream_t st) {
   const RopeBwdArgs<f16>& a = m.b;
   const int per_head = a.head_dim / 2 / kSpan;
@@ -555,8 +586,13 @@ int bwd_mid(const char* fn, const RopeBwdMidArgs& m, hipStream_t st) {
     return fail(RUS_ERR_UNSUPPORTED, "%s: %d query heads per KV head (at most %d)", fn,
                 a.h_q / a.h_kv, kMaxGroupSum);
   const int64_t tpb = kThreads / slots;
-  const dim3 grid(static_cast<unsigned>((a.n_tokens + tpb - 1) / tpb));
-  hipLaunchKernelGGL(rope_bwd_mid_kernel, grid, dim3(kThreads), 0, st, m);
+  auto grid = [&](int64_t per) { return dim3(static_cast<unsigned>((a.n_tokens + per - 1) / per)); };
+  if (a.n_tokens >= kMidTokens4)
+    hipLaunchKernelGGL((rope_bwd_mid_kernel<4>), grid(tpb * 4), dim3(kThreads), 0, st, m);
+  else if (a.n_tokens >= kMidTokens2)
+    hipLaunchKernelGGL((rope_bwd_mid_kernel<2>), grid(tpb * 2), dim3(kThreads), 0, st, m);
+  else
+    hipLaunchKernelGGL((rope_bwd_mid_kernel<1>), grid(tpb), dim3(kThreads), 0, st, m);
   return check_launch(fn);
 }
 

@@ -463,3 +463,45 @@ def test_lora_down_rows_of_long_batches_equals_short_ones(drop, n, d, r):
     for got, want, xx, aa in zip(whole, (mq, mv), (xq, xv), (aq, av)):
         ok, err = _close(got, want, a=xx, b=aa.t())
         assert ok, err
+
+
+@pytest.mark.parametrize("scale", [1.0, 2.0**-18])
+@pytest.mark.parametrize("n", [5, 2047, 2051, 6149])
+def test_rope_products_of_one_to_four_tokens_per_thread(n, scale):
+    """One, two and four tokens per thread, with and without head partials, down to gradients and
+    mid rows that are subnormal in fp16 (2^-18): packed outputs equal the plain kernel's bit for bit;
+    products against float64 within half an fp16 ulp plus the fp32 sums' bound (at most 16 terms in a
+    lane, then 8 + 8 levels: 2^-19 of the sum of magnitudes)."""
+    hq, hkv, hd, r = 12, 2, 128, 16
+    g = torch.Generator(device=DEV).manual_seed(n)
+
+    def rnd(*shape, std=1.0):
+        return torch.randn(*shape, generator=g, device=DEV) * std
+
+    def check(got, x, b, factor=1.0):
+        x, b = x.double(), b.double()
+        want, mag = x @ b, x.abs() @ b.abs()
+        ulp = ref.fp16_ulp((want.abs() + 2.0**-19 * mag).float().cpu()).to(DEV)
+        err = (got.double() / factor - want).abs()
+        assert bool((err <= 0.5001 * ulp + 2.0**-19 * mag).all()), float((err / ulp).max())
+
+    dq = rnd(n, hq, hd, std=scale).half()
+    parts = [rnd(hq, n, hd, std=scale) for _ in range(2)]
+    dk, dv = (K.sum_splits(p.view(hkv, hq // hkv, n, hd).transpose(0, 1).contiguous()
+                           .view(hq // hkv, hkv * n, hd)).view(hkv, n, hd).transpose(0, 1)
+              .contiguous() for p in parts)
+    ang = rnd(600, hd)
+    rope = (ang.cos().half(), ang.sin().half(), torch.randint(0, 600, (n,), generator=g, device=DEV))
+    bq, bv = rnd(hq * hd, r, std=0.5).half(), rnd(hkv * hd, r, std=0.5).half()
+    want = K.qkv_rope_bwd_lora(dq, dk, dv, *rope, 2.0, 0.5, h_q=hq, h_kv=hkv, head_dim=hd)
+    factors = (bq.t().contiguous(), bv.t().contiguous())
+    for got in (K.qkv_rope_bwd_lora_mid(dq, dk, dv, *rope, 2.0, 0.5, *factors),
+                K.qkv_rope_bwd_lora_mid_parts(dq, *parts, *rope, 2.0, 0.5, *factors)):
+        for a, b in zip(got[:3], want):
+            assert torch.equal(a, b)
+        check(got[3], want[1].view(n, -1), bq)
+        check(got[4], want[2].view(n, -1), bv)
+    mid = rnd(n, r, std=scale).half()  # forward: V + 2 delta with V = 0 is 2 delta exactly
+    qkv = torch.zeros(n, (hq + 2 * hkv) * hd, dtype=torch.float16, device=DEV)
+    v = K.qkv_rope_fwd_mid(qkv, mid, mid, bq, bv, *rope, 2.0, 2.0, hq, hkv, hd)[2]
+    check(v.view(n, -1), mid, bv.t(), factor=2.0)
