@@ -29,12 +29,26 @@ constexpr uint64_t kPhiloxW0 = 0x9E3779B97F4A7C15ull;
 constexpr uint64_t kPhiloxW1 = 0xBB67AE8584CAA73Bull;
 constexpr int kThreads = 256;
 
+// hi, lo of the 128-bit product x * M from four 32 x 32 + 64 multiply-adds (none overflows). The
+// multiplies bound keep_bits_kernel; a product and its high half formed apart took six.
+template <uint64_t M>
+__device__ __forceinline__ void mul128(uint64_t x, uint64_t& hi, uint64_t& lo) {
+  constexpr uint64_t ml = M & 0xffffffffu, mh = M >> 32;
+  const uint64_t xl = x & 0xffffffffu, xh = x >> 32;
+  const uint64_t p0 = xl * ml;
+  const uint64_t p1 = xh * ml + (p0 >> 32);
+  const uint64_t p2 = xl * mh + (p1 & 0xffffffffu);
+  hi = xh * mh + (p1 >> 32) + (p2 >> 32);
+  lo = (p2 << 32) | (p0 & 0xffffffffu);
+}
+
 // Philox4x64 with 10 rounds; returns the four output words in c.
 __device__ __forceinline__ void philox4x64_10(uint64_t (&c)[4], uint64_t k0, uint64_t k1) {
 #pragma unroll
   for (int r = 0; r < 10; ++r) {
-    const uint64_t lo0 = kPhiloxM0 * c[0], hi0 = __umul64hi(kPhiloxM0, c[0]);
-    const uint64_t lo1 = kPhiloxM1 * c[2], hi1 = __umul64hi(kPhiloxM1, c[2]);
+    uint64_t lo0, hi0, lo1, hi1;
+    mul128<kPhiloxM0>(c[0], hi0, lo0);
+    mul128<kPhiloxM1>(c[2], hi1, lo1);
     const uint64_t n0 = hi1 ^ c[1] ^ k0, n2 = hi0 ^ c[3] ^ k1;
     c[0] = n0;
     c[1] = lo1;
