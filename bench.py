@@ -34,7 +34,7 @@ if REPO not in sys.path:
 METRIC = "train tokens/s (packed 1.5B NF4 QLoRA); lm_head-CE & NF4-dequant HBM GB/s"
 HBM_PEAK_GBS = 8000.0  # MI355X HBM3E
 FP16_PEAK_TFLOPS = 2500.0  # MI355X dense fp16 MFMA
-LMHEAD_KERNELS = ("lmhead_ce_fwd", "lmhead_ce_fwd_keep", "lmhead_ce_logits",
+LMHEAD_KERNELS = ("lmhead_ce_fwd", "lmhead_ce_fwd_keep", "lmhead_ce_fwd_probs", "lmhead_ce_logits",
                   "lmhead_ce_grad_logits", "lmhead_ce_grad_hidden")
 # kernels whose roofline is the fp16 MFMA peak (the rest are bound by HBM bandwidth)
 MFMA_KERNELS = LMHEAD_KERNELS + ("gemm_parts", "nf4_gemm", "attn_fwd", "attn_bwd")

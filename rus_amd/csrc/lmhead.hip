@@ -15,11 +15,12 @@
 //     first argmax and rewrites the row in place as G, and lmhead_grad_hidden_kernel forms
 //     G . (W^T)^T split-K over the vocabulary into fp32 partials that dh_reduce_kernel sums;
 //   * single pass over vocabulary chunks (a head streamed from the host, or v_chunk given):
-//     lmhead_stats_kernel<KEEP> keeps per-token online statistics per 256 vocab rows in
-//     registers and the chunk's logits; lmhead_chunk_scale_kernel turns them into
-//     P = e^{z - M} (M the running maximum) and the same split-K GEMM adds P . W_chunk into fp32
-//     partials rescaled when M grows; lmhead_dh_finish_kernel divides by s and subtracts the
-//     label rows.
+//     lmhead_stats_kernel<kProbs> keeps per-token online statistics per 256 vocab rows in
+//     registers and stores P = 2^(z log2 e - K), K a reference per token from the chunks before;
+//     lmhead_probs_rescale_kernel aligns the half tiles whose reference moved and the same split-K
+//     GEMM adds P . W_chunk into fp32 partials rescaled when K grows; lmhead_dh_finish_kernel
+//     divides by s and subtracts the label rows. (kLogits with lmhead_chunk_scale_kernel, the same
+//     from kept logits by the running maximum, serves callers of those entry points.)
 // The GEMMs run the mainloops of mfma_gemm.h: 256 x 256 block tiles on v_mfma_f32_32x32x16_f16
 // filled by direct global -> LDS copies. The logits, statistics and hidden-gradient kernels run
 // eight waves of 128 x 64 (two per SIMD) with K staged 64 deep through two 64 KiB buffers; the

@@ -1972,6 +1972,8 @@ class LMHeadPass:
         c = self.done
         before = self.state[(c + 1) % 2] if c else (None, None)
         after = self.state[c % 2]
+        if c == len(self.chunk_max):  # chunks shorter than announced
+            self.chunk_max.append(torch.zeros_like(self.target))
         lm_head_ce_fwd_chunk(hidden, w_rows, labels, start, self.parts, self.target,
                              probs=(self.z, before[0], self.half_ref, self.chunk_max[c]))
         _launch("lmhead_ce_probs_rescale", 20 * self.n_tok, 0, "rus_lmhead_ce_probs_rescale",

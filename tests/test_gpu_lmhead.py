@@ -376,3 +376,38 @@ def test_lmhead_of_token_tiles_partly_filled(n):
     out = K.lm_head_ce(h.to(DEV), w.to(DEV), lab.to(DEV), num_items_in_batch=64.0,
                        need_grad=False)
     _check_against_oracle(h, w, lab, out, denom=64.0, check_dh=False)
+
+
+@pytest.mark.parametrize("n,v,chunk", [(37, 1216, 256), (300, 1100, 512)])
+def test_pass_over_kept_logits_agrees_with_the_stored_probabilities(n, v, chunk):
+    """The launchers that keep a chunk's logits and scale them by the running maximum, against the
+    single pass: both round P to fp16 once (2^-11 relative), so two gradients differ by at most
+    2^-10 of sum P |w| plus the fp32 sums (doubled: p below comes from unrounded logits)."""
+    g = torch.Generator().manual_seed(v)
+    d = 128
+    h = (torch.randn(n, d, generator=g) * 2).half().to(DEV)
+    w = (torch.randn(v, d, generator=g) * 0.3).half().to(DEV)
+    labels = torch.randint(0, v, (n,), generator=g).to(DEV)
+    want = K.lm_head_ce(h, w, labels, num_items_in_batch=64.0, v_chunk=chunk)
+    wt = K.lm_head_weight_t(w)
+    parts, target = K.LMHeadPartials(K.lm_head_num_parts(v), n, DEV), torch.zeros(n, device=DEV)
+    z = torch.empty(n, K._round_up(chunk, 64), dtype=torch.float16, device=DEV)
+    m_run, alpha = torch.empty(n, device=DEV), torch.empty(n, device=DEV)
+    acc = torch.empty(1, n, d, device=DEV)
+    for c in range(0, v, chunk):
+        rows = w[c:c + chunk]
+        K.lm_head_ce_fwd_chunk(h, rows, labels, c, parts, target, logits_out=z)
+        K.lm_head_ce_chunk_scale(z, rows.shape[0], parts, c // 256, m_run, alpha, c == 0)
+        K.lm_head_ce_grad_hidden_scaled(z, wt[:, c:], rows.shape[0], acc, c > 0, alpha)
+    lse, nll, _, amax = K.lm_head_ce_combine(parts, target, labels)
+    denom = torch.tensor([64.0], device=DEV)
+    dh = K.lm_head_ce_dh_finish(acc, m_run, lse, labels, w, denom, 1.0, None, torch.float32)
+    assert torch.equal(amax, want[3]) and torch.allclose(lse, want[1], rtol=1e-6, atol=1e-5)
+    hp = K.LMHeadPass(n, d, v, v, DEV, True)  # chunks shorter than announced
+    for c in range(0, v, 256):
+        hp.add_chunk(h, w[c:c + 256], wt[:, c:], c, labels)
+    short = hp.finish(labels, 64.0, w)
+    p = torch.softmax(h.double() @ w.double().t(), -1)
+    tol = 1024.0 * (2.0**-9 * (p @ w.double().abs()) + 1e-4)
+    for other in (dh, short[5]):
+        assert bool(((other.double() - want[5].double()).abs() <= tol).all())
