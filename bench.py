@@ -358,8 +358,8 @@ def config_records(seed: int = 0, reps: int = 40) -> dict:
         us = e0.elapsed_time(e1) * 1e3 / 3
         c2.append(_mfma(f"lm_head_ce fwd+bwd (single pass, chunks of {chunk} rows: {what})",
                         [n2, D, V], us, 2 * flops,
-                        note="4*N*D*V over the whole pass (per chunk: statistics GEMM keeping "
-                             "the logits, P = e^{z-M}, hidden-gradient GEMM into rescaled "
+                        note="4*N*D*V over the whole pass (per chunk: statistics GEMM storing "
+                             "P = 2^(z log2 e - K), hidden-gradient GEMM into rescaled "
                              "partials; then combine and finish)"))
     out["2"] = c2
     del h, W, wt, lab
