@@ -186,7 +186,7 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
     int lab_adj = -1000;  // label row local to vrow0, minus 4h (compared with the r/mt part)
     if (tok < g.N) {
       const int64_t l = p.labels[tok] - p.vocab_start - vrow0;
-      lab_adj = (l >= 0 && l < kWM) ? static_cast<int>(l) - 4 * h : -1000;
+      lab_adj = (l >= 0 && l < min(kWM, rows_left)) ? static_cast<int>(l) - 4 * h : -1000;
     }
     float m = -INFINITY, tgt = 0.0f;
     int idx = 0x7fffffff;  // local row minus 4h until the end

@@ -411,3 +411,20 @@ def test_pass_over_kept_logits_agrees_with_the_stored_probabilities(n, v, chunk)
     tol = 1024.0 * (2.0**-9 * (p @ w.double().abs()) + 1e-4)
     for other in (dh, short[5]):
         assert bool(((other.double() - want[5].double()).abs() <= tol).all())
+
+
+def test_labels_past_the_vocabulary_within_its_last_tile():
+    """A label of the last 256-row tile that is no vocabulary row counts as outside the vocabulary
+    (target logit 0, no weight row), whatever lies in the tile's padding."""
+    n, d, v = 70, 128, 700  # rows 700 .. 767 pad the third tile
+    g = torch.Generator().manual_seed(3)
+    h = torch.randn(n, d, generator=g).half().to(DEV)
+    w = (torch.randn(v, d, generator=g) * 0.2).half().to(DEV)
+    labels = torch.randint(0, v, (n,), generator=g).to(DEV)
+    labels[::2] = torch.arange(700, 735, device=DEV)
+    far = torch.where(labels >= v, labels + 1000, labels)
+    for kw in ({"v_chunk": 256}, {"v_chunk": 1024}, {"need_grad": False}, {"block_tokens": 256}):
+        a, b = (K.lm_head_ce(h, w, lab, **kw) for lab in (labels, far))
+        for x, y in zip(a, b):
+            assert (x is None and y is None) or torch.equal(x, y), kw
+        assert torch.equal(a[0][::2], a[1][::2])  # nll = lse - 0
