@@ -23,7 +23,7 @@
 extern "C" {
 #endif
 
-#define RUS_ABI_VERSION 18
+#define RUS_ABI_VERSION 19
 
 #define RUS_DTYPE_F16 0
 #define RUS_DTYPE_F32 1
@@ -633,20 +633,38 @@ int rus_lmhead_ce_grad_hidden_scaled(const void* probs, int64_t ld_p, const void
                                      const float* alpha, void* stream);
 
 /*
- * rus_lmhead_ce_fwd that also stores the chunk's probabilities P[t][v - vocab_start] =
- * fp16(2^(z log2 e - K)) (columns up to round_up(n_vocab, 64), zeros past n_vocab), K a
- * reference per token and 128 vocabulary rows: ref[t] (log2 units, as rus_lmhead_ce_probs_rescale
- * left it; NULL for the first chunk) unless the largest logit there lies more than 15 above it, else
- * a reference of its own, written like the others to half_ref[2 * (r / 256) + (r / 128) % 2][t]
- * (row stride part_stride). chunk_max[t] (0 before the call) receives the chunk's maximum as
- * ordered bits. Replaces: as rus_lmhead_ce_fwd_keep, with the exponentials of the gradient pass.
+ * rus_lmhead_ce_fwd over the rows other than each token's label (whose logit goes to target), that
+ * also stores the chunk's probabilities P[t][v - vocab_start] = fp16(2^(z log2 e - K)) (0 at the
+ * label; columns up to round_up(n_vocab, 64), zeros past n_vocab), K a reference per token and 128
+ * vocabulary rows: ref[t] (log2 units, as rus_lmhead_ce_probs_rescale left it; NULL for the first
+ * chunk) unless the largest logit there lies more than 15 above it, else a reference of its own,
+ * written like the others to half_ref[2 * (r / 256) + (r / 128) % 2][t] (row stride part_stride).
+ * part_r, laid out like part_m: (P - unrounded) / unrounded at the part's largest logit.
+ * chunk_max[t] (0 before the call) receives the chunk's maximum as ordered bits. The label's
+ * gradient cancels to W[y] (p_y - 1), which an fp16 P of the label would leave its rounding in.
+ * Replaces: as rus_lmhead_ce_fwd_keep, with the exponentials of the gradient pass.
  */
 int rus_lmhead_ce_fwd_probs(const void* hidden, const void* weight, const int64_t* labels,
                             int64_t n_tok, int64_t d, int64_t ld_h, int64_t ld_w, int64_t n_vocab,
                             int64_t vocab_start, float* part_m, float* part_s, float* part_w,
-                            int32_t* part_idx, int64_t part_base, int64_t part_stride,
-                            float* target, void* probs, int64_t ld_p, const float* ref,
-                            float* half_ref, uint32_t* chunk_max, void* stream);
+                            int32_t* part_idx, float* part_r, int64_t part_base,
+                            int64_t part_stride, float* target, void* probs, int64_t ld_p,
+                            const float* ref, float* half_ref, uint32_t* chunk_max, void* stream);
+
+/*
+ * rus_lmhead_ce_combine over the partials of rus_lmhead_ce_fwd_probs: the label joins by its logit
+ * where it indexes the vocabulary of n_vocab rows (lse, nll, entropy and argmax as
+ * rus_lmhead_ce_combine gives them), and for rus_lmhead_ce_dh_finish_probs: rest[t] = 1 - p_y, as
+ * the sum over the other rows; top[t] the row of the largest probability beside the label's, and
+ * fix[t] that probability times its relative rounding in P (0 where it is below 1/16).
+ * Replaces: as rus_lmhead_ce_combine.
+ */
+int rus_lmhead_ce_combine_probs(const float* part_m, const float* part_s, const float* part_w,
+                                const int32_t* part_idx, const float* part_r, int64_t n_parts,
+                                int64_t part_stride, const float* target, const int64_t* labels,
+                                int64_t n_tok, int64_t n_vocab, float* lse, float* nll,
+                                float* entropy, int64_t* argmax, float* rest, float* fix,
+                                int32_t* top, void* stream);
 
 /*
  * Between rus_lmhead_ce_fwd_probs and rus_lmhead_ce_grad_hidden_scaled of one chunk: brings a
@@ -654,7 +672,7 @@ int rus_lmhead_ce_fwd_probs(const void* hidden, const void* weight, const int64_
  * (all n_tok floats; ref_in / run_in NULL for the first chunk, else the outputs of the chunk before,
  * in buffers of their own): run_out = this chunk's reference, alpha = 2^(run_in - run_out) (0 at
  * first), ref_out = the reference for the next chunk, m_run = run_out in natural log (for
- * rus_lmhead_ce_dh_finish). Replaces: as rus_lmhead_ce_chunk_scale.
+ * rus_lmhead_ce_dh_finish_probs). Replaces: as rus_lmhead_ce_chunk_scale.
  */
 int rus_lmhead_ce_probs_rescale(void* probs, int64_t ld_p, int64_t n_tok, int64_t n_vocab,
                                 const float* half_ref, int64_t half_stride,
@@ -691,6 +709,19 @@ int rus_lmhead_ce_dh_finish(const float* parts, int32_t n_parts, int64_t n_tok, 
                             const void* w_rows, int64_t ld_w, int64_t n_vocab, int32_t w_on_host,
                             const float* denom, float scale, const float* scale_dev, void* out,
                             int32_t out_dtype, void* stream);
+
+/*
+ * rus_lmhead_ce_dh_finish for partials of P without the label (rus_lmhead_ce_fwd_probs):
+ *   out[t][c] = (sum_s parts[s][t][c] * e^{M_run[t] - lse[t]} - rest[t] W[y_t][c]
+ *                - fix[t] W[top[t]][c]) * 2^16 / denom * scale (* *scale_dev when given)
+ * with rest, fix and top of rus_lmhead_ce_combine_probs. Replaces: as rus_lmhead_ce_dh_finish.
+ */
+int rus_lmhead_ce_dh_finish_probs(const float* parts, int32_t n_parts, int64_t n_tok, int64_t d,
+                                  const float* m_run, const float* lse, const int64_t* labels,
+                                  const void* w_rows, int64_t ld_w, int64_t n_vocab,
+                                  int32_t w_on_host, const float* denom, float scale,
+                                  const float* scale_dev, const float* rest, const float* fix,
+                                  const int32_t* top, void* out, int32_t out_dtype, void* stream);
 
 /*
  * out[i] = T(scale * (*scale_dev) * sum_p parts[p * n_elem + i]), T = out_dtype (fp16 or fp32);

@@ -11,7 +11,7 @@ import threading
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "librus_amd.so"
-ABI_VERSION = 18
+ABI_VERSION = 19
 
 DTYPE_F16 = 0
 DTYPE_F32 = 1
@@ -139,11 +139,15 @@ SIGNATURES: dict[str, list] = {
                                          _vp, _vp],
     "rus_lmhead_ce_chunk_scale": [_vp, _i64, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _i32, _vp],
     "rus_lmhead_ce_fwd_probs": [_vp, _vp, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp, _vp, _vp,
-                                _vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp],
+                                _vp, _vp, _i64, _i64, _vp, _vp, _i64, _vp, _vp, _vp, _vp],
+    "rus_lmhead_ce_combine_probs": [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp, _vp, _i64, _i64, _vp,
+                                    _vp, _vp, _vp, _vp, _vp, _vp, _vp],
     "rus_lmhead_ce_probs_rescale": [_vp, _i64, _i64, _i64, _vp, _i64, _vp, _vp, _vp, _vp, _vp, _vp,
                                     _vp, _vp],
     "rus_lmhead_ce_dh_finish": [_vp, _i32, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i32, _vp,
                                 _f32, _vp, _vp, _i32, _vp],
+    "rus_lmhead_ce_dh_finish_probs": [_vp, _i32, _i64, _i64, _vp, _vp, _vp, _vp, _i64, _i64, _i32,
+                                      _vp, _f32, _vp, _vp, _vp, _vp, _vp, _i32, _vp],
 }
 
 _lock = threading.Lock()

@@ -16,11 +16,13 @@
 //     G . (W^T)^T split-K over the vocabulary into fp32 partials that dh_reduce_kernel sums;
 //   * single pass over vocabulary chunks (a head streamed from the host, or v_chunk given):
 //     lmhead_stats_kernel<kProbs> keeps per-token online statistics per 256 vocab rows in
-//     registers and stores P = 2^(z log2 e - K), K a reference per token from the chunks before;
+//     registers and stores P = 2^(z log2 e - K), K a reference per token from the chunks before,
+//     and 0 for the label, whose term would cancel against -W[y] (see kProbs);
 //     lmhead_probs_rescale_kernel aligns the half tiles whose reference moved and the same split-K
-//     GEMM adds P . W_chunk into fp32 partials rescaled when K grows; lmhead_dh_finish_kernel
-//     divides by s and subtracts the label rows. (kLogits with lmhead_chunk_scale_kernel, the same
-//     from kept logits by the running maximum, serves callers of those entry points.)
+//     GEMM adds P . W_chunk into fp32 partials rescaled when K grows; lmhead_combine_kernel adds the
+//     label to the statistics and lmhead_dh_finish_kernel divides by s and subtracts
+//     (1 - p_label) W[y]. (kLogits with lmhead_chunk_scale_kernel, which keeps the label in P and
+//     takes the running maximum as the reference, serves callers of those entry points.)
 // The GEMMs run the mainloops of mfma_gemm.h: 256 x 256 block tiles on v_mfma_f32_32x32x16_f16
 // filled by direct global -> LDS copies. The logits, statistics and hidden-gradient kernels run
 // eight waves of 128 x 64 (two per SIMD) with K staged 64 deep through two 64 KiB buffers; the
@@ -116,6 +118,7 @@ struct StatsParams {
   int64_t ld_z;
   int kpad;
   // kProbs: P = 2^(z log2 e - K), with a reference K per token and 128 vocabulary rows
+  float* part_r;        // [parts][part_stride] relative rounding of the part's largest P
   const float* ref;     // [n_tok] reference from the chunks before (nullptr: the first chunk)
   float* half_ref;      // [2 * parts of the chunk][part_stride]: the K each half tile used
   uint32_t* chunk_max;  // [n_tok] ordered bits of the chunk's maximum (0 before the launch)
@@ -125,20 +128,31 @@ struct StatsParams {
 // kLogits a kernel between the two GEMMs of a chunk read and rewrote all its logits (43 us per
 // [2048, 32768] chunk, memory-bound, 9 us at 100 tokens); probabilities written once need a launch
 // that only looks at the references (5 us). 2048 tokens x 151936: 2571 -> 2372 us, 345: 770 -> 725.
+//
+// With kProbs the statistics and P leave out the token's label: dH = sum_(v != y) p_v W_v -
+// (1 - p_y) W_y with 1 - p_y = sum_(v != y) p_v, formed from the sums without the label, whereas
+// p_y in the fp16 product leaves its rounding (2^-12 of W_y) where 1 - p_y may be far smaller. The
+// references follow the other logits for the same reason: against the label's, P would sink below
+// fp16's range. dH of 300 tokens x 8322 rows against float64, 2-norm relative, with the label in P /
+// in P against the running maximum (the label exact, its neighbours not) / left out: mean nll 0.12
+// 1.5e-3 / 7.6e-6 / 2.6e-6, 1.4e-3 0.13 / 7.2e-4 / 2.6e-6, 1.5e-5 9.1 / 3.4e-2 / 3.7e-6; another row
+// at p 0.999 1.9e-4 / 1.1e-6 / 6.4e-7. 2048 tokens x 151936: 2269 us with it, 2266 without.
 enum StatsOut { kNone = 0, kLogits = 1, kProbs = 2 };
 
 // A token's reference stays the one it came with unless a half tile's largest logit lies more than
 // kRefWindow (log2 units) above it; P is at most 2^15 in fp16. A half tile past the window (every
 // one of the first chunk) takes its own, a multiple of kRefStep not above its maximum, so that the
 // half tiles of a token mostly agree (P < 2^kRefStep) and none needs rescaling. Either way the
-// largest P is at least 2^-1/2: fp16 resolves every probability as well as it would against the
-// maximum (dH against float64 at 707 tokens: 1.29e-6 relative either way). The offset is free: it only
-// moves where P's roundings fall (with 0 one gradient of the 28-layer comparison with the oracle,
-// within 1% of it by a hair, lands at 1.003%).
-constexpr float kRefWindow = 15.0f, kRefStep = 8.0f, kRefOffset = 0.5f;
+// largest P of all is at least 1: fp16 resolves every smaller probability as well as it would
+// against the maximum. The largest itself would be exact there and is not here, so its relative
+// rounding (part_r) goes to the finishing kernel, which takes it back where that probability counts.
+constexpr float kRefWindow = 15.0f, kRefStep = 8.0f;
+
+// In the label's place: below every fp16 logit, finite (0 * -inf in the entropy's sum is no number).
+constexpr float kNoLogit = -1e30f;
 
 __device__ __forceinline__ float own_ref(float y) {
-  return kRefStep * floorf(y / kRefStep) + kRefOffset;
+  return kRefStep * floorf(y / kRefStep);
 }
 
 // fp32 -> uint32 in the same order (NaN aside); 0 is below every value.
@@ -166,7 +180,7 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
   const int h = lane >> 5;
   const int vrow0 = tl.m0 + wm * kWM;  // local vocab row of this wave's first accumulator row
   const bool full = tl.m0 + kBM <= g.M;
-  float rm[NT], rs[NT], rw[NT];
+  float rm[NT], rs[NT], rw[NT], rr[NT];
   int ri[NT];
   // Logits as the reference's fp16 GEMM output: rounded once, in place.
 #pragma unroll
@@ -183,15 +197,27 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
 #pragma unroll
   for (int nt = 0; nt < NT; ++nt) {
     const int tok = tl.n0 + wn * RW + nt * 32 + (lane & 31);
-    int lab_adj = -1000;  // label row local to vrow0, minus 4h (compared with the r/mt part)
+    int lab = -1;  // label row local to vrow0, where this lane holds it
     if (tok < g.N) {
       const int64_t l = p.labels[tok] - p.vocab_start - vrow0;
-      lab_adj = (l >= 0 && l < min(kWM, rows_left)) ? static_cast<int>(l) - 4 * h : -1000;
+      if (l >= 0 && l < min(kWM, rows_left) && (l >> 2 & 1) == h) lab = static_cast<int>(l);
     }
-    float m = -INFINITY, tgt = 0.0f;
+    float m = -INFINITY;
     int idx = 0x7fffffff;  // local row minus 4h until the end
-    rm[nt] = m, rs[nt] = rw[nt] = 0.0f, ri[nt] = idx;
+    rm[nt] = m, rs[nt] = rw[nt] = rr[nt] = 0.0f, ri[nt] = idx;
     if (tl.n0 + wn * RW + nt * 32 >= g.N) continue;  // no token here
+    if (__ballot(lab >= 0)) {  // one wave in forty at 151936 rows: 32 tokens x 128 rows
+      float tgt = 0.0f;
+#pragma unroll
+      for (int mt = 0; mt < kMT; ++mt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const bool hit = lab == mt * 32 + 8 * (r >> 2) + (r & 3) + 4 * h;
+          tgt = hit ? acc[mt][nt][r] : tgt;
+          if constexpr (OUT == kProbs) acc[mt][nt][r] = hit ? kNoLogit : acc[mt][nt][r];
+        }
+      if (lab >= 0) p.target[tok] = tgt;  // one lane of one block
+    }
     if (full) {
 #pragma unroll
       for (int mt = 0; mt < kMT; ++mt)
@@ -201,7 +227,6 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
           const float z = acc[mt][nt][r];
           idx = z > m ? rl : idx;  // rows ascend: strict > keeps the first index
           m = fmaxf(m, z);
-          tgt = rl == lab_adj ? z : tgt;
         }
     } else {
 #pragma unroll
@@ -214,8 +239,13 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
             m = z;
             idx = rl;
           }
-          tgt = rl == lab_adj ? z : tgt;
         }
+    }
+    if constexpr (OUT == kProbs) {
+      if (m == kNoLogit) {  // the label alone
+        m = -INFINITY;
+        idx = 0x7fffffff;
+      }
     }
     idx = idx == 0x7fffffff ? idx : vrow0 + idx + 4 * h;
     // The lane pair (l, l^32) holds the two interleaved halves of the wave's 128 rows.
@@ -234,6 +264,8 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
       if (!(m > -INFINITY)) ref = given > -INFINITY ? given : 0.0f;  // no finite logit here
       if (h == 0 && tok < g.N)
         p.half_ref[static_cast<int64_t>(2 * (tl.m0 / kBM) + wm) * p.part_stride + tok] = ref;
+      const float top = exp2_fast(__builtin_fmaf(m, kLog2e, -ref));  // the largest P, as below
+      if (top >= 0x1p-14f) rr[nt] = (static_cast<float>(from_f32<f16>(top)) - top) / top;
     }
     if (OUT == kProbs || m > -INFINITY) {
       mb = ref;
@@ -279,8 +311,6 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
     rs[nt] = s;
     rw[nt] = w;
     ri[nt] = idx;
-    // The label's row lives in exactly one lane of one block: that lane writes the target.
-    if (lab_adj + 4 * h >= 0 && ((lab_adj + 4 * h) >> 2 & 1) == h) p.target[tok] = tgt;
   }
 
   if constexpr (OUT == kProbs)
@@ -289,7 +319,7 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
 
   // Merge the two vocab halves (wm = 0, 1) of the block through LDS; wm = 0 writes the partial.
   if constexpr (OUT != kNone) __syncthreads();  // the stored tile's staging reads of the LDS are done
-  float* xm = reinterpret_cast<float*>(smem);  // [token column of the tile] x (m, s, w, idx)
+  float* xm = reinterpret_cast<float*>(smem);  // [token column of the tile] x (m, s, w, idx, r)
   if (wm == 1 && h == 0) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt) {
@@ -298,6 +328,7 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
       xm[kBN + o] = rs[nt];
       xm[2 * kBN + o] = rw[nt];
       reinterpret_cast<int*>(xm)[3 * kBN + o] = ri[nt];
+      if constexpr (OUT == kProbs) xm[4 * kBN + o] = rr[nt];
     }
   }
   __syncthreads();
@@ -317,15 +348,21 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
         s = s * ca + sB * cb;
         w = w * ca + wB * cb;
       }
-      if (mB > m) idx = iB;  // the second half's rows all follow the first half's
+      if (mB > m) {  // the second half's rows all follow the first half's
+        idx = iB;
+        if constexpr (OUT == kProbs) rr[nt] = xm[4 * kBN + o];
+      }
       m = M;
-      if (tok < g.N && idx != 0x7fffffff) {
+      if (tok < g.N) {  // also where no logit is above -inf: (-inf, 0, 0)
         const int64_t o2 = static_cast<int64_t>(part) * p.part_stride + tok;
         p.part_m[o2] = m;
         p.part_s[o2] = s;
         p.part_w[o2] = w;
-        p.part_idx[o2] = idx + p.vocab_start;
-        if constexpr (OUT == kProbs) atomicMax(p.chunk_max + tok, ordered_bits(m));
+        p.part_idx[o2] = idx == 0x7fffffff ? idx : idx + p.vocab_start;
+        if constexpr (OUT == kProbs) {
+          p.part_r[o2] = rr[nt];
+          atomicMax(p.chunk_max + tok, ordered_bits(m));
+        }
       }
     }
   }
@@ -598,14 +635,17 @@ __global__ __launch_bounds__(kZgThreads) void lmhead_probs_rescale_kernel(
 // dH (times 2^16 / denom, times scale) from the online accumulation:
 //   out[t][c] = (sum_s parts[s][t][c] * e^{M[t] - lse[t]} - W[y_t][c]) * 2^16 / denom * scale
 // for labelled tokens (y_t != -100; the W row term only when y_t indexes the vocabulary), 0 for
-// the others. w_rows may be device memory or device-mapped pinned host memory. Four columns per
-// thread.
-template <typename T>
+// the others. PROBS (partials without the label, from rus_lmhead_ce_fwd_probs): W[y_t][c] times
+// rest[t] = 1 - p_y, and less the rounding of the largest other probability, fix[t] W[top[t]][c]
+// where fix[t] is not 0. w_rows may be device memory or device-mapped pinned host memory. Four
+// columns per thread.
+template <typename T, bool PROBS>
 __global__ __launch_bounds__(256) void lmhead_dh_finish_kernel(
     const float* __restrict__ parts, int n_parts, int n_tok, int d, const float* __restrict__ m_run,
     const float* __restrict__ lse, const int64_t* __restrict__ labels,
     const f16* __restrict__ w_rows, int64_t ld_w, int64_t n_vocab, const float* __restrict__ denom,
-    float scale_h, const float* __restrict__ scale_d, T* __restrict__ out) {
+    float scale_h, const float* __restrict__ scale_d, const float* __restrict__ rest,
+    const float* __restrict__ fix, const int32_t* __restrict__ top, T* __restrict__ out) {
   const int64_t n = static_cast<int64_t>(n_tok) * d;
   const int64_t i = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
   if (i >= n) return;
@@ -620,8 +660,17 @@ __global__ __launch_bounds__(256) void lmhead_dh_finish_kernel(
     if (scale_d) scale *= *scale_d;
     float wy[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (y >= 0 && y < n_vocab) load_f32<f16, 4>(w_rows + y * ld_w + c, wy);
+    if constexpr (PROBS) {
+      float wt[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+      const float r = rest[t], x = fix[t];
+      const int64_t v = top[t];
+      if (x != 0.0f && v >= 0 && v < n_vocab) load_f32<f16, 4>(w_rows + v * ld_w + c, wt);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) o[e] = (a[e] * f - wy[e]) * scale;
+      for (int e = 0; e < 4; ++e) o[e] = (a[e] * f - r * wy[e] - x * wt[e]) * scale;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[e] = (a[e] * f - wy[e]) * scale;
+    }
   }
   store_from_f32<T, 4>(out + i, o);
 }
@@ -786,39 +835,57 @@ __global__ __launch_bounds__(kRowThreads) void lmhead_rows_kernel(
 constexpr int kCombTok = 16, kCombSub = 64, kCombDepth = 8;
 
 struct Stat {
-  float m, s, w;
+  float m, s, w, r;
   int i;
 };
 
-__device__ __forceinline__ void merge_stat(Stat& a, float m, float s, float w, int i) {
+__device__ __forceinline__ void merge_stat(Stat& a, float m, float s, float w, float r, int i) {
   if (m > a.m) {
     const float c = exp2_fast((a.m - m) * kLog2e);
     a.s = a.s * c + s;
     a.w = a.w * c + w;
     a.m = m;
+    a.r = r;
     a.i = i;
   } else if (m > -INFINITY) {
     const float c = exp2_fast((m - a.m) * kLog2e);
     a.s += s * c;
     a.w += w * c;
-    if (m == a.m && i < a.i) a.i = i;
+    if (m == a.m && i < a.i) {
+      a.r = r;
+      a.i = i;
+    }
   }
 }
 
+// PROBS: the partials leave out the token's label (kProbs), which joins here by its logit, and dh
+// gets what the finishing kernel needs of it. A largest other probability below kFixMin is not
+// worth its weight row: its rounding is 2^-12 of that at most, as every other probability's is.
+constexpr float kFixMin = 0x1p-4f;
+
+struct CombineDh {
+  const float* part_r;
+  int64_t n_vocab;
+  float* rest;   // 1 - p_y
+  float* fix;    // p of the largest probability beside the label's times its rounding in P, or 0
+  int32_t* top;  // and its vocabulary row
+};
+
+template <bool PROBS>
 __global__ __launch_bounds__(kCombTok * kCombSub) void lmhead_combine_kernel(
     const float* __restrict__ pm, const float* __restrict__ ps, const float* __restrict__ pw,
     const int32_t* __restrict__ pi, int n_parts, int64_t stride, const float* __restrict__ target,
     const int64_t* __restrict__ labels, int n_tok, float* __restrict__ lse,
-    float* __restrict__ nll, float* __restrict__ ent, int64_t* __restrict__ amax) {
+    float* __restrict__ nll, float* __restrict__ ent, int64_t* __restrict__ amax, CombineDh dh) {
   __shared__ Stat part[kCombSub][kCombTok + 1];
   const int col = threadIdx.x % kCombTok, sub = threadIdx.x / kCombTok;
   const int tok = blockIdx.x * kCombTok + col;
-  Stat st{-INFINITY, 0.0f, 0.0f, 0x7fffffff};
+  Stat st{-INFINITY, 0.0f, 0.0f, 0.0f, 0x7fffffff};
   const int per = (n_parts + kCombSub - 1) / kCombSub;
   const int q0 = sub * per, q1 = min(q0 + per, n_parts);
   if (tok < n_tok) {
     for (int q = q0; q < q1; q += kCombDepth) {
-      float m[kCombDepth], s[kCombDepth], w[kCombDepth];
+      float m[kCombDepth], s[kCombDepth], w[kCombDepth], r[kCombDepth];
       int ix[kCombDepth];
 #pragma unroll
       for (int j = 0; j < kCombDepth; ++j) {
@@ -827,32 +894,54 @@ __global__ __launch_bounds__(kCombTok * kCombSub) void lmhead_combine_kernel(
         s[j] = ps[o];
         w[j] = pw[o];
         ix[j] = pi[o];
+        r[j] = PROBS ? dh.part_r[o] : 0.0f;
       }
 #pragma unroll
       for (int j = 0; j < kCombDepth; ++j)
-        if (q + j < q1) merge_stat(st, m[j], s[j], w[j], ix[j]);
+        if (q + j < q1) merge_stat(st, m[j], s[j], w[j], r[j], ix[j]);
     }
   }
   part[sub][col] = st;
   __syncthreads();
   for (int width = kCombSub / 8; width >= 1; width /= 8) {  // 64 -> 8 -> 1
-    Stat t{-INFINITY, 0.0f, 0.0f, 0x7fffffff};
+    Stat t{-INFINITY, 0.0f, 0.0f, 0.0f, 0x7fffffff};
     if (sub < width)
       for (int k = 0; k < 8; ++k) {
         const Stat a = part[8 * sub + k][col];
-        merge_stat(t, a.m, a.s, a.w, a.i);
+        merge_stat(t, a.m, a.s, a.w, a.r, a.i);
       }
     __syncthreads();
     if (sub < width) part[sub][col] = t;
     __syncthreads();
   }
   if (sub != 0 || tok >= n_tok) return;
-  const Stat t = part[0][col];
+  Stat t = part[0][col];
+  const int64_t y = labels[tok];
+  const float z = target[tok];
+  float others = t.s;  // the sum without the label, on the final maximum
+  const float m_others = t.m;
+  if constexpr (PROBS) {
+    dh.top[tok] = t.i;
+    if (y >= 0 && y < dh.n_vocab) {
+      const float M = fmaxf(t.m, z);
+      const float c = exp2_fast((t.m - M) * kLog2e), e = exp2_fast((z - M) * kLog2e);
+      others = t.s * c;
+      t.s = others + e;
+      t.w = t.w * c + e * z;
+      if (z > t.m || (z == t.m && y < t.i)) t.i = static_cast<int>(y);
+      t.m = M;
+    }
+  }
   const float L = t.m + logf(t.s);
   lse[tok] = L;
   ent[tok] = L - t.w / t.s;
-  nll[tok] = labels[tok] != -100 ? L - target[tok] : 0.0f;
+  nll[tok] = y != -100 ? L - z : 0.0f;
   amax[tok] = t.i;
+  if constexpr (PROBS) {
+    const float p_top = exp2_fast((m_others - L) * kLog2e);
+    dh.rest[tok] = others / t.s;
+    dh.fix[tok] = p_top >= kFixMin ? p_top * t.r : 0.0f;
+  }
 }
 
 // out[i] = T( scale * sum_p parts[p][i] ), four elements per thread (16-byte accesses when every
@@ -919,8 +1008,8 @@ static int lmhead_fwd(const char* fn, const void* hidden, const void* weight,
                       int64_t n_vocab, int64_t vocab_start, float* part_m, float* part_s,
                       float* part_w, int32_t* part_idx, int64_t part_base, int64_t part_stride,
                       float* target, void* logits, int64_t ld_z, void* stream,
-                      bool probs = false, const float* ref = nullptr, float* half_ref = nullptr,
-                      uint32_t* chunk_max = nullptr) {
+                      float* part_r = nullptr, const float* ref = nullptr,
+                      float* half_ref = nullptr, uint32_t* chunk_max = nullptr) {
   if (n_tok < 0 || n_tok >= (1 << 30) || n_vocab < 0 || n_vocab >= (1 << 30) || d <= 0 ||
       d % kBK || vocab_start < 0 || vocab_start + n_vocab >= (int64_t(1) << 31))
     return fail(RUS_ERR_INVALID,
@@ -954,8 +1043,9 @@ static int lmhead_fwd(const char* fn, const void* hidden, const void* weight,
   StatsParams p{labels,      part_m,      part_s, part_w,  part_idx,
                 target,      part_stride, static_cast<int>(part_base),
                 static_cast<int>(vocab_start), static_cast<f16*>(logits), ld_z,
-                static_cast<int>((n_vocab + kBK - 1) / kBK * kBK), ref, half_ref, chunk_max};
-  if (probs)
+                static_cast<int>((n_vocab + kBK - 1) / kBK * kBK), part_r, ref, half_ref,
+                chunk_max};
+  if (part_r)
     hipLaunchKernelGGL(lmhead_stats_kernel<kProbs>, dim3(launch_grid(g)), dim3(kThreads8), 0,
                        static_cast<hipStream_t>(stream), g, p);
   else if (logits)
@@ -996,17 +1086,17 @@ extern "C" int rus_lmhead_ce_fwd_probs(const void* hidden, const void* weight,
                                        const int64_t* labels, int64_t n_tok, int64_t d,
                                        int64_t ld_h, int64_t ld_w, int64_t n_vocab,
                                        int64_t vocab_start, float* part_m, float* part_s,
-                                       float* part_w, int32_t* part_idx, int64_t part_base,
-                                       int64_t part_stride, float* target, void* probs,
-                                       int64_t ld_p, const float* ref, float* half_ref,
-                                       uint32_t* chunk_max, void* stream) {
+                                       float* part_w, int32_t* part_idx, float* part_r,
+                                       int64_t part_base, int64_t part_stride, float* target,
+                                       void* probs, int64_t ld_p, const float* ref,
+                                       float* half_ref, uint32_t* chunk_max, void* stream) {
   const char* fn = "rus_lmhead_ce_fwd_probs";
-  if (n_tok > 0 && n_vocab > 0 && (!probs || !half_ref || !chunk_max || !aligned(half_ref, 4) ||
-                                   !aligned(chunk_max, 4)))
+  if (n_tok > 0 && n_vocab > 0 && (!probs || !part_r || !half_ref || !chunk_max ||
+                                   !aligned(half_ref, 4) || !aligned(chunk_max, 4)))
     return fail(RUS_ERR_INVALID, "%s: null or misaligned buffer", fn);
   return lmhead_fwd(fn, hidden, weight, labels, n_tok, d, ld_h, ld_w, n_vocab, vocab_start,
                     part_m, part_s, part_w, part_idx, part_base, part_stride, target, probs,
-                    ld_p, stream, true, ref, half_ref, chunk_max);
+                    ld_p, stream, part_r, ref, half_ref, chunk_max);
 }
 
 extern "C" int rus_lmhead_ce_grad_from_logits(void* logits_grad, int64_t ld_g,
@@ -1035,12 +1125,12 @@ extern "C" int rus_lmhead_ce_grad_from_logits(void* logits_grad, int64_t ld_g,
   return check_launch(fn);
 }
 
-extern "C" int rus_lmhead_ce_combine(const float* part_m, const float* part_s, const float* part_w,
-                                     const int32_t* part_idx, int64_t n_parts,
-                                     int64_t part_stride, const float* target,
-                                     const int64_t* labels, int64_t n_tok, float* lse,
-                                     float* nll, float* entropy, int64_t* argmax, void* stream) {
-  const char* fn = "rus_lmhead_ce_combine";
+template <bool PROBS>
+static int lmhead_combine(const char* fn, const float* part_m, const float* part_s,
+                          const float* part_w, const int32_t* part_idx, int64_t n_parts,
+                          int64_t part_stride, const float* target, const int64_t* labels,
+                          int64_t n_tok, float* lse, float* nll, float* entropy, int64_t* argmax,
+                          const CombineDh& dh, void* stream) {
   if (n_tok < 0 || n_tok >= (1 << 30) || n_parts <= 0 || n_parts >= (1 << 30) ||
       part_stride < n_tok)
     return fail(RUS_ERR_INVALID, "%s: bad sizes", fn);
@@ -1049,11 +1139,37 @@ extern "C" int rus_lmhead_ce_combine(const float* part_m, const float* part_s, c
       !entropy || !argmax)
     return fail(RUS_ERR_INVALID, "%s: null pointer argument", fn);
   const dim3 grid(static_cast<unsigned>((n_tok + kCombTok - 1) / kCombTok));
-  hipLaunchKernelGGL(lmhead_combine_kernel, grid, dim3(kCombTok * kCombSub), 0,
+  hipLaunchKernelGGL(lmhead_combine_kernel<PROBS>, grid, dim3(kCombTok * kCombSub), 0,
                      static_cast<hipStream_t>(stream), part_m, part_s, part_w, part_idx,
                      static_cast<int>(n_parts), part_stride, target, labels,
-                     static_cast<int>(n_tok), lse, nll, entropy, argmax);
+                     static_cast<int>(n_tok), lse, nll, entropy, argmax, dh);
   return check_launch(fn);
+}
+
+extern "C" int rus_lmhead_ce_combine(const float* part_m, const float* part_s, const float* part_w,
+                                     const int32_t* part_idx, int64_t n_parts,
+                                     int64_t part_stride, const float* target,
+                                     const int64_t* labels, int64_t n_tok, float* lse,
+                                     float* nll, float* entropy, int64_t* argmax, void* stream) {
+  return lmhead_combine<false>("rus_lmhead_ce_combine", part_m, part_s, part_w, part_idx, n_parts,
+                               part_stride, target, labels, n_tok, lse, nll, entropy, argmax,
+                               CombineDh{}, stream);
+}
+
+extern "C" int rus_lmhead_ce_combine_probs(const float* part_m, const float* part_s,
+                                           const float* part_w, const int32_t* part_idx,
+                                           const float* part_r, int64_t n_parts,
+                                           int64_t part_stride, const float* target,
+                                           const int64_t* labels, int64_t n_tok, int64_t n_vocab,
+                                           float* lse, float* nll, float* entropy, int64_t* argmax,
+                                           float* rest, float* fix, int32_t* top, void* stream) {
+  const char* fn = "rus_lmhead_ce_combine_probs";
+  if (n_vocab < 0 || n_vocab >= (int64_t(1) << 31)) return fail(RUS_ERR_INVALID, "%s: bad sizes", fn);
+  if (n_tok > 0 && (!part_r || !rest || !fix || !top))
+    return fail(RUS_ERR_INVALID, "%s: null pointer argument", fn);
+  return lmhead_combine<true>(fn, part_m, part_s, part_w, part_idx, n_parts, part_stride, target,
+                              labels, n_tok, lse, nll, entropy, argmax,
+                              CombineDh{part_r, n_vocab, rest, fix, top}, stream);
 }
 
 namespace rus {
@@ -1263,13 +1379,13 @@ extern "C" int rus_lmhead_ce_probs_rescale(void* probs, int64_t ld_p, int64_t n_
   return check_launch(fn);
 }
 
-extern "C" int rus_lmhead_ce_dh_finish(const float* parts, int32_t n_parts, int64_t n_tok,
-                                       int64_t d, const float* m_run, const float* lse,
-                                       const int64_t* labels, const void* w_rows, int64_t ld_w,
-                                       int64_t n_vocab, int32_t w_on_host, const float* denom,
-                                       float scale, const float* scale_dev, void* out,
-                                       int32_t out_dtype, void* stream) {
-  const char* fn = "rus_lmhead_ce_dh_finish";
+template <bool PROBS>
+static int lmhead_dh_finish(const char* fn, const float* parts, int32_t n_parts, int64_t n_tok,
+                            int64_t d, const float* m_run, const float* lse, const int64_t* labels,
+                            const void* w_rows, int64_t ld_w, int64_t n_vocab, int32_t w_on_host,
+                            const float* denom, float scale, const float* scale_dev,
+                            const float* rest, const float* fix, const int32_t* top, void* out,
+                            int32_t out_dtype, void* stream) {
   if (n_parts <= 0 || n_tok < 0 || n_tok >= (1 << 30) || d <= 0 || d % 4 || d >= (1 << 30) ||
       n_vocab < 0 || ld_w < d || (out_dtype != RUS_DTYPE_F16 && out_dtype != RUS_DTYPE_F32))
     return fail(RUS_ERR_INVALID, "%s: bad arguments (d must be a multiple of 4)", fn);
@@ -1290,16 +1406,43 @@ extern "C" int rus_lmhead_ce_dh_finish(const float* parts, int32_t n_parts, int6
   const dim3 grid(static_cast<unsigned>((n / 4 + 255) / 256));
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (out_dtype == RUS_DTYPE_F16)
-    hipLaunchKernelGGL(lmhead_dh_finish_kernel<f16>, grid, dim3(256), 0, st, parts, n_parts,
+    hipLaunchKernelGGL((lmhead_dh_finish_kernel<f16, PROBS>), grid, dim3(256), 0, st, parts, n_parts,
                        static_cast<int>(n_tok), static_cast<int>(d), m_run, lse, labels,
-                       static_cast<const f16*>(w), ld_w, n_vocab, denom, scale, scale_dev,
-                       static_cast<f16*>(out));
+                       static_cast<const f16*>(w), ld_w, n_vocab, denom, scale, scale_dev, rest,
+                       fix, top, static_cast<f16*>(out));
   else
-    hipLaunchKernelGGL(lmhead_dh_finish_kernel<float>, grid, dim3(256), 0, st, parts, n_parts,
+    hipLaunchKernelGGL((lmhead_dh_finish_kernel<float, PROBS>), grid, dim3(256), 0, st, parts, n_parts,
                        static_cast<int>(n_tok), static_cast<int>(d), m_run, lse, labels,
-                       static_cast<const f16*>(w), ld_w, n_vocab, denom, scale, scale_dev,
-                       static_cast<float*>(out));
+                       static_cast<const f16*>(w), ld_w, n_vocab, denom, scale, scale_dev, rest,
+                       fix, top, static_cast<float*>(out));
   return check_launch(fn);
+}
+
+extern "C" int rus_lmhead_ce_dh_finish(const float* parts, int32_t n_parts, int64_t n_tok,
+                                       int64_t d, const float* m_run, const float* lse,
+                                       const int64_t* labels, const void* w_rows, int64_t ld_w,
+                                       int64_t n_vocab, int32_t w_on_host, const float* denom,
+                                       float scale, const float* scale_dev, void* out,
+                                       int32_t out_dtype, void* stream) {
+  return lmhead_dh_finish<false>("rus_lmhead_ce_dh_finish", parts, n_parts, n_tok, d, m_run, lse,
+                                 labels, w_rows, ld_w, n_vocab, w_on_host, denom, scale, scale_dev,
+                                 nullptr, nullptr, nullptr, out, out_dtype, stream);
+}
+
+extern "C" int rus_lmhead_ce_dh_finish_probs(const float* parts, int32_t n_parts, int64_t n_tok,
+                                             int64_t d, const float* m_run, const float* lse,
+                                             const int64_t* labels, const void* w_rows,
+                                             int64_t ld_w, int64_t n_vocab, int32_t w_on_host,
+                                             const float* denom, float scale,
+                                             const float* scale_dev, const float* rest,
+                                             const float* fix, const int32_t* top, void* out,
+                                             int32_t out_dtype, void* stream) {
+  const char* fn = "rus_lmhead_ce_dh_finish_probs";
+  if (n_tok > 0 && (!rest || !fix || !top))
+    return fail(RUS_ERR_INVALID, "%s: null or misaligned pointer", fn);
+  return lmhead_dh_finish<true>(fn, parts, n_parts, n_tok, d, m_run, lse, labels, w_rows, ld_w,
+                                n_vocab, w_on_host, denom, scale, scale_dev, rest, fix, top, out,
+                                out_dtype, stream);
 }
 
 extern "C" int rus_lmhead_dh_reduce(const float* parts, int32_t n_parts, int64_t n_elem,

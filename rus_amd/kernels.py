@@ -1502,8 +1502,9 @@ def lm_head_ce_fwd_chunk(hidden: torch.Tensor, weight_rows: torch.Tensor, labels
     (replaces one iteration of the reference's forward chunk loop, ops.py:217-251). With
     ``logits_out`` ([n_tok, >= round_up(n, 64)] fp16) the rounded logits are kept there too, for
     ``lm_head_ce_grad_from_logits``. ``probs`` (out like logits_out, reference [n_tok] or None,
-    half-tile references [>= 2 parts, n_tok], zeroed maxima [n_tok]) stores the chunk's
-    probabilities relative to per-token references instead (``LMHeadPass``)."""
+    half-tile references [>= 2 parts, n_tok], zeroed maxima [n_tok], roundings like parts.m)
+    stores the chunk's probabilities relative to per-token references instead, and leaves the
+    tokens' labels out of them and of the statistics (``LMHeadPass``)."""
     fn = "lm_head_ce_fwd_chunk"
     _require_device(fn, hidden, weight_rows, labels, target, logits_out)
     if vocab_start % LM_TILE:
@@ -1522,10 +1523,11 @@ def lm_head_ce_fwd_chunk(hidden: torch.Tensor, weight_rows: torch.Tensor, labels
     nbytes = (n_tok + n_vocab) * d * 2 + 16 * n_tok * lm_head_num_parts(n_vocab)
     args = (h.data_ptr(), w.data_ptr(), lab.data_ptr(), n_tok, d, h.stride(0), w.stride(0),
             n_vocab, vocab_start, parts.m.data_ptr(), parts.s.data_ptr(), parts.w.data_ptr(),
-            parts.idx.data_ptr(), part_base, n_tok, target.data_ptr())
+            parts.idx.data_ptr())
+    tail = (part_base, n_tok, target.data_ptr())
     if logits_out is None and probs is None:
         _launch("lmhead_ce_fwd", nbytes, 2.0 * n_tok * d * n_vocab, "rus_lmhead_ce_fwd", *args,
-                _stream(h))
+                *tail, _stream(h))
         return
     kp = _round_up(n_vocab, LM_K)
     z = logits_out if probs is None else probs[0]
@@ -1536,20 +1538,23 @@ def lm_head_ce_fwd_chunk(hidden: torch.Tensor, weight_rows: torch.Tensor, labels
         raise ValueError(f"{fn}: logits_out exceeds the 4 GiB operand limit of the MFMA kernels")
     if probs is None:
         _launch("lmhead_ce_fwd_keep", nbytes + n_tok * kp * 2, 2.0 * n_tok * d * n_vocab,
-                "rus_lmhead_ce_fwd_keep", *args, z.data_ptr(), z.stride(0), _stream(h))
+                "rus_lmhead_ce_fwd_keep", *args, *tail, z.data_ptr(), z.stride(0), _stream(h))
         return
-    _, ref, half_ref, chunk_max = probs
+    _, ref, half_ref, chunk_max, part_r = probs
     if half_ref.dtype != torch.float32 or not half_ref.is_contiguous() or half_ref.shape[1] != n_tok \
-            or half_ref.shape[0] < 2 * lm_head_num_parts(n_vocab) or chunk_max.numel() != n_tok:
-        raise ValueError(f"{fn}: half-tile references or maxima too small for this chunk")
+            or half_ref.shape[0] < 2 * lm_head_num_parts(n_vocab) or chunk_max.numel() != n_tok \
+            or part_r.shape != parts.m.shape:
+        raise ValueError(f"{fn}: half-tile references, maxima or roundings too small for this chunk")
     _launch("lmhead_ce_fwd_probs", nbytes + n_tok * kp * 2, 2.0 * n_tok * d * n_vocab,
-            "rus_lmhead_ce_fwd_probs", *args, z.data_ptr(), z.stride(0), _ptr(ref),
-            half_ref.data_ptr(), chunk_max.data_ptr(), _stream(h))
+            "rus_lmhead_ce_fwd_probs", *args, part_r.data_ptr(), *tail, z.data_ptr(), z.stride(0),
+            _ptr(ref), half_ref.data_ptr(), chunk_max.data_ptr(), _stream(h))
 
 
-def lm_head_ce_combine(parts: LMHeadPartials, target: torch.Tensor, labels: torch.Tensor):
+def lm_head_ce_combine(parts: LMHeadPartials, target: torch.Tensor, labels: torch.Tensor,
+                       probs=None):
     """(lse, nll, entropy, argmax) per token from the partials (replaces lm_head_finish_kernel,
-    kernels.py:534-565)."""
+    kernels.py:534-565). ``probs`` (roundings like parts.m, vocabulary rows, rest, fix, top [n_tok])
+    for partials without the labels: the last three are written for ``lm_head_ce_dh_finish``."""
     fn = "lm_head_ce_combine"
     _require_device(fn, target, labels)
     n = parts.n_tok
@@ -1559,10 +1564,17 @@ def lm_head_ce_combine(parts: LMHeadPartials, target: torch.Tensor, labels: torc
     ent = torch.empty(n, dtype=torch.float32, device=dev)
     amax = torch.empty(n, dtype=torch.int64, device=dev)
     lab = labels.reshape(-1).contiguous()
-    _launch("lmhead_ce_combine", 16 * n * parts.n_parts + 32 * n, 0,
-            "rus_lmhead_ce_combine", parts.m.data_ptr(), parts.s.data_ptr(), parts.w.data_ptr(),
-              parts.idx.data_ptr(), parts.n_parts, n, target.data_ptr(), lab.data_ptr(), n,
-              lse.data_ptr(), nll.data_ptr(), ent.data_ptr(), amax.data_ptr(), _stream(target))
+    args = (parts.m.data_ptr(), parts.s.data_ptr(), parts.w.data_ptr(), parts.idx.data_ptr())
+    tail = (parts.n_parts, n, target.data_ptr(), lab.data_ptr(), n)
+    outs = (lse.data_ptr(), nll.data_ptr(), ent.data_ptr(), amax.data_ptr())
+    if probs is None:
+        _launch("lmhead_ce_combine", 16 * n * parts.n_parts + 32 * n, 0, "rus_lmhead_ce_combine",
+                *args, *tail, *outs, _stream(target))
+        return lse, nll, ent, amax
+    part_r, n_vocab, rest, fix, top = probs
+    _launch("lmhead_ce_combine", 20 * n * parts.n_parts + 44 * n, 0,
+            "rus_lmhead_ce_combine_probs", *args, part_r.data_ptr(), *tail, n_vocab, *outs,
+            rest.data_ptr(), fix.data_ptr(), top.data_ptr(), _stream(target))
     return lse, nll, ent, amax
 
 
@@ -1892,11 +1904,12 @@ def lm_head_ce_grad_hidden_scaled(probs: torch.Tensor, weight_t_cols: torch.Tens
 def lm_head_ce_dh_finish(parts: torch.Tensor, m_run: torch.Tensor, lse: torch.Tensor,
                          labels: torch.Tensor, w_rows: torch.Tensor, denom: torch.Tensor,
                          scale: float = 1.0, scale_dev: torch.Tensor | None = None,
-                         out_dtype=torch.float32) -> torch.Tensor:
+                         out_dtype=torch.float32, probs=None) -> torch.Tensor:
     """Hidden gradient (x 2^16 / denom x scale) of the single-pass head: (sum_s parts[s] *
     e^{m_run - lse} - W[y]) per labelled token, 0 for label -100. ``w_rows`` is the lm_head
     weight [V, d] on the device or pinned on the host (its label rows are then read over the
-    bus)."""
+    bus). ``probs`` (rest, fix, top of ``lm_head_ce_combine``) for partials without the labels:
+    - rest W[y] - fix W[top] in the place of - W[y]."""
     fn = "lm_head_ce_dh_finish"
     _require_device(fn, parts, m_run, lse, labels, denom, scale_dev)
     n_split, n_tok, d = parts.shape
@@ -1915,10 +1928,12 @@ def lm_head_ce_dh_finish(parts: torch.Tensor, m_run: torch.Tensor, lse: torch.Te
         raise ValueError(f"{fn}: labels must be int64 with {n_tok} entries")
     out = torch.empty((n_tok, d), dtype=out_dtype, device=parts.device)
     _launch("lmhead_ce_dh_finish", parts.numel() * 4 + out.numel() * out.element_size(), 0,
-            "rus_lmhead_ce_dh_finish", parts.data_ptr(), n_split, n_tok, d, m_run.data_ptr(),
+            "rus_lmhead_ce_dh_finish" if probs is None else "rus_lmhead_ce_dh_finish_probs",
+            parts.data_ptr(), n_split, n_tok, d, m_run.data_ptr(),
             lse.data_ptr(), lab.contiguous().data_ptr(), w_rows.data_ptr(), w_rows.stride(0),
             w_rows.shape[0], 1 if on_host else 0, denom.data_ptr(), float(scale),
-            _ptr(scale_dev), out.data_ptr(), _dtype_code(fn, out_dtype), _stream(parts))
+            _ptr(scale_dev), *(t.data_ptr() for t in probs or ()), out.data_ptr(),
+            _dtype_code(fn, out_dtype), _stream(parts))
     return out
 
 
@@ -1927,9 +1942,10 @@ class LMHeadPass:
 
     Per chunk: the statistics GEMM (partial m, s, w, argmax and the target logit per 256 rows)
     and, when the hidden gradient is wanted, P = fp16(2^(z log2 e - K)) in a [n_tok, chunk] buffer
-    (K a reference per token, from the chunks before), accumulated as P . W_chunk into
-    fp32 split-K partials rescaled whenever K grows. ``finish`` combines the statistics (lse,
-    nll, entropy, argmax, loss) and forms dH = sum_v (softmax - onehot) W_v x 2^16 / denom. W is
+    (K a reference per token, from the chunks before; 0 for the label, which the statistics leave
+    out as well), accumulated as P . W_chunk into fp32 split-K partials rescaled whenever K grows.
+    ``finish`` combines the statistics (lse, nll, entropy, argmax, loss; the label joins by its
+    logit) and forms dH = (sum_{v != y} p_v W_v - (1 - p_y) W_y) x 2^16 / denom. W is
     read once, and no [n_tok, V] array exists (the reference reads W twice and recomputes the
     logits, solution/ops.py:217-322)."""
 
@@ -1949,9 +1965,12 @@ class LMHeadPass:
             self.half_ref = torch.empty((2 * lm_head_num_parts(cols), n_tok),
                                         dtype=torch.float32, device=device)
             # per token: the next chunk's reference and the partials' reference of each chunk
-            # parity, the running maximum, and the partials' factor
-            rows = torch.empty((6, n_tok), dtype=torch.float32, device=device).unbind(0)
+            # parity, the latter in natural log, the partials' factor, 1 - p_y, and the rounding
+            # of the largest other probability with its vocabulary row
+            rows = torch.empty((9, n_tok), dtype=torch.float32, device=device).unbind(0)
             self.state, self.m_run, self.alpha = (rows[0:2], rows[2:4]), rows[4], rows[5]
+            self.label = (rows[6], rows[7], rows[8].view(torch.int32))
+            self.part_r = torch.empty_like(self.parts.m)
             # every chunk's GEMM reads and rewrites all the fp32 partials (the rescaled
             # accumulation), so splits beyond one round of CUs cost a partial pass per chunk for
             # a few percent of mainloop: at most one round
@@ -1975,7 +1994,8 @@ class LMHeadPass:
         if c == len(self.chunk_max):  # chunks shorter than announced
             self.chunk_max.append(torch.zeros_like(self.target))
         lm_head_ce_fwd_chunk(hidden, w_rows, labels, start, self.parts, self.target,
-                             probs=(self.z, before[0], self.half_ref, self.chunk_max[c]))
+                             probs=(self.z, before[0], self.half_ref, self.chunk_max[c],
+                                    self.part_r))
         _launch("lmhead_ce_probs_rescale", 20 * self.n_tok, 0, "rus_lmhead_ce_probs_rescale",
                 self.z.data_ptr(), self.z.stride(0), self.n_tok, n, self.half_ref.data_ptr(),
                 self.n_tok, self.chunk_max[c].data_ptr(), _ptr(before[0]), _ptr(before[1]),
@@ -1987,12 +2007,13 @@ class LMHeadPass:
     def finish(self, labels: torch.Tensor, num_items_in_batch, w_rows_all: torch.Tensor,
                dh_scale: float = 1.0, dh_dtype=torch.float32, scale_dev=None):
         """(nll, lse, entropy, argmax, denom, dh, loss); dh None without the gradient."""
-        lse, nll, ent, amax = lm_head_ce_combine(self.parts, self.target, labels)
+        probs = (self.part_r, self.n_vocab, *self.label) if self.need_grad else None
+        lse, nll, ent, amax = lm_head_ce_combine(self.parts, self.target, labels, probs)
         loss, denom = lm_head_ce_loss(nll, labels, num_items_in_batch)
         dh = None
         if self.need_grad:
             dh = lm_head_ce_dh_finish(self.dparts, self.m_run, lse, labels, w_rows_all, denom,
-                                      dh_scale, scale_dev, dh_dtype)
+                                      dh_scale, scale_dev, dh_dtype, self.label)
         return nll, lse, ent, amax, denom, dh, loss
 
 

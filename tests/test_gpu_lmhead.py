@@ -413,6 +413,82 @@ def test_pass_over_kept_logits_agrees_with_the_stored_probabilities(n, v, chunk)
         assert bool(((other.double() - want[5].double()).abs() <= tol).all())
 
 
+def _peaked(n, d, v, label_up, other_up, seed):
+    """Tokens whose label's and one other row's logit are raised above the rest (0: not raised),
+    with ignored labels and labels outside the vocabulary among them."""
+    g = torch.Generator().manual_seed(seed)
+    h = torch.randn(n, d, generator=g)
+    w = torch.randn(v, d, generator=g) * 0.05
+    rows = torch.randperm(v, generator=g)[: 2 * n]
+    dirs = h / h.pow(2).sum(1, keepdim=True)
+    w[rows[:n]] += label_up * dirs
+    w[rows[n:]] += other_up * dirs
+    labels = rows[:n].clone()
+    labels[3::11] = -100
+    labels[5], labels[6] = v + 300, -7
+    return h.half().to(DEV), w.half().to(DEV), labels.to(DEV)
+
+
+# log(sum of the other logits) is about 9.3: mean nll near 1e-1, 1e-3 and 1e-5 with the label the
+# argmax; another row at p 0.999; label and another row at about one half each; nothing raised
+@pytest.mark.parametrize("label_up,other_up", [(11.6, 0), (16.2, 0), (20.8, 0), (0, 16.2),
+                                               (18.0, 18.0), (0, 0)])
+@pytest.mark.parametrize("layout", ["chunks", "one chunk", "256 rows", "streamed", "blocks"])
+def test_hidden_gradient_of_peaked_tokens(layout, label_up, other_up):
+    """dH of tokens that the model predicts well, or wrongly with confidence, against float64 softmax
+    of the device's own fp16 logits. In the single pass only the probabilities beside the label and
+    the largest other one are rounded to fp16 (2^-11 relative, 2^-24 of the largest below fp16's
+    normal range); the rest is fp32 relative to lse's size. The token blocks round G once and form
+    p - 1 from lse, whose fp32 resolution stays in the label's coefficient."""
+    from rus_amd import ops
+    from rus_amd.hostload import HostHead
+
+    n, d, v = 300, 256, 8192 + 130
+    h, w, labels = _peaked(n, d, v, label_up, other_up, seed=int(10 * label_up + other_up))
+    if layout == "streamed":
+        head = HostHead(w.cpu(), DEV, v_chunk=2048, resident=False)
+        out = ops._lm_head_streamed(h, labels, head, None, True)
+    else:
+        chunk = {"chunks": 2048, "one chunk": 33 * 256, "256 rows": 256, "blocks": None}[layout]
+        out = K.lm_head_ce(h, w, labels, v_chunk=chunk)
+    nll, lse, dh = out[0], out[1], out[5]
+    z = torch.empty(n, K._round_up(v, 64), dtype=torch.float16, device=DEV)
+    K.lm_head_ce_logits(h, w, z)
+    torch.cuda.synchronize()
+    z, wd, y = z[:, :v].double().cpu(), w.double().cpu(), labels.cpu()
+    want_lse = torch.logsumexp(z, -1)
+    e32 = 2.0**-22 * (4 + want_lse.abs())
+    assert bool(((lse.double().cpu() - want_lse).abs() <= e32).all())
+    inside = (y >= 0) & (y < v)
+    at = torch.arange(n)
+    yc = torch.where(inside, y, 0)
+    p = torch.exp(z - want_lse[:, None])
+    p_y = torch.where(inside, p[at, yc], 0.0)
+    others = p.clone()
+    others[at[inside], y[inside]] = 0
+    rest = torch.where(inside, others.sum(1), 0.0)
+    want_nll = torch.where(inside, -torch.log1p(-rest), want_lse) * (y != -100)
+    assert bool(((nll.double().cpu() - want_nll).abs() <= e32).all())
+    scale = 65536.0 / int((y != -100).sum())
+    live = (y != -100)[:, None]
+    want = (others @ wd - rest[:, None] * wd[yc]) * scale * live
+    top = others.amax(1)
+    rounded = others.clone()
+    if layout != "blocks":
+        rounded[at, others.argmax(1)] *= (top < 0.065).double()
+    mag = others @ wd.abs() + rest[:, None] * wd[yc].abs()
+    tol = 2.0**-11 * (rounded @ wd.abs()) + 2.0**-24 * top[:, None] * wd.abs().sum(0)
+    tol = tol + 2 * e32[:, None] * mag
+    if layout == "blocks":
+        tol = tol + 2.0**-11 * rest[:, None] * wd[yc].abs() + 2.0**-25 / scale * wd.abs().sum(0) \
+            + e32[:, None] * p_y[:, None] * wd[yc].abs()
+    got = dh.double().cpu()
+    err = (got - want).abs()
+    assert bool((err <= tol * scale + 1e-30).all()), float((err / (tol * scale + 1e-30)).max())
+    if layout != "blocks":
+        assert float((got - want).norm() / want.norm()) <= 1e-3
+
+
 def test_labels_past_the_vocabulary_within_its_last_tile():
     """A label of the last 256-row tile that is no vocabulary row counts as outside the vocabulary
     (target logit 0, no weight row), whatever lies in the tile's padding."""
