@@ -300,11 +300,12 @@ __device__ __forceinline__ void stats_epilogue(char* smem, const GemmArgs& g, co
     w += __shfl_xor(w, 32, kWave);
     if constexpr (OUT == kProbs) {
       // The partial's sums are relative to its maximum. Far below the reference (2^-100 of the
-      // token's total at most) the exponentials may be all zero: any bounded sum will do.
+      // token's total at most) the exponentials may be all zero: any bounded sum will do, but a NaN
+      // among them stays one.
       const float up = ref - m * kLog2e;
       const float f = exp2_fast(up);
-      s = up > 100.0f ? 1.0f : s * f;
-      w = up > 100.0f ? m : w * f;
+      s = up > 100.0f ? s * 0.0f + 1.0f : s * f;
+      w = up > 100.0f ? w * 0.0f + m : w * f;
       if (!(m > -INFINITY)) s = w = 0.0f;
     }
     rm[nt] = m;

@@ -504,3 +504,22 @@ def test_labels_past_the_vocabulary_within_its_last_tile():
         for x, y in zip(a, b):
             assert (x is None and y is None) or torch.equal(x, y), kw
         assert torch.equal(a[0][::2], a[1][::2])  # nll = lse - 0
+
+
+@pytest.mark.parametrize("kw", [{"v_chunk": 256}, {"v_chunk": 512}, {"v_chunk": 1280},
+                                {"need_grad": False}, {"block_tokens": 256}])
+def test_nan_logit_far_below_the_maximum_stays_in_the_loss(kw):
+    """A NaN among logits far below the rest (here e^-400 of the total) is not summed away."""
+    n, d, v = 300, 128, 1100
+    g = torch.Generator().manual_seed(5)
+    h, w = torch.randn(n, d, generator=g), torch.randn(v, d, generator=g) * 0.1
+    h[:, 0] = 4.0
+    w[:, 0] = 50.0
+    w[256:512, 0] = -50.0
+    w[300, 5] = float("nan")
+    labels = torch.randint(0, 200, (n,), generator=g)
+    out = K.lm_head_ce(h.half().to(DEV), w.half().to(DEV), labels.to(DEV), **kw)
+    for i in (0, 1, 2, 6):  # nll, lse, entropy, loss
+        assert bool(out[i].isnan().all()), i
+    if out[5] is not None:
+        assert bool(out[5].isnan().all())
