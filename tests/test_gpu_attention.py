@@ -238,3 +238,43 @@ def test_attention_wide_blocks_match_oracle(lens, hq, hkv):
     """Batches large enough for the 128-token blocks (edges of blocks and tiles, rows shorter than a
     block, ragged offsets), with large scores in one of them so that the running maximum moves."""
     _run(lens, hq, hkv, seed=sum(lens) + hq, qk_scale=3.0 if hkv == 1 else 1.0)
+
+
+def _exact(q, k, v, dout, lens):
+    """float64 (out, dq, dk, dv) on the device, one head at a time."""
+    leaves = [t.double().requires_grad_(True) for t in (q, k, v)]
+    qd, kd, vd = leaves
+    grp, outs, a = q.shape[1] // k.shape[1], [], 0
+    for n in lens:
+        causal = torch.ones(n, n, dtype=torch.bool, device=q.device).tril()
+        heads = []
+        for h in range(q.shape[1]):
+            s = qd[a:a + n, h] @ kd[a:a + n, h // grp].t().contiguous() / math.sqrt(128)
+            p = torch.softmax(s.masked_fill(~causal, -math.inf), -1)
+            heads.append(p @ vd[a:a + n, h // grp])
+        outs.append(torch.stack(heads, 1))
+        a += n
+    out = torch.cat(outs)
+    return [out.detach(), *torch.autograd.grad(out, leaves, dout.double())]
+
+
+@pytest.mark.parametrize("qk_scale", [1.0, 3.0])
+def test_wide_attention_is_as_accurate_as_the_narrow_blocks(qk_scale):
+    """16 rows of 512 in one call (128-token blocks) and one call each (32-token blocks): the errors
+    of both against float64 are those of P's fp16 rounding and of the outputs', and the first must not
+    exceed the second's by more than 1% (their own scatter over inputs is 0.3%)."""
+    lens, (hq, hkv) = [512] * 16, (12, 2)
+    q, k, v, dout, cu = _inputs(lens, hq, hkv, seed=2, qk_scale=qk_scale)
+    q, k, v, dout = _dev(q, k, v, dout)
+
+    def run(a, b, rows):
+        c = torch.tensor(rows, dtype=torch.int32, device=DEV)
+        x = [t[a:b].contiguous() for t in (q, k, v, dout)]
+        out, lse = K.attn_varlen_fwd(*x[:3], c)
+        return [out, *K.attn_varlen_bwd(x[3], *x[:3], out, lse, c)]
+
+    wide = run(0, cu[-1], cu)
+    narrow = [torch.cat(t) for t in zip(*(run(a, a + 512, [0, 512]) for a in cu[:-1]))]
+    for name, w, s, x in zip(("out", "dq", "dk", "dv"), wide, narrow, _exact(q, k, v, dout, lens)):
+        e_w, e_s = (float((t.double() - x).norm() / x.norm()) for t in (w, s))
+        assert e_w <= 1.01 * e_s, (name, e_w, e_s)
