@@ -1247,19 +1247,22 @@ attn_bwd_wide_kernel(AttnArgs a) {
     bwd_wide_dq(a, blk - a.n_blocks, head, lds);
 }
 
-// Whether a batch takes the wide kernels: when its 128-token blocks are at least min_blocks, or
-// kShortWideBlocks if its rows average at most one such block. The lines are where both kernels
-// take the same time (256 CUs; 12 / 2 heads, old -> wide): forward 2,048 tokens = 192 blocks in
-// rows of 512 18.0 -> 17.0 us, as one row 43 -> 48, 3,072 tokens 37 -> 28; backward with partials
-// 1,536 tokens (144 blocks) in rows of 512 39 -> 34 us, of 1,024 and 512 50 -> 55, 2,048 tokens as
-// one row 113 -> 102, in rows of 512 45 -> 34; 14 rows of 100 forward 11.4 -> 8.6, backward
-// 27 -> 17. Scores are scaled after their maximum is taken, hence scale > 0.
-constexpr int kFwdWideBlocks = 256, kBwdWideBlocks = 192, kShortWideBlocks = 128;
+// Whether a batch takes the wide kernels: when its 128-token blocks are at least min_blocks. How long
+// its rows are is known on the device only (and changes from replay to replay of a captured graph),
+// and a long row is what the wide kernels do worse: one block walks its whole length where the
+// 32-token blocks' waves share it. So the lines are where no mixture of rows is slower (256 CUs, us,
+// 32-token blocks -> wide). Backward with partials, 12 / 2 heads: 192 blocks 2,048 tokens in rows of
+// 512 44 -> 33, as one row 112 -> 100, 800 + 18 rows of 64 48 -> 44 (but 156 blocks, 1,024 + 10 rows
+// of 64, 51 -> 56). Forward: 300 blocks 1,500 + 27 rows of 64 42 -> 41, 1,024 + 35 rows of 64 34 ->
+// 31, one row of 3,300 90 -> 83; 288 blocks one row of 4,600 with 8 heads 110 -> 112, 256 blocks two
+// rows of 2,000 with 8 heads 46 -> 51. Below the lines rows of one length would gain (14 rows of 100
+// forward 12.3 -> 10.2, backward 27 -> 17), one long row among short ones lose as much (1,024 + 13
+// rows of 20 forward 21 -> 30, backward 46 -> 53). Scores are scaled after their maximum is taken,
+// hence scale > 0.
+constexpr int kFwdWideBlocks = 300, kBwdWideBlocks = 192;
 
-bool wide(int64_t n_tok, int n_seq, int h_q, float scale, int min_blocks) {
-  const int64_t blocks = (n_tok + kWide - 1) / kWide * h_q;
-  return scale > 0.0f &&
-         blocks >= (n_tok <= kWide * static_cast<int64_t>(n_seq) ? kShortWideBlocks : min_blocks);
+bool wide(int64_t n_tok, int h_q, float scale, int min_blocks) {
+  return scale > 0.0f && (n_tok + kWide - 1) / kWide * h_q >= min_blocks;
 }
 
 // Bound of the 128-token blocks over all rows (at most the caller's bound of 32-token blocks).
@@ -1316,7 +1319,7 @@ extern "C" int rus_attn_varlen_fwd(const void* q, const void* k, const void* v,
   a.h_kv = h_kv;
   a.scale = scale;
   a.scale_log2 = scale * kLog2e;
-  if (wide(n_tokens, n_seq, h_q, scale, kFwdWideBlocks)) {
+  if (wide(n_tokens, h_q, scale, kFwdWideBlocks)) {
     a.n_blocks = wide_blocks(n_tokens, n_seq, max_blocks);
     hipLaunchKernelGGL(attn_fwd_wide_kernel, dim3(wide_grid(a.n_blocks, a)), dim3(64 * kW), 0,
                        static_cast<hipStream_t>(stream), a);
@@ -1374,7 +1377,7 @@ static int attn_bwd(const char* fn, const void* q, const void* k, const void* v,
   a.dk = static_cast<f16*>(dk);
   a.dv = static_cast<f16*>(dv);
   a.max_blocks = max_blocks;
-  if (wide(n_tokens, n_seq, h_q, scale, kBwdWideBlocks)) {
+  if (wide(n_tokens, h_q, scale, kBwdWideBlocks)) {
     a.n_blocks = wide_blocks(n_tokens, n_seq, max_blocks);
     hipLaunchKernelGGL(attn_bwd_wide_kernel, dim3(wide_grid(2 * a.n_blocks, a)), dim3(64 * kW), 0,
                        st, a);

@@ -278,3 +278,22 @@ def test_wide_attention_is_as_accurate_as_the_narrow_blocks(qk_scale):
     for name, w, s, x in zip(("out", "dq", "dk", "dv"), wide, narrow, _exact(q, k, v, dout, lens)):
         e_w, e_s = (float((t.double() - x).norm() / x.norm()) for t in (w, s))
         assert e_w <= 1.01 * e_s, (name, e_w, e_s)
+
+
+def test_mixed_rows_below_the_wide_lines_take_the_narrow_blocks():
+    """One long row among short ones, too few blocks for the 128-token kernels: the 32-token blocks,
+    whose results do not depend on the rest of the batch, so each row alone gives the same bits."""
+    lens = [1024] + [35] * 11
+    q, k, v, dout, cu = _inputs(lens, 12, 2, seed=4)
+    q, k, v, dout = _dev(q, k, v, dout)
+
+    def run(a, b, rows):
+        c = torch.tensor(rows, dtype=torch.int32, device=DEV)
+        x = [t[a:b].contiguous() for t in (q, k, v, dout)]
+        out, lse = K.attn_varlen_fwd(*x[:3], c)
+        return [out, *K.attn_varlen_bwd(x[3], *x[:3], out, lse, c)]
+
+    whole = run(0, cu[-1], cu)
+    alone = [torch.cat(t) for t in zip(*(run(a, b, [0, b - a]) for a, b in zip(cu[:-1], cu[1:])))]
+    for a, b in zip(whole, alone):
+        assert torch.equal(a, b)
