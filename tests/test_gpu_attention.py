@@ -297,3 +297,69 @@ def test_mixed_rows_below_the_wide_lines_take_the_narrow_blocks():
     alone = [torch.cat(t) for t in zip(*(run(a, b, [0, b - a]) for a, b in zip(cu[:-1], cu[1:])))]
     for a, b in zip(whole, alone):
         assert torch.equal(a, b)
+
+
+# batches for the 128-token blocks of both passes: over 64 rows, empty ones among them, none longer
+# than a block; a few long rows
+WIDE_SHORT = [(37 * i) % 129 for i in range(100)]
+WIDE_LONG = [1500, 0, 300, 129, 1400]
+
+
+@pytest.mark.parametrize("lens,hq,hkv", [
+    (WIDE_SHORT, 12, 2),
+    (WIDE_LONG, 12, 2),
+    ([512] * 4, 12, 2),  # 192 blocks: 32-token blocks forward, 128-token blocks backward
+    ([1700, 1790, 1500], 8, 8),
+    ([2400, 2500], 8, 1),
+])
+def test_attention_wide_row_mixtures_match_oracle(lens, hq, hkv):
+    _run(lens, hq, hkv, seed=len(lens), qk_scale=3.0 if hkv == 1 else 1.0)
+
+
+@pytest.mark.parametrize("lens", [WIDE_SHORT, [1700, 1500]])
+def test_attention_wide_rising_scores(lens):
+    """As test_attention_rising_scores for the 128-token blocks: the running maximum moves at every
+    pair of key tiles, by more than 2^8 where the row is long."""
+    q, k, v, dout, cu = _inputs(lens, 12, 2, seed=8)
+    ramp = torch.cat([torch.linspace(0.0, 1.0, n) for n in lens])
+    k = (k.float() * 0.1 + 24.0 * ramp[:, None, None]).half()
+    q = (q.float() * 0.1 + 1.0).half()
+    out_ref, lse_ref = ref.attention_varlen_fwd(q, k, v, cu)
+    bounds = _bounds(q, k, v, dout, cu)
+    qd, kd, vd, dd = _dev(q, k, v, dout)
+    cud = torch.tensor(cu, dtype=torch.int32, device=DEV)
+    out, lse = K.attn_varlen_fwd(qd, kd, vd, cud)
+    grads = K.attn_varlen_bwd(dd, qd, kd, vd, out, lse, cud)
+    torch.cuda.synchronize()
+    _check("out", out, out_ref, bounds[0])
+    torch.testing.assert_close(lse.double().cpu(), lse_ref, rtol=1e-6, atol=1e-4)
+    want = ref.attention_varlen_bwd(dout, q, k, v, cu)
+    for name, g, w, b in zip(("dq", "dk", "dv"), grads, want, bounds[1:]):
+        _check(name, g, w, b)
+
+
+@pytest.mark.parametrize("lens", [WIDE_SHORT, WIDE_LONG])
+def test_attention_wide_deterministic_extra_blocks_and_partials(lens):
+    """The 128-token blocks give the same bits again and with more blocks announced than there are;
+    their per-query-head partials, summed in head order and rounded once, are dk and dv."""
+    hq, hkv = 12, 2
+    q, k, v, dout, cu = _inputs(lens, hq, hkv, seed=1)
+    qd, kd, vd, dd = _dev(q, k, v, dout)
+    cud = torch.tensor(cu, dtype=torch.int32, device=DEV)
+    more = K.attn_max_blocks(sum(lens), len(lens)) + 40
+    o1, l1 = K.attn_varlen_fwd(qd, kd, vd, cud)
+    o2, l2 = K.attn_varlen_fwd(qd, kd, vd, cud, max_blocks=more)
+    g1 = K.attn_varlen_bwd(dd, qd, kd, vd, o1, l1, cud)
+    g2 = K.attn_varlen_bwd(dd, qd, kd, vd, o2, l2, cud, max_blocks=more)
+    parts = K.attn_varlen_bwd_parts(dd, qd, kd, vd, o1, l1, cud)
+    torch.cuda.synchronize()
+    assert torch.equal(o1, o2) and torch.equal(l1, l2)
+    for a, b in zip(g1, g2):
+        assert torch.equal(a, b)
+    assert torch.equal(parts[0], g1[0])
+    for part, full in zip(parts[1:], g1[1:]):
+        part = part.view(hkv, hq // hkv, -1, 128)
+        acc = part[:, 0].clone()
+        for j in range(1, hq // hkv):
+            acc += part[:, j]
+        assert torch.equal(acc.half().permute(1, 0, 2).contiguous(), full)
