@@ -744,10 +744,11 @@ bool wide_w_plan(const BwdWArgs& a, int r, WideW& w) {
   return true;
 }
 
-// LoRA-down by row blocks (lora_rows.h): block b forms mid_q / mid_v of tokens T b .. + T - 1.
+// LoRA-down by row blocks (lora_rows.h): block b forms mid_q / mid_v of four tokens (or T) from 4 b on.
+template <bool DROP>
 __global__ __launch_bounds__(256) void lora_down_rows_kernel(DownRows a) {
   __shared__ float park[kDownParkFloats];
-  lora_down_rows<4, kDownRows>(a, static_cast<int64_t>(blockIdx.x) * kDownRows, park);
+  lora_down_rows4<DROP>(a, static_cast<int64_t>(blockIdx.x) * kDownRows, park);
 }
 
 template <int T>
@@ -1213,9 +1214,12 @@ extern "C" int rus_lora_down_rows(const rus_lora_rows* q, void* stream) {
   // Tiles in LDS where the widths allow (one block per CU); 4, 8 or 16 tokens per block keep the grid
   // within one round of 256 CUs up to 4,096 tokens, and A is copied once per block. The fragments
   // from memory take 13.5 / 18.1 / 54.0 us at 707 / 2,048 / 8,161 tokens, the tiles 9.6 / 10.5 / 19.6.
-  if (q->d % 512 || q->d > 512 * kDownTiles || !aligned(q->bits_q, 16) || !aligned(q->bits_v, 16))
-    hipLaunchKernelGGL(lora_down_rows_kernel, blocks(kDownRows), dim3(256), 0, st, a);
-  else if (n <= 1024)
+  if (q->d % 512 || q->d > 512 * kDownTiles || !aligned(q->bits_q, 16) || !aligned(q->bits_v, 16)) {
+    if (q->bits_q)
+      hipLaunchKernelGGL(lora_down_rows_kernel<true>, blocks(kDownRows), dim3(256), 0, st, a);
+    else
+      hipLaunchKernelGGL(lora_down_rows_kernel<false>, blocks(kDownRows), dim3(256), 0, st, a);
+  } else if (n <= 1024)
     hipLaunchKernelGGL(lora_down_tiled_kernel<4>, blocks(4), dim3(256), 0, st, a);
   else if (n <= 2048)
     hipLaunchKernelGGL(lora_down_tiled_kernel<8>, blocks(8), dim3(256), 0, st, a);

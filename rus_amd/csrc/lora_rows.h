@@ -117,30 +117,29 @@ __device__ __forceinline__ void down_rows_finish(const DownRows& a, int64_t t0, 
   }
 }
 
-// mid_q / mid_v of tokens t0 .. t0 + T - 1 (those below n_tok; T 4 to 32), by all four waves of
-// the block: wave w reduces columns [w d/4, (w+1) d/4) on v_mfma_f32_32x32x16_f16 with ranks as
-// rows (rows 0 .. r-1 the q ranks against drop_q(x), r .. 2r-1 the v ranks against drop_v(x), the
-// rest zero) and tokens as columns (T .. 31 zero); the waves' sums meet in `park` (T * 128 floats
-// of LDS) and are added in wave order, then rounded to fp16 once: a token's result does not depend
-// on T. Every thread of the block must call it (it holds barriers); x's rows must be visible to
-// the whole block.
-template <int U, int T>
-__device__ __forceinline__ void lora_down_rows(const DownRows& a, int64_t t0, float* park) {
+// mid_q / mid_v of tokens t0 .. t0 + 3 (those below n_tok), by all four waves of the block: wave w
+// reduces columns [w d/4, (w+1) d/4) on v_mfma_f32_32x32x16_f16 with ranks as rows (rows 0 .. r-1
+// the q ranks against drop_q(x), r .. 2r-1 the v ranks against drop_v(x), the rest zero) and tokens
+// as columns (4 .. 31 zero); the waves' sums meet in `park` (kDownParkFloats of LDS) and are added
+// in wave order, then rounded to fp16 once. Every thread of the block must call it (it holds
+// barriers); x's rows must be visible to the whole block. DROP (keep bits given) is a template
+// argument: with both forms in one loop the plain one took 9.8 us at d = 2,048, 707 tokens and rank
+// 16, the dropping one 16.2; apart 7.9 and 13.9.
+template <bool DROP>
+__device__ __forceinline__ void lora_down_rows4(const DownRows& a, int64_t t0, float* park) {
+  constexpr int U = 4;  // K steps whose loads are issued together (registers against latency)
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, h = lane >> 5, col = lane & 31;
   const bool is_q = col < a.r, is_v = col >= a.r && col < 2 * a.r;
   const f16* arow = is_q ? a.aq + static_cast<int64_t>(col) * a.d
                          : a.av + static_cast<int64_t>(is_v ? col - a.r : 0) * a.d;
   const int64_t t = t0 + col;
-  const bool live = col < T && t < a.n_tok;
+  const bool live = col < kDownRows && t < a.n_tok;
   const f16* xrow = a.x + (live ? t : 0) * a.sx;
-  const bool drop = a.bits_q != nullptr;  // uniform
-  const uint32_t* mq = drop ? a.bits_q + (live ? t : 0) * a.words : nullptr;
-  const uint32_t* mv = drop ? a.bits_v + (live ? t : 0) * a.words : nullptr;
+  const uint32_t* mq = DROP ? a.bits_q + (live ? t : 0) * a.words : nullptr;
+  const uint32_t* mv = DROP ? a.bits_v + (live ? t : 0) * a.words : nullptr;
   const int per = a.d / 4;  // a multiple of 16
   const int c_begin = wave * per;
   f32x16 acc = f32x16{};
-  // U: K steps whose loads are issued together (register budget vs latency; no effect on the
-  // arithmetic)
   for (int s0 = 0; s0 < per; s0 += 16 * U) {
     f16x8 af[U], xf[U];
     uint32_t wq[U], wv[U];
@@ -149,7 +148,7 @@ __device__ __forceinline__ void lora_down_rows(const DownRows& a, int64_t t0, fl
       const int c = c_begin + min(s0 + 16 * u, per - 16) + 8 * h;
       af[u] = (is_q || is_v) ? ld8(arow + c) : zero8();
       xf[u] = live ? ld8(xrow + c) : zero8();
-      if (drop) {
+      if constexpr (DROP) {
         wq[u] = live ? mq[c >> 5] : 0u;
         wv[u] = live ? mv[c >> 5] : 0u;
       }
@@ -159,7 +158,7 @@ __device__ __forceinline__ void lora_down_rows(const DownRows& a, int64_t t0, fl
     for (int u = 0; u < U; ++u) {
       // Steps past the wave's range add zero products: no branch, the batch's loads stay ahead.
       const f16x8 x = s0 + 16 * u < per ? xf[u] : zero8();
-      if (drop) {
+      if constexpr (DROP) {
         const int sh = (c_begin + min(s0 + 16 * u, per - 16) + 8 * h) & 31;
         acc = mfma(is_q ? af[u] : zero8(), drop8(x, wq[u], sh, a.scale_q), acc);
         acc = mfma(is_v ? af[u] : zero8(), drop8(x, wv[u], sh, a.scale_v), acc);
@@ -168,10 +167,10 @@ __device__ __forceinline__ void lora_down_rows(const DownRows& a, int64_t t0, fl
       }
     }
   }
-  down_rows_finish<T>(a, t0, acc, park);
+  down_rows_finish<kDownRows>(a, t0, acc, park);
 }
 
-// lora_down_rows with both operands through LDS: the same MFMA sequence on the same operands, so
+// lora_down_rows4 with both operands through LDS: the same MFMA sequence on the same operands, so
 // the same bits. A fragment read straight from memory touches 32 rows x 32 bytes; here each wave
 // copies its quarter of the columns in tiles of 128 (32 rank rows of A and T token rows of x, whole
 // 256-byte rows per 16 lanes, chunk c of row r at c ^ swz(r)), all at once: one memory latency.
@@ -296,7 +295,7 @@ __device__ __forceinline__ void stage_down_rows(const DownRows& a, int64_t t0, f
   __syncthreads();
 }
 
-// lora_down_rows<., 4> with the block's x rows and keep bits already in LDS (stage_down_rows): the
+// lora_down_rows4 with the block's x rows and keep bits already in LDS (stage_down_rows): the
 // same MFMA sequence on the same operands, so the same bits. Only the A fragments come from
 // global memory, U K steps of them issued together; x and the bits are read from LDS at each
 // step, so a batch holds 4 U registers per lane.
@@ -328,7 +327,7 @@ __device__ __forceinline__ void lora_down_rows4_staged(const DownRows& a, int64_
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int c = c_begin + min(s0 + 16 * u, per - 16) + 8 * h;
-      // Steps past the wave's range add zero products, as in lora_down_rows.
+      // Steps past the wave's range add zero products, as in lora_down_rows4.
       const f16x8 x = (live && s0 + 16 * u < per) ? ld8(xrow + c) : zero8();
       if (drop) {
         const uint32_t wq = live ? mq[c >> 5] : 0u, wv = live ? mv[c >> 5] : 0u;
