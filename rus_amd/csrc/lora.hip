@@ -724,7 +724,7 @@ __global__ __launch_bounds__(256) void lora_bwd_wide_kernel(WideW a, ExpandArgs 
 }
 
 // Whether the MFMA weight-gradient blocks take a call, and their launch plan.
-bool wide_w_plan(const BwdWArgs& a, int r, WideW& w) {
+bool wide_w_plan(const BwdWArgs& a, int r, int64_t workspace_floats, WideW& w) {
   constexpr int64_t kMinTok = 256;
   if (r != 16 || a.n_tok < kMinTok) return false;
   for (int k = 0; k < 4; ++k)
@@ -732,8 +732,9 @@ bool wide_w_plan(const BwdWArgs& a, int r, WideW& w) {
   w.w = a;
   const int64_t nx = (a.cols[0] + 63) / 64, nq = (a.cols[1] + 127) / 128,
                 nv = (a.cols[3] + 127) / 128;
-  // two to three blocks of 40 KiB LDS per CU; chunks of at least 256 tokens, so that the partials
-  // fit the workspace the 128-token chunks are sized for
+  // two to three blocks of 40 KiB LDS per CU, and at most ceil(n / 256) chunks: with the nb 64-column
+  // blocks of all four operands, 2 n_blk <= nb + 2 and nb >= 4, so the partials fit the workspace of
+  // the 128-token chunks, ceil(n / 128) nb kTPart / 2 floats (to the last one at 257 tokens, nb = 4)
   const int64_t want = std::max<int64_t>(1, std::min((a.n_tok + 255) / 256, 640 / (nx + nq + nv)));
   const int64_t chunk = ((a.n_tok + want - 1) / want + kTTok - 1) / kTTok * kTTok;
   w.nx = static_cast<int>(nx);
@@ -741,7 +742,7 @@ bool wide_w_plan(const BwdWArgs& a, int r, WideW& w) {
   w.n_blk = static_cast<int>(nx + nq + nv);
   w.chunk = static_cast<int>(chunk);
   w.n_chunk = static_cast<int>((a.n_tok + chunk - 1) / chunk);
-  return true;
+  return static_cast<int64_t>(w.n_blk) * w.n_chunk * kTPart <= workspace_floats;
 }
 
 // LoRA-down by row blocks (lora_rows.h): block b forms mid_q / mid_v of four tokens (or T) from 4 b on.
@@ -1114,7 +1115,7 @@ extern "C" int rus_lora_bwd_w(const void* x, int64_t stride_x, const uint32_t* b
     return e;
   hipStream_t st = static_cast<hipStream_t>(stream);
   WideW w;
-  if (wide_w_plan(a, r, w)) {
+  if (wide_w_plan(a, r, workspace_floats, w)) {
     const dim3 wgrid(static_cast<uint32_t>(w.n_blk * w.n_chunk));
     if (bits_q)
       hipLaunchKernelGGL((lora_bwd_wide_kernel<true, false>), wgrid, dim3(256), 0, st, w,
@@ -1169,7 +1170,7 @@ extern "C" int rus_lora_bwd_xw(const void* x, int64_t stride_x, const uint32_t* 
                 bits_q ? 1.0f / (1.0f - p_q) : 1.0f, bits_v ? 1.0f / (1.0f - p_v) : 1.0f};
   hipStream_t st = static_cast<hipStream_t>(stream);
   WideW w;
-  if (wide_w_plan(a, r, w)) {
+  if (wide_w_plan(a, r, workspace_floats, w)) {
     const int64_t xcw = (d / 32 + kSW - 1) / kSW;
     const dim3 wgrid(static_cast<uint32_t>(static_cast<int64_t>(w.n_blk) * w.n_chunk +
                                            xcw * tiles(n_tokens)));

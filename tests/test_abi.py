@@ -208,6 +208,28 @@ def test_dequant_carried_lora_down_must_read_the_norm_output():
                   None)
 
 
+def test_lora_workspace_holds_the_mfma_weight_gradient_partials():
+    """The MFMA blocks of the rank-16 weight gradients (64 columns of x, 128 of dq or dv, 2,048 floats
+    each) over their token chunks fit the workspace that the 64-column, 128-token blocks are sized
+    for, at every size (exactly, at 257 to 320 tokens with one block per operand)."""
+    from rus_amd import kernels as K
+
+    up = lambda a, b: -(-a // b)
+    tight = 0
+    for n in [*range(256, 1400), 2048, 2049, 8161, 16384, 100001]:
+        for d, dq, dv in ((64, 8, 8), (64, 128, 8), (72, 136, 8), (192, 200, 72), (896, 896, 128),
+                          (1536, 1536, 256), (3584, 3584, 512), (8192, 8192, 1024),
+                          (40960, 40960, 40960)):
+            n_blk = up(d, 64) + up(dq, 128) + up(dv, 128)
+            want = max(1, min(up(n, 256), 640 // n_blk))
+            chunk = up(up(n, want), 64) * 64
+            need = up(n, chunk) * n_blk * 2048
+            have = K.lora_workspace_size(K.LORA_BWD_W, n, d, dq, dv, 16)[0]
+            assert need <= have, (n, d, dq, dv)
+            tight += need == have
+    assert tight
+
+
 def test_lora_workspace_sizes_follow_the_block_decomposition():
     from rus_amd import kernels as K
 
