@@ -383,8 +383,8 @@ attn_fwd_kernel(AttnArgs a) {
 
 // ---------------------------------------------------------------------------------------------
 // Backward, on the LDS tiles: row fragments for S = Q K^T and dP = dO V^T, transposed fragments
-// for dV += P^T dO, dK += dS^T Q and dQ^T += K^T dS^T. D = rowsum(dO o O) is formed once per
-// (head, query) by a small kernel before the main launch.
+// for dV += P^T dO, dK += dS^T Q and dQ^T += K^T dS^T. D = rowsum(dO o O) is formed by each block for
+// the query rows it visits (below).
 // ---------------------------------------------------------------------------------------------
 // Waves per backward block: 4 (80 KiB of LDS and at most 256 registers, so two blocks share a
 // CU and one block's waits overlap the other's work; 8 waves in one block per CU ran 13% slower).

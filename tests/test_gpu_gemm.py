@@ -67,8 +67,9 @@ def test_gemm_parts_matches_fp32_product(m, n, k, n_split, b_kn):
 @pytest.mark.parametrize("m", [1, 128, 129, 256, 385])
 @pytest.mark.parametrize("n", [8, 64, 72, 128, 136, 192, 200, 256, 264, 384])
 def test_gemm_parts_of_tiles_partly_inside_the_matrix(m, n, b_kn):
-    """Row halves and column quarters of a tile outside the matrix are neither copied nor
-    multiplied: sizes on both sides of each, over one to three 64-deep stages per split."""
+    """Row halves and column quarters of a tile outside the matrix are not multiplied (their copies
+    re-read the last row or columns): sizes on both sides of each, over one to three 64-deep stages
+    per split."""
     for k, n_split in ((64, 1), (128, 1), (320, 2)):
         a, b = _operands(m, n, k, b_kn, seed=m + n + k)
         _check(a, b, b_kn, n_split, k)
