@@ -766,7 +766,7 @@ int rus_attn_varlen_fwd(const void* q, const void* k, const void* v, const int32
  * partials [h_q, n_tokens, 128] each, dK scaled). Both passes (dQ, and the partials of dK / dV)
  * run as one launch, each block forming D = rowsum(dO o O) of the query rows it visits; a second
  * one sums each group's heads. max_blocks at most 32767.
- * counters: int32, at least max_blocks * h_kv (checked, but not read: no launch counts arrivals).
+ * counters: not used (no launch counts arrivals): NULL and 0, or int32, at least max_blocks * h_kv.
  * Replaces: the autograd backward of solution/ops.py:669-696 (torch SDPA backward plus the
  * sum over the expanded K/V heads), run by solution/ops.py:903-928.
  */

@@ -1343,12 +1343,12 @@ static int attn_bwd(const char* fn, const void* q, const void* k, const void* v,
       !aligned(dq, 16) || !aligned(workspace, 16))
     return fail(RUS_ERR_INVALID, "%s: null or misaligned argument", fn);
   if (group_sum) {
-    if (!dk || !dv || !aligned(dk, 16) || !aligned(dv, 16) || !counters || !aligned(counters, 4))
+    if (!dk || !dv || !aligned(dk, 16) || !aligned(dv, 16) || !aligned(counters, 4))
       return fail(RUS_ERR_INVALID, "%s: null or misaligned argument", fn);
     if (h_q / h_kv > kMaxGroup)
       return fail(RUS_ERR_UNSUPPORTED, "%s: %d query heads per KV head (at most %d)", fn,
                   h_q / h_kv, kMaxGroup);
-    if (n_counters < static_cast<int64_t>(max_blocks) * h_kv)
+    if ((counters || n_counters) && n_counters < static_cast<int64_t>(max_blocks) * h_kv)
       return fail(RUS_ERR_INVALID, "%s: %lld counters, need max_blocks * h_kv = %lld", fn,
                   static_cast<long long>(n_counters),
                   static_cast<long long>(max_blocks) * h_kv);

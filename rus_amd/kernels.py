@@ -379,7 +379,6 @@ class NF4Operand:
 
 _gemm_plans: dict[tuple[int, int, int, int, int], tuple[int, int, int]] = {}
 _gemm_counters: dict[tuple[int, int], torch.Tensor] = {}
-_attn_counters: dict[tuple[int, int], torch.Tensor] = {}
 
 
 def nf4_gemm_plan(m: int, w_rows: int, w_cols: int, trans: bool, split: int = 0):
@@ -1755,12 +1754,10 @@ def attn_varlen_bwd(dout: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: tor
     ws = torch.empty(2 * hq * n * d, dtype=torch.float32, device=q.device)
     # q, dO, O, dQ; k, v, dK, dV; the partials written and read back; lse
     nbytes = 2 * (4 * q.numel() + 4 * k.numel()) + 4 * 2 * hq * n * d * 2 + lse.numel() * 4
-    cnt = _counter_buffer(_attn_counters, q.device, mb * k.shape[1])
     _launch("attn_bwd", nbytes, 2.5 * _attn_flops(lens, hq), "rus_attn_varlen_bwd",
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), dout.data_ptr(),
             lse.data_ptr(), cu_seqlens.data_ptr(), n_rows, n, mb, hq, k.shape[1], d, scale,
-            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), cnt.data_ptr(),
-            cnt.numel(), _stream(q))
+            dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), ws.data_ptr(), None, 0, _stream(q))
     return dq, dk, dv
 
 
