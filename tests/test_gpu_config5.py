@@ -239,6 +239,32 @@ def test_bench_engine_step_matches_oracle(full_model):
     _check_gradient_table(table, STRICT_BENCH)
 
 
+@pytest.mark.parametrize("batch_seed,dropout_seed,length_seed", [(21, 99, 5), (23, 777, 11)])
+def test_value_gradients_stay_far_nearer_to_the_oracle_than_eager(full_model, batch_seed,
+                                                                  dropout_seed, length_seed):
+    """STRICT_BENCH's tensors on other batches (513 and 907 tokens), by the distance of the fp16
+    autograd step on the same masks. Their own distances are fp16 rounding noise that grows with the
+    batch and moves by up to 5% from build to build (tensor 94 at 695 tokens: 0.93% to 1.04% over five
+    builds that differ in the order of sums only), so 1e-2 by itself says little beside it; the fused
+    path's share of the eager distance was 0.19 to 0.40 over four batches and two builds."""
+    cfg, model, _ = full_model
+    batch = _batch(cfg.vocab_size, M.lengths_lognormal(4, seed=length_seed), seed=batch_seed)
+    engine = ops.Qwen2FusedEngine(model, DEV, resident_weights=True, recompute=False,
+                                  dequant_once=True, dropout_seed=dropout_seed)
+    gs = GraphedTrainStep(engine, bucket=64, training=True)
+    seed = int(engine.dropout_seed.item()) + 1
+    loss = float(gs.step(*batch))
+    torch.cuda.synchronize()
+    grads = _graph_grads(engine)
+    _, grads_e = _eager_step(engine, batch, True,
+                             seed=torch.tensor([seed], dtype=torch.int64, device=DEV))
+    loss_ref, grads_ref = _oracle_step(model, batch, dropout_seed=seed)
+    assert abs(loss - loss_ref) <= 2e-3 * abs(loss_ref), (loss, loss_ref)
+    table = _gradient_table(grads, grads_e, grads_ref)
+    bad = [(gi, a, b) for gi, a, b in table if gi in STRICT_BENCH and a > 0.45 * b]
+    assert not bad, bad
+
+
 def test_full_model_graph_step_matches_oracle(full_model):
     cfg, model, _ = full_model
     batch = _batch(cfg.vocab_size, [72, 41], seed=13)
