@@ -264,6 +264,36 @@ def test_kept_logit_entry_points_validate_on_the_host(name, args, msg):
         _lib.call(name, *args)
 
 
+@pytest.mark.parametrize(
+    "name,args,msg",
+    [
+        # stored probabilities: no roundings or maxima, a stride below round_up(n_vocab, 64)
+        ("rus_lmhead_ce_fwd_probs", (16, 16, 16, 4, 64, 64, 64, 100, 0, 16, 16, 16, 16, None, 0, 4,
+                                     16, 16, 128, None, 16, 16, None), "null or misaligned"),
+        ("rus_lmhead_ce_fwd_probs", (16, 16, 16, 4, 64, 64, 64, 100, 0, 16, 16, 16, 16, 16, 0, 4,
+                                     16, 16, 128, None, 16, None, None), "null or misaligned"),
+        ("rus_lmhead_ce_fwd_probs", (16, 16, 16, 4, 64, 64, 64, 100, 0, 16, 16, 16, 16, 16, 0, 4,
+                                     16, 16, 120, None, 16, 16, None), "ld_z"),
+        # a state updated in place, a state half given
+        ("rus_lmhead_ce_probs_rescale", (16, 128, 4, 100, 16, 4, 16, 32, 48, 32, 64, 16, 16, None),
+         "in place"),
+        ("rus_lmhead_ce_probs_rescale", (16, 128, 4, 100, 16, 4, 16, 32, None, 64, 80, 16, 16,
+                                         None), "null pointer"),
+        ("rus_lmhead_ce_combine_probs", (16, 16, 16, 16, None, 2, 4, 16, 16, 4, 300, 16, 16, 16, 16,
+                                         16, 16, 16, None), "null pointer"),
+        ("rus_lmhead_ce_combine_probs", (16, 16, 16, 16, 16, 2, 3, 16, 16, 4, 300, 16, 16, 16, 16,
+                                         16, 16, 16, None), "bad sizes"),
+        ("rus_lmhead_ce_dh_finish_probs", (16, 1, 4, 64, 16, 16, 16, 16, 64, 300, 0, 16, 1.0, None,
+                                           16, None, 16, 16, 1, None), "null"),
+        ("rus_lmhead_ce_dh_finish_probs", (16, 1, 4, 66, 16, 16, 16, 16, 66, 300, 0, 16, 1.0, None,
+                                           16, 16, 16, 16, 1, None), "multiple of 4"),
+    ],
+)
+def test_stored_probability_entry_points_validate_on_the_host(name, args, msg):
+    with pytest.raises(RuntimeError, match=msg):
+        _lib.call(name, *args)
+
+
 def test_lm_head_plans_equal_their_exhaustive_search():
     """The chunk length and split count against every candidate, over token counts, vocabularies,
     CU counts and budgets (ties: the longest chunk, the fewest splits)."""
