@@ -523,3 +523,43 @@ def test_nan_logit_far_below_the_maximum_stays_in_the_loss(kw):
         assert bool(out[i].isnan().all()), i
     if out[5] is not None:
         assert bool(out[5].isnan().all())
+
+
+@pytest.mark.parametrize("v,chunk", [(513, 512), (513, 256), (385, 256), (2, 256), (1, 256)])
+def test_label_alone_in_its_rows_and_equal_to_the_maximum(v, chunk):
+    """The label as the only vocabulary row of a chunk, of a half tile and of the vocabulary, and level
+    with the maximum from either side of it (the first index is the argmax): float64 over the device's
+    own logits, tolerances of fp32 and of one fp16 rounding of the other probabilities."""
+    n, d = 40, 64
+    g = torch.Generator().manual_seed(v)
+    h = torch.randn(n, d, generator=g)
+    w = torch.randn(v, d, generator=g) * 0.3
+    labels = torch.full((n,), v - 1)
+    if v > 300:
+        h[:, 0], w[:, 0] = 4.0, 0.0
+        w[7, 0] = 8.0
+        w[300] = w[7]  # both 32 above the rest, equal in every element
+        labels[::3], labels[1::3] = 7, 300
+    h, w, labels = h.half().to(DEV), w.half().to(DEV), labels.to(DEV)
+    nll, lse, ent, amax, _, dh, _ = K.lm_head_ce(h, w, labels, v_chunk=chunk)
+    z = torch.empty(n, K._round_up(v, 64), dtype=torch.float16, device=DEV)
+    K.lm_head_ce_logits(h, w, z)
+    torch.cuda.synchronize()
+    z, wd, y = z[:, :v].double().cpu(), w.double().cpu(), labels.cpu()
+    at = torch.arange(n)
+    want_lse = torch.logsumexp(z, -1)
+    p = torch.exp(z - want_lse[:, None])
+    e32 = 2.0**-22 * (4 + z.abs().amax(-1))
+    assert bool(((lse.double().cpu() - want_lse).abs() <= e32).all())
+    assert bool(((nll.double().cpu() - (want_lse - z[at, y])).abs() <= e32).all())
+    assert bool(((ent.double().cpu() - (want_lse - (p * z).sum(-1))).abs() <= 4 * e32).all())
+    assert torch.equal(amax.cpu(), (z == z.amax(-1, keepdim=True)).int().argmax(-1))
+    p[at, y] = 0
+    rest = p.sum(1, keepdim=True)
+    scale = 65536.0 / n
+    want, mag = (p @ wd - rest * wd[y]) * scale, (p @ wd.abs() + rest * wd[y].abs()) * scale
+    err = (dh.double().cpu() - want).abs()
+    tol = (2.0**-11 + 2 * e32[:, None]) * mag + 2.0**-24 * scale * wd.abs().sum(0)
+    assert bool((err <= tol).all()), float((err / tol.clamp(min=1e-30)).max())
+    if v == 1:
+        assert float(dh.abs().max()) == 0.0
