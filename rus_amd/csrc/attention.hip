@@ -1210,23 +1210,33 @@ __device__ __forceinline__ void bwd_wide_dkdv(const AttnArgs& a, int blk, int he
 }
 
 // dk / dv [key, g, :] = fp16(sum over the KV group's heads in head order) of the partials: a launch
-// of its own, 4 us at 707 tokens. Summed by the last of a group's blocks to arrive it took 7 us
-// with 32-token blocks and 24 us with 128-token ones (one block reading 128 keys x 6 heads from
-// beyond its L2 at the end of the launch). Thread = 4 head dims of one key; y = dk, dv.
+// of its own. Summed by the last of a group's blocks to arrive it took 7 us with 32-token blocks and
+// 24 us with 128-token ones (one block reading 128 keys x 6 heads from beyond its L2 at the end of
+// the launch). Thread = 4 head dims of one key; y = dk, dv. The group's size is a template argument
+// so that all its loads are in flight at once: bound by that one latency and the launch, 4 at a time
+// cost 0.3-0.9 us more (707 tokens of 8 / 1 heads, whole backward: last block 18.9 us, 4 at a time
+// 16.4, this 15.7; 100 tokens of 14 / 2 15.0, 12.2, 11.4). Where 32-token blocks just fill the chip
+// the last block's sum was partly hidden, which no launch after them is: 1,206 tokens of 12 / 2 27.5
+// us against 28.3 now, 2,048 of 8 / 1 28.6 against 30.1; beyond, 178 against 92. (The partials are
+// stored past the L2, store_partial: with plain stores the launch's end waits for their write-back,
+// 5-10% of the small batches.)
+template <int kGrp>
 __global__ __launch_bounds__(256) void attn_group_sum_kernel(AttnArgs a) {
-  const int grp = a.h_q / a.h_kv;
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   const int c = 4 * static_cast<int>(t & 31), g = static_cast<int>((t >> 5) % a.h_kv);
   const int64_t key = (t >> 5) / a.h_kv;
   if (key >= a.n_tok) return;
   const float* src = (blockIdx.y == 0 ? a.dk_part : a.dv_part) +
-                     (static_cast<int64_t>(g) * grp * a.n_tok + key) * kHD + c;
-  f32x4 s = *reinterpret_cast<const f32x4*>(src);
-#pragma unroll 4
-  for (int j = 1; j < grp; ++j) s += *reinterpret_cast<const f32x4*>(src + j * a.n_tok * kHD);
+                     (static_cast<int64_t>(g) * kGrp * a.n_tok + key) * kHD + c;
+  f32x4 v[kGrp];
+#pragma unroll
+  for (int j = 0; j < kGrp; ++j)
+    v[j] = *reinterpret_cast<const f32x4*>(src + j * a.n_tok * kHD);
+#pragma unroll
+  for (int j = 1; j < kGrp; ++j) v[0] += v[j];
   f16x4 w;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = from_f32<f16>(s[i]);
+  for (int i = 0; i < 4; ++i) w[i] = from_f32<f16>(v[0][i]);
   *reinterpret_cast<f16x4*>((blockIdx.y == 0 ? a.dk : a.dv) + (key * a.h_kv + g) * kHD + c) = w;
 }
 
@@ -1386,9 +1396,14 @@ static int attn_bwd(const char* fn, const void* q, const void* k, const void* v,
   }
   if (int e = check_launch(fn)) return e;
   if (!group_sum) return RUS_OK;
-  hipLaunchKernelGGL(attn_group_sum_kernel,
-                     dim3(static_cast<unsigned>((n_tokens * h_kv * 32 + 255) / 256), 2), dim3(256),
-                     0, st, a);
+  const dim3 sum_grid(static_cast<unsigned>((n_tokens * h_kv * 32 + 255) / 256), 2);
+#define RUS_GROUP_SUM(G) \
+  case G: hipLaunchKernelGGL(attn_group_sum_kernel<G>, sum_grid, dim3(256), 0, st, a); break;
+  switch (h_q / h_kv) {
+    RUS_GROUP_SUM(1) RUS_GROUP_SUM(2) RUS_GROUP_SUM(3) RUS_GROUP_SUM(4)
+    RUS_GROUP_SUM(5) RUS_GROUP_SUM(6) RUS_GROUP_SUM(7) RUS_GROUP_SUM(8)
+  }
+#undef RUS_GROUP_SUM
   return check_launch(fn);
 }
 

@@ -202,6 +202,26 @@ def test_attention_partials_equal_group_sum(lens, hq, hkv):
         assert torch.equal(acc.half().permute(1, 0, 2).contiguous(), full)
 
 
+@pytest.mark.parametrize("hq,hkv", [(2, 1), (6, 2), (5, 1), (14, 2)])
+def test_attention_group_sum_of_every_group_size(hq, hkv):
+    """dk and dv of the group sizes the other tests leave out (2, 3, 5, 7): the partials in head order,
+    rounded once, with a last block of the sum that is part empty."""
+    q, k, v, dout, cu = _inputs([33, 4], hq, hkv, seed=hq)
+    qd, kd, vd, dd = _dev(q, k, v, dout)
+    cud = torch.tensor(cu, dtype=torch.int32, device=DEV)
+    out, lse = K.attn_varlen_fwd(qd, kd, vd, cud)
+    full = K.attn_varlen_bwd(dd, qd, kd, vd, out, lse, cud)
+    parts = K.attn_varlen_bwd_parts(dd, qd, kd, vd, out, lse, cud)
+    torch.cuda.synchronize()
+    assert torch.equal(parts[0], full[0])
+    for part, got in zip(parts[1:], full[1:]):
+        part = part.view(hkv, hq // hkv, -1, 128)
+        acc = part[:, 0].clone()
+        for j in range(1, hq // hkv):
+            acc += part[:, j]
+        assert torch.equal(acc.half().permute(1, 0, 2).contiguous(), got)
+
+
 def test_rope_mid_over_attention_partials_equals_group_sum_path():
     # Attention partials -> RoPE backward that sums them equals attention group sum -> RoPE
     # backward, for all five outputs, bit for bit (bench-shaped heads, rank 16).
