@@ -1212,14 +1212,14 @@ __device__ __forceinline__ void bwd_wide_dkdv(const AttnArgs& a, int blk, int he
 // dk / dv [key, g, :] = fp16(sum over the KV group's heads in head order) of the partials: a launch
 // of its own. Summed by the last of a group's blocks to arrive it took 7 us with 32-token blocks and
 // 24 us with 128-token ones (one block reading 128 keys x 6 heads from beyond its L2 at the end of
-// the launch). Thread = 4 head dims of one key; y = dk, dv. The group's size is a template argument
-// so that all its loads are in flight at once: bound by that one latency and the launch, 4 at a time
-// cost 0.3-0.9 us more (707 tokens of 8 / 1 heads, whole backward: last block 18.9 us, 4 at a time
-// 16.4, this 15.7; 100 tokens of 14 / 2 15.0, 12.2, 11.4). Where 32-token blocks just fill the chip
-// the last block's sum was partly hidden, which no launch after them is: 1,206 tokens of 12 / 2 27.5
-// us against 28.3 now, 2,048 of 8 / 1 28.6 against 30.1; beyond, 178 against 92. (The partials are
-// stored past the L2, store_partial: with plain stores the launch's end waits for their write-back,
-// 5-10% of the small batches.)
+// the launch). Thread = 4 head dims of one key; y = dk, dv. The group's size is a template argument,
+// so that the heads past the first four are in flight together too (one by one: 100 tokens of 14 / 2
+// heads, whole backward, 12.1 us, this 11.7; 707 of 8 / 1 16.4, 15.7). All eight together gain
+// another 0.2 us there and lose 1-2% from 8,161 tokens on, where the reads bound it (5.5 TB/s).
+// Where 32-token blocks just fill the chip the last block's sum was partly hidden, which no launch
+// after them is: 1,206 tokens of 12 / 2 27.5 us against 28.3 now, 2,048 of 8 / 1 28.6 against 30.4;
+// beyond, 178 against 91. (The partials are stored past the L2, store_partial: with plain stores the
+// launch's end waits for their write-back, 5-10% of the small batches.)
 template <int kGrp>
 __global__ __launch_bounds__(256) void attn_group_sum_kernel(AttnArgs a) {
   const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
@@ -1228,15 +1228,22 @@ __global__ __launch_bounds__(256) void attn_group_sum_kernel(AttnArgs a) {
   if (key >= a.n_tok) return;
   const float* src = (blockIdx.y == 0 ? a.dk_part : a.dv_part) +
                      (static_cast<int64_t>(g) * kGrp * a.n_tok + key) * kHD + c;
-  f32x4 v[kGrp];
+  constexpr int kDepth = 4;  // heads whose loads are in flight together
+  f32x4 s;
 #pragma unroll
-  for (int j = 0; j < kGrp; ++j)
-    v[j] = *reinterpret_cast<const f32x4*>(src + j * a.n_tok * kHD);
+  for (int j0 = 0; j0 < kGrp; j0 += kDepth) {
+    f32x4 v[kDepth];
 #pragma unroll
-  for (int j = 1; j < kGrp; ++j) v[0] += v[j];
+    for (int j = 0; j < kDepth; ++j)
+      if (j0 + j < kGrp) v[j] = *reinterpret_cast<const f32x4*>(src + (j0 + j) * a.n_tok * kHD);
+#pragma unroll
+    for (int j = 0; j < kDepth; ++j)
+      if (j0 + j < kGrp) s = j0 + j == 0 ? v[0] : s + v[j];
+    __builtin_amdgcn_sched_barrier(0);
+  }
   f16x4 w;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = from_f32<f16>(v[0][i]);
+  for (int i = 0; i < 4; ++i) w[i] = from_f32<f16>(s[i]);
   *reinterpret_cast<f16x4*>((blockIdx.y == 0 ? a.dk : a.dv) + (key * a.h_kv + g) * kHD + c) = w;
 }
 
