@@ -505,3 +505,29 @@ def test_rope_products_of_one_to_four_tokens_per_thread(n, scale):
     qkv = torch.zeros(n, (hq + 2 * hkv) * hd, dtype=torch.float16, device=DEV)
     v = K.qkv_rope_fwd_mid(qkv, mid, mid, bq, bv, *rope, 2.0, 2.0, hq, hkv, hd)[2]
     check(v.view(n, -1), mid, bv.t(), factor=2.0)
+
+
+@pytest.mark.parametrize("hq,hkv", [(4, 2), (24, 4)])
+@pytest.mark.parametrize("n", [2049, 6149])
+def test_rope_bwd_mid_tokens_per_thread_at_other_head_counts(hq, hkv, n):
+    """Four and one tokens per block and pass (12 / 2 heads: two): two and four tokens per thread give
+    the bits of slices short enough for one."""
+    hd, r = 128, 16
+    g = torch.Generator(device=DEV).manual_seed(hq + n)
+
+    def rnd(*shape):
+        return torch.randn(*shape, generator=g, device=DEV)
+
+    dq, parts = rnd(n, hq, hd).half(), [rnd(hq, n, hd) for _ in range(2)]
+    ang = rnd(600, hd)
+    cos, sin = ang.cos().half(), ang.sin().half()
+    pos = torch.randint(0, 600, (n,), generator=g, device=DEV)
+    factors = (rnd(r, hq * hd).half(), rnd(r, hkv * hd).half())
+    heads = dict(h_q=hq, h_kv=hkv, head_dim=hd)
+    whole = K.qkv_rope_bwd_lora_mid_parts(dq, *parts, cos, sin, pos, 2.0, 0.5, *factors, **heads)
+    for a in range(0, n, 1500):
+        s = slice(a, min(a + 1500, n))
+        got = K.qkv_rope_bwd_lora_mid_parts(dq[s].contiguous(), *(p[:, s].contiguous() for p in parts),
+                                            cos, sin, pos[s].contiguous(), 2.0, 0.5, *factors, **heads)
+        for x, y in zip(got, whole):
+            assert torch.equal(x, y[s])
