@@ -22,7 +22,8 @@
 //     GEMM adds P . W_chunk into fp32 partials rescaled when K grows; lmhead_combine_kernel adds the
 //     label to the statistics and lmhead_dh_finish_kernel divides by s and subtracts
 //     (1 - p_label) W[y]. (kLogits with lmhead_chunk_scale_kernel, which keeps the label in P and
-//     takes the running maximum as the reference, serves callers of those entry points.)
+//     takes the running maximum as the reference, is there for callers of those entry points alone:
+//     the package runs kProbs.)
 // The GEMMs run the mainloops of mfma_gemm.h: 256 x 256 block tiles on v_mfma_f32_32x32x16_f16
 // filled by direct global -> LDS copies. The logits, statistics and hidden-gradient kernels run
 // eight waves of 128 x 64 (two per SIMD) with K staged 64 deep through two 64 KiB buffers; the

@@ -1427,7 +1427,8 @@ def lm_head_chunk_cols(n_tok: int, n_vocab: int, n_cu: int = 256,
     """Vocabulary rows per chunk of the single-pass head: a multiple of 256 whose fp16 logits
     [n_tok, cols] fit ``budget``, chosen to minimise an estimate of the statistics GEMM time
     (whole rounds of one-per-CU 256x256 tiles, ~45 us each) plus a per-chunk cost (~60 us: two
-    launches, the fp32 partials read and rewritten, a GEMM's ramp). Among the chunks of one number
+    launches, the fp32 partials read and rewritten, a GEMM's ramp), both at hidden 1,536; their
+    ratio decides, and both grow with the hidden size. Among the chunks of one number
     of rounds the longest costs the least (no more chunks, no more rounds of the rest), so only
     those are compared: a few per call, which every new n_tok makes (150 us of host time when
     every length was).
